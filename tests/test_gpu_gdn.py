@@ -423,6 +423,25 @@ def test_chunked_carry_gives_up_and_is_redone(dev, orc, monkeypatch, io):
     _check(o1, s1, o_ref, s_ref, *tol, label=f"chunked {io}, overlap, carry waits limited to 0")
 
 
+@pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("hq,hv,T", [(1, 1, 1), (3, 7, 63), (16, 32, 64), (16, 33, 65), (5, 31, 129), (16, 48, 200),
+                                     (48, 16, 257), (2, 65, 320)])
+def test_chunked_column_tiles(dev, orc, hq, hv, T, io):
+    """The carry's two widths (16 columns a workgroup up to 32 heads, 32 above) at head counts
+    around the line and off the multiples of 8 it pads to, odd and even chunk counts, one
+    token to a full last chunk, QK heads shared or not, from a nonzero state.  State bound,
+    fp32 I/O: every operand is an fp16 hi + lo pair (2^-22 relative each, at most four of them
+    in a product chain) summed in fp32 over 64 keys a chunk: 64 * 2^-24 + 4 * 2^-22 = 5e-6,
+    taken four times for the chunks a value lives through."""
+    rng = np.random.default_rng(1000 + hv + T)
+    q, k, v, g, beta, st = _inputs(rng, 1, T, hq, hv, sstd=0.02)
+    if io == "f32":
+        q, k, v = (x.astype(np.float32) + 2e-4 * rng.standard_normal(x.shape).astype(np.float32) for x in (q, k, v))
+    o, s = _gpu(dev, "chunked", q, k, v, g, beta, st)
+    o_ref, s_ref = orc.gdn_serial(q, k, v, g, beta, st)
+    _check(o, s, o_ref, s_ref, *(TOL["chunked"] if io == "f16" else (2e-3, 2e-5)), label=f"{io} Hq={hq} Hv={hv} T={T}")
+
+
 def _ws_fill(ws, kind):
     import torch
     if kind == "ones":      # every flag and abort word reads 1 ("ready", "redo")

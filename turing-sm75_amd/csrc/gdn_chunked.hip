@@ -4,29 +4,22 @@
 // the exact inverse).  Per V-head and chunk of C = 64 tokens, rows = tokens t, with
 // G_t = in-chunk inclusive cumsum of g_log:
 //   A[t][s]   = beta_t (k_t . k_s) e^{G_t - G_s}      s < t        (strictly lower)
-//   Tm        = (I + A)^-1
-//   W         = Tm diag(beta e^G) K          (C x dk)
-//   U         = Tm diag(beta) V              (C x dv)
+//   T'        = (I + A)^-1 diag(beta)
 //   Aqk[t][s] = (q_t . k_s) e^{G_t - G_s}      s <= t
-//   Vnew      = U - W S                      (S is dk x dv, the state entering the chunk)
+//   Vnew      = T' (V - diag(e^G) K S)           (S is dk x dv, the state entering the chunk)
 //   O         = scale (diag(e^G) Q S + Aqk Vnew)
 //   S'        = e^{G_{C-1}} S + K^T diag(e^{G_{C-1} - G}) Vnew
 // Only differences G_t - G_s with s <= t are exponentiated, so nothing overflows.
 //
 // gdn_chunk_prep  -- one workgroup per (b, h, chunk), all chunks in parallel: G by a wave
-//   scan, K K^T and Q K^T on v_mfma_f32_32x32x16_f16 (the all-zero upper tile skipped),
-//   the exact (I + A)^-1 by 16x16 blocks in fp32 (diagonal blocks by forward substitution,
-//   then each wave owns one block column, so no cross-wave dependency), W and U on MFMA
-//   with K and V read transposed by ds_read_b64_tr_b16.  W, U, Aqk leave through LDS
-//   staging as 16-byte stores, already in the operand layouts the carry kernel loads.
-// gdn_chunk_carry -- one workgroup per (b, h, 32 state columns), sequential over chunks.
-//   Two "chain" waves each own a 16-column strip of S in fp32 MFMA accumulators and run
-//   only the loop-carried part: W S and the state update (32 v_mfma_f32_16x16x32_f16 per
-//   chunk).  Two "output" waves trail by one chunk and compute Q S + Aqk Vnew from the
-//   S / Vnew operands the chain waves leave in LDS.  Every operand tile is staged one chunk
-//   ahead with gfx950 LDS-DMA (global_load_lds_dwordx4) into double-buffered slots, so no
-//   register holds prefetched data and each wave reads its MFMA operands from LDS in
-//   batches ahead of the MFMAs.
+//   scan, K K^T and Q K^T on v_mfma_f32_32x32x16_f16 (the all-zero upper tile skipped), the
+//   exact (I + A)^-1 by 16x16 blocks in fp32.  T' (fp16 hi + lo), Aqk and the per-token factors
+//   go to the workspace in the operand layouts the carry loads.
+// gdn_chunk_carry -- one workgroup per (b, h, 16 or 32 state columns), sequential over chunks.
+//   V and K S meet before T' is applied, so neither T' V nor T' K ever exists in memory: per
+//   chunk and head the prep leaves 19 KiB, which the carry reads besides q, k and v's rows
+//   (with W = T' diag(e^G) K and U = T' V formed by the prep it was 57 KiB each way: 372 MB per
+//   call at 32 heads, T = 4096, against 106 MB of inputs and outputs).
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -44,26 +37,36 @@ namespace {
 constexpr int kC = 64;     // chunk
 constexpr int kD = 128;    // dk = dv
 constexpr int kThreads = 256;
-constexpr int kStrips = 2; // 16-column strips per carry workgroup
-constexpr int kCarryThreads = 512;  // waves 0-1 chain, 2-3 output, 4-7 DMA
+constexpr int kCarryThreads = 512;
+constexpr int kAbortWgs = 4;  // carry workgroups per head beside the prep (32 columns each)
 
-// Workspace per (b, h, chunk).
-constexpr int kWsW = 0;                     // fp16 [64 t][128]: column i stored at perm32(i)
-constexpr int kWsU = kWsW + kC * kD * 2;    // fp32 [8 strip][4 mtile][64 lane][4]
-constexpr int kWsAqk = kWsU + kC * kD * 4;  // fp16 [64 t][64]: column s stored at perm32(s)
-// fp32 [64] e^{G_t} qn_t, [64] e^{G_63 - G_t} kn_t, [64] {e^{G_63}, 0, ...}, [64] zeros, where
-// qn_t, kn_t are the l2-norm factors of the fused entry point's raw q / k rows (1 otherwise)
-constexpr int kWsG = kWsAqk + kC * kC * 2;
-constexpr int kWsChunk = kWsG + kC * 16;    // 58368 B, multiple of 256
-// fp32 q / k / v / out (the reference's own I/O): the prep also leaves the chunk's K and Q
-// rows in fp16, unswizzled [64 t][128], for the carry's copies (LDS-DMA cannot convert)
-constexpr int kWsK = kWsChunk;
+// Workspace per (b, h, chunk).  T' and Aqk are in operand order: slot (w, ks), lane (g, c) holds
+// row 16 w + c, columns 32 ks + 8 g .. + 7 in 16 bytes; the slots (0, 1) and (1, 1) lie above the
+// diagonal and are left out.
+constexpr int kTSlots = 6;
+__device__ __forceinline__ int op_slot(int w, int ks) { return w < 2 ? w : 2 * w - 2 + ks; }
+constexpr int kWsT = 0;                            // fp16 T' hi
+constexpr int kWsTlo = kWsT + kTSlots * 1024;      // fp16 T' - hi
+constexpr int kWsAqk = kWsTlo + kTSlots * 1024;    // fp16 Aqk
+// fp32 [64] e^{G_t} qn_t, [64] e^{G_t} kn_t, [64] e^{G_63 - G_t} kn_t, [64] e^{G_63}, where qn_t,
+// kn_t are the l2-norm factors of the fused entry point's raw q / k rows (1 otherwise)
+constexpr int kWsG = kWsAqk + kTSlots * 1024;
+// The chunk's K and Q rows as fp16, written once per QK head (by the V-head of the same number, whose
+// slot holds them): K as rows, Q in operand order (slot (w, kk), lane (g, c): token 16 w + c, dk
+// 32 kk + 8 g .. + 7), with fp32 I/O then K - fp16(K).  In the inputs a head's rows lie Hq * 256
+// bytes apart: with Hq a multiple of 16 they share one L2 channel, and the 8 carry workgroups of
+// a head wait for it (T = 4096, 32 heads: 112 us a call with 16 QK heads, 96 us with 11).
+constexpr int kWsK = kWsG + kC * 16;
 constexpr int kWsQ = kWsK + kC * kD * 2;
-// and the low halves of the K rows (K - fp16(K), fp16): the state update takes K as an exact
-// hi + lo pair, since rounding the fp32 K to one fp16 operand there is most of the fp32 path's
-// state error (~2.3e-4 of 3.4e-4 on the reference's own inputs, numpy model)
 constexpr int kWsKlo = kWsQ + kC * kD * 2;
-constexpr int kWsChunkF32 = kWsKlo + kC * kD * 2;  // 107520 B
+constexpr int kWsUsed = kWsKlo;                  // 52224 B
+constexpr int kWsUsedF32 = kWsKlo + kC * kD * 2; // 68608 B
+// Bytes from one chunk's workspace to the next: what callers have sized their buffers by
+// (tsa_gdn_chunked_workspace_bytes) and what decides whether the no-allocation scratch holds a
+// call, so it stays though a chunk now uses less.
+constexpr int kWsChunk = 58368;
+constexpr int kWsChunkF32 = 107520;
+static_assert(kWsUsed <= kWsChunk && kWsUsedF32 <= kWsChunkF32, "a chunk's workspace fits its slot");
 template <bool kF32> constexpr int ws_chunk() { return kF32 ? kWsChunkF32 : kWsChunk; }
 
 // Ready flags, after all chunk workspaces: one word per (b, h, chunk), then an abort word per
@@ -73,8 +76,8 @@ template <bool kF32> constexpr int ws_chunk() { return kF32 ? kWsChunkF32 : kWsC
 // as set before the prep sets it in this call.  A call that runs them in order writes and
 // reads no flags (both kernels get a null flag pointer: the kernel boundary orders the prep's
 // stores before the carry), and the carry zeroes the abort words itself.  Beside the carry
-// the prep writes 1 there once the chunk's workspace is in memory; the carry's DMA waves wait
-// for it before copying the chunk.
+// the prep writes 1 there once the chunk's workspace is in memory; the carry's waves wait
+// for it before loading the chunk's workspace.
 // A wait gives up after a limit on the 100 MHz real-time counter (2 ms; the environment
 // variable TSA_GDN_CARRY_WAIT_US sets it in microseconds, 0 = give up whenever a chunk is
 // not ready at the first look, which is how the tests exercise the path).  When the prep
@@ -124,13 +127,6 @@ struct CarryJob {
     float* om = nullptr;   // [B*Hv][Tr][kD]: M, the Phi chains' outputs
 };
 
-// Within each aligned 32-block, index 16a + 4g + b is stored at 8g + 4a + b.  A 16x16x32
-// MFMA lane of group g then finds its 8 k-values {16a + 4g + b} in one 16-byte run; that
-// k order is the one in which a 16x16 accumulator (rows 4g + r) is reused as a B operand.
-__device__ __forceinline__ int perm32(int i) {
-    return (i & ~31) | (((i >> 2) & 3) << 3) | (((i >> 4) & 1) << 2) | (i & 3);
-}
-
 // 16-B chunk swizzle for [rows][128] fp16 LDS tiles (same argument as attn_fwd.hip): 16
 // consecutive rows at one chunk, and 4 aligned rows x 2 chunks, are bank-conflict free.
 __device__ __forceinline__ int swz(int r) {
@@ -160,18 +156,31 @@ __device__ __forceinline__ half8_t cat8(const half4_t& a, const half4_t& b) {
 }
 
 // Device-scope stores of the workspace (sc1): written through to the device's coherence
-// point, so the carry, whose copies of them are device-scope loads too, sees them from any
+// point, so a carry beside the prep, whose loads of them are device-scope too, sees them from any
 // XCD as soon as this wave's vmcnt has drained -- no L2 write-back or invalidate needed
 // (both measured far too slow to issue once per workgroup or chunk).
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void store_dev(unsigned char* p, const uint4& v) {
     const u32x4_t x = {v.x, v.y, v.z, v.w};
     // s_nop 1: a store of more than 8 bytes may still read its data registers in the next
     // cycle, and the compiler does not see into this asm to keep them unchanged that long
     asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(x) : "memory");
 }
+__device__ __forceinline__ void store_dev8(unsigned char* p, const uint2& v) {
+    const u32x2_t x = {v.x, v.y};
+    asm volatile("global_store_dwordx2 %0, %1, off sc1" ::"v"(p), "v"(x) : "memory");
+}
 __device__ __forceinline__ void store_dev(float* p, float v) {
     asm volatile("global_store_dword %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
+}
+
+// x as a value in a register.  The two halves of a split must come from the same fp32 value: left
+// alone, the compiler folds a product into the high half's conversion (one rounding) but not
+// into the low half's subtraction, and a product near a tie loses half an fp16 ulp.
+__device__ __forceinline__ float rounded(float x) {
+    asm volatile("" : "+v"(x));
+    return x;
 }
 
 // 8 consecutive q / k / v elements as 8 fp16 values (one uint4), from fp16 or fp32 memory:
@@ -183,7 +192,7 @@ __device__ __forceinline__ uint4 load8h(const float* p) {
                        (half_t)b.x, (half_t)b.y, (half_t)b.z, (half_t)b.w};
     return __builtin_bit_cast(uint4, h);
 }
-// The same 8 fp32 elements as an exact pair of fp16 halves: hi = fp16(x), lo = fp16(x - hi).
+// The same 8 elements as an exact pair of fp16 halves: hi = fp16(x), lo = fp16(x - hi).
 __device__ __forceinline__ void load8hl(const float* p, uint4& hi, uint4& lo) {
     const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
     const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
@@ -196,10 +205,7 @@ __device__ __forceinline__ void load8hl(const float* p, uint4& hi, uint4& lo) {
     hi = __builtin_bit_cast(uint4, h);
     lo = __builtin_bit_cast(uint4, l);
 }
-__device__ __forceinline__ void load8hl(const half_t* p, uint4& hi, uint4& lo) {
-    hi = *reinterpret_cast<const uint4*>(p);
-    lo = make_uint4(0, 0, 0, 0);
-}
+__device__ __forceinline__ void load8hl(const half_t* p, uint4& hi, uint4&) { hi = load8h(p); }
 
 // ----------------------------------------------------------------------------------
 // Prep
@@ -214,44 +220,36 @@ __device__ __forceinline__ int tri_off(int row, int col) {
     return (((i * (i + 1)) >> 1) + j) * 256 + r * 16 + ((((c >> 2) ^ (r >> 2)) & 3) << 2) + (c & 3);
 }
 
-// 37 KB, so four workgroups share a CU.  Region x holds A and Aqk / Tm during the solve,
-// then V for the U product; K's region takes the W staging.
+// A and Tm take the places of the Q and K rows once K K^T and Q K^T are done.
 struct PrepLds {
-    half_t K[kC * kD];          // K rows, swizzled; W staging at the end
     union {
-        struct {
-            float A[10 * 256];  // strictly lower A, packed blocks
-            union {
-                half_t Aqk[kC * kC];  // Aqk staging
-                float Tm[10 * 256];   // (I + A)^-1, packed blocks
-            };
-        } s;
-        half_t V[kC * kD];      // V rows, swizzled
-    } x;
+        half_t K[kC * kD];     // K rows, swizzled
+        float Tm[10 * 256];    // (I + A)^-1, packed blocks
+    };
+    union {
+        half_t Q[kC * kD];     // Q rows, swizzled
+        float A[10 * 256];     // strictly lower A, packed blocks
+    };
     float G[kC];
     float bt[kC];
-    float bg[kC];
     float kn[kC];  // l2-norm factors 1 / max(||k_t||, eps), 1 / max(||q_t||, eps) (fused only)
     float qn[kC];
 };
 
-// kFused: q / k are the raw rows (normalised here: the factors scale A, Aqk, W and the
-// workspace's e^G / e^{G_63 - G}, so the carry multiplies raw K / Q rows by them for free),
-// and g_log / beta are computed from the raw projections a / b (gate arguments).
-// TIO: the q / k / v element type (fp16, or fp32 with the K / Q rows left in fp16 in the
-// workspace for the carry).
-// Four workgroups per CU (128 VGPRs); the fp32-I/O form holds its fp32 loads before converting
-// them and needs more registers, so it runs three per CU rather than spill.
+// kFused: q / k are the raw rows (normalised here: the factors scale A, Aqk and the per-token
+// factors, so the carry takes the raw K / Q rows), and g_log / beta are computed from the raw
+// projections a / b (gate arguments).
+// TIO: the q / k element type.
+// With fp32 I/O K K^T takes K as hi + lo (hi hi + hi lo + lo hi): the carry's K S does, and an A of
+// rounded rows beside it would be its state error (1.0e-4 instead of 1e-5 on a slow gate, T = 2048).
 template <typename TIO> constexpr int prep_wgs_per_cu() { return std::is_same<TIO, float>::value ? 3 : 4; }
 template <bool kFused, typename TIO>
 __global__ void __launch_bounds__(kThreads, prep_wgs_per_cu<TIO>())
-gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k,
-               const TIO* __restrict__ v, const float* __restrict__ g_log,
+gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k, const float* __restrict__ g_log,
                const float* __restrict__ beta, GdnRawGates gates, unsigned char* __restrict__ ws,
                unsigned* __restrict__ flags, int T, int Hq, int Hv, int nch, int BHv) {
     __shared__ __align__(16) PrepLds sm;
-    // fp32 I/O: the low fp16 halves of the chunk's V rows (swizzled like V), 16 KiB more LDS
-    __shared__ __align__(16) half_t vlo_lds[std::is_same<TIO, float>::value ? kC * kD : 8];
+    __shared__ __align__(16) half_t klo_lds[std::is_same<TIO, float>::value ? kC * kD : 8];  // low halves of the K rows
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hi = lane >> 5;
     // chunk-major: workgroups are dispatched in the order the carry consumes chunks, and
     // (b, h, chunk) lands on the XCD of the head's carry workgroups when BHv % 8 == 0
@@ -263,11 +261,11 @@ gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k,
     unsigned char* wsc = ws + ((size_t)bh * nch + ch) * ws_chunk<kF32>();
     const int mt = wave >> 1, nt = wave & 1;  // this wave's 32x32 tile of K K^T / Q K^T
 
-    // ---- 1. K rows to LDS, V rows and this wave's Q operand rows to registers.  Every global
-    // load of the phase is issued first (wave 0's gate inputs, K, V, Q), from row-clamped
-    // addresses, and rows past T are zeroed where the values are consumed: a branch around a
-    // load makes the compiler wait for every load in flight where the paths join, which had
-    // serialised the phase into one memory latency per K row group ----
+    // ---- 1. K and Q rows to LDS.  Every global load of the phase is issued first (wave 0's gate
+    // inputs, K, Q), from row-clamped addresses, and rows past T are zeroed where the values are
+    // consumed: a branch around a load makes the compiler wait for every load in flight where the
+    // paths join.  A row is 16 lanes of 16 bytes: loading Q in the shape of its MFMA operand (32
+    // rows x 32 bytes an instruction) cost 128 cycles of the CU's load path each instead of 20 ----
     const int lastt = T - 1;
     float gx = 0.f, gy = 0.f;  // wave 0: the gate inputs of token t0 + lane
     if (wave == 0) {
@@ -275,62 +273,46 @@ gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k,
         gx = kFused ? gates.a[bt * Hv + h] : g_log[bt * Hv + h];
         gy = kFused ? gates.b[bt * Hv + h] : beta[bt * Hv + h];
     }
-    // with fp32 I/O K and V also keep their low fp16 halves: K_lo goes to the workspace for the
-    // carry's state update, V_lo feeds the U product as a second B operand
-    uint4 kreg[4], vreg[4], klo[4], vlo[4];
+    uint4 kreg[4], qreg[4], klo[4];
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
         const int id = it * kThreads + tid;
-        const size_t bt = (size_t)b * T + min(t0 + (id >> 4), lastt);
-        load8hl(k + (bt * Hq + hq) * kD + (id & 15) * 8, kreg[it], klo[it]);
-        load8hl(v + (bt * Hv + h) * kD + (id & 15) * 8, vreg[it], vlo[it]);
+        const size_t o = (((size_t)b * T + min(t0 + (id >> 4), lastt)) * Hq + hq) * kD + (id & 15) * 8;
+        load8hl(k + o, kreg[it], klo[it]);
+        qreg[it] = load8h(q + o);
     }
-    half8_t qa[kD / 16];
-    const int qt_row = t0 + 32 * mt + (lane & 31);
-    {
-        const TIO* qrow = q + (((size_t)b * T + min(qt_row, lastt)) * Hq + hq) * kD + 8 * hi;
-#pragma unroll
-        for (int s = 0; s < kD / 16; ++s) qa[s] = __builtin_bit_cast(half8_t, load8h(qrow + 16 * s));
-    }
+    const bool copies = h < Hq;  // this workgroup leaves its QK head's rows to the carry
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
         const int id = it * kThreads + tid;
         const int r = id >> 4, c = id & 15;
-        const uint4 kv = t0 + r > lastt ? make_uint4(0, 0, 0, 0) : kreg[it];
+        const bool past = t0 + r > lastt;
+        const uint4 kv = past ? make_uint4(0, 0, 0, 0) : kreg[it], qv = past ? make_uint4(0, 0, 0, 0) : qreg[it];
+        const uint4 kl = past ? make_uint4(0, 0, 0, 0) : klo[it];
         *reinterpret_cast<uint4*>(sm.K + tile_off(r, c)) = kv;
-        if (kF32) {
-            store_dev(wsc + kWsK + (size_t)(r * kD + c * 8) * 2, kv);
-            store_dev(wsc + kWsKlo + (size_t)(r * kD + c * 8) * 2, t0 + r > lastt ? make_uint4(0, 0, 0, 0) : klo[it]);
+        *reinterpret_cast<uint4*>(sm.Q + tile_off(r, c)) = qv;
+        if (kF32) *reinterpret_cast<uint4*>(klo_lds + tile_off(r, c)) = kl;
+        if (copies) {
+            store_dev(wsc + kWsK + (size_t)id * 16, kv);
+            if (kF32) store_dev(wsc + kWsKlo + (size_t)id * 16, kl);
         }
         if (kFused) {  // the row's 16 threads are 16 consecutive lanes of one wave
-            const half8_t k8 = __builtin_bit_cast(half8_t, kv);
-            float ss = 0.f;
+            const half8_t k8 = __builtin_bit_cast(half8_t, kv), q8 = __builtin_bit_cast(half8_t, qv);
+            float sk = 0.f, sq = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ss = fmaf((float)k8[e], (float)k8[e], ss);
-            ss += __shfl_xor(ss, 8);
-            ss += __shfl_xor(ss, 4);
-            ss += __shfl_xor(ss, 2);
-            ss += __shfl_xor(ss, 1);
-            if (c == 0) sm.kn[r] = 1.f / fmaxf(sqrtf(ss), gates.eps);
-        }
-    }
-    {
+            for (int e = 0; e < 8; ++e) {
+                sk = fmaf((float)k8[e], (float)k8[e], sk);
+                sq = fmaf((float)q8[e], (float)q8[e], sq);
+            }
 #pragma unroll
-        for (int s = 0; s < kD / 16; ++s) qa[s] = qt_row > lastt ? half8_t{} : qa[s];
-        if (kF32 && nt == 0) {  // waves 0 and 2 hold the chunk's 64 Q rows
-            const int row = 32 * mt + (lane & 31);
-#pragma unroll
-            for (int s = 0; s < kD / 16; ++s)
-                store_dev(wsc + kWsQ + (size_t)(row * kD + 16 * s + 8 * hi) * 2, __builtin_bit_cast(uint4, qa[s]));
-        }
-        if (kFused) {  // the two halves of the row are lanes l and l ^ 32
-            float ss = 0.f;
-#pragma unroll
-            for (int s = 0; s < kD / 16; ++s)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) ss = fmaf((float)qa[s][e], (float)qa[s][e], ss);
-            ss += __shfl_xor(ss, 32);
-            if (nt == 0 && hi == 0) sm.qn[32 * mt + (lane & 31)] = 1.f / fmaxf(sqrtf(ss), gates.eps);
+            for (int off = 8; off > 0; off >>= 1) {
+                sk += __shfl_xor(sk, off);
+                sq += __shfl_xor(sq, off);
+            }
+            if (c == 0) {
+                sm.kn[r] = 1.f / fmaxf(sqrtf(sk), gates.eps);
+                sm.qn[r] = 1.f / fmaxf(sqrtf(sq), gates.eps);
+            }
         }
     }
     if (wave == 0) {
@@ -353,96 +335,106 @@ gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k,
         sm.bt[lane] = be;
     }
     lds_barrier();
-
-    // ---- 2. K K^T and Q K^T; A (fp32, strictly lower) and Aqk (fp16 staging) ----
-    if (mt == 0 && nt == 1) {
-        // every (t < 32, s >= 32) entry is above the diagonal: Aqk is zero there
+    if (copies) {  // Q in operand order
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int t = 8 * (r >> 2) + 4 * hi + (r & 3);
-            sm.x.s.Aqk[t * kC + perm32(32 + (lane & 31))] = (half_t)0.f;
+        for (int it = 0; it < 4; ++it) {
+            const int id = it * kThreads + tid, sl = id >> 6, l = id & 63;
+            store_dev(wsc + kWsQ + (size_t)id * 16,
+                      *reinterpret_cast<const uint4*>(sm.Q + tile_off(16 * (sl >> 2) + (l & 15), 4 * (sl & 3) + (l >> 4))));
         }
-    } else {
-        const int ra = 32 * mt + (lane & 31), rb = 32 * nt + (lane & 31);
-        float16_t kk = {}, qk = {};
+    }
+
+    // ---- 2. K K^T and Q K^T, transposed (a lane holds token t = 32 mt + lane % 32 and keys
+    // s = 32 nt + 8 q + 4 hi + 0..3 in registers 4q..4q+3): A goes to LDS in 16-byte pieces, Aqk
+    // straight to the workspace in 8-byte pieces of the carry's operand order ----
+    const bool upper = mt == 0 && nt == 1;
+    const int t = 32 * mt + (lane & 31), rs = 32 * nt + (lane & 31);
+    float16_t kk = {}, qk = {};
+    if (!upper) {
 #pragma unroll
         for (int s = 0; s < kD / 16; ++s) {
             const int c = 2 * s + hi;
-            const half8_t ak = *reinterpret_cast<const half8_t*>(sm.K + tile_off(ra, c));
-            const half8_t bk = *reinterpret_cast<const half8_t*>(sm.K + tile_off(rb, c));
-            kk = mfma32(ak, bk, kk);
-            qk = mfma32(qa[s], bk, qk);
-        }
-        const float Gs = sm.G[rb];
-        const float kns = kFused ? sm.kn[rb] : 1.f;
-        const int sp = perm32(rb);
-        // this lane's rows t = 32mt + 8q + 4hi + 0..3: four 16-byte reads per factor (one
-        // 4-byte read per row had made this phase a chain of ~65 small LDS round trips)
-        float4 g4[4], b4[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int t0q = 32 * mt + 8 * q + 4 * hi;
-            if (!kFused) {
-                g4[q] = *reinterpret_cast<const float4*>(sm.G + t0q);
-                b4[q] = *reinterpret_cast<const float4*>(sm.bt + t0q);
+            const half8_t at = *reinterpret_cast<const half8_t*>(sm.K + tile_off(t, c));
+            const half8_t bs = *reinterpret_cast<const half8_t*>(sm.K + tile_off(rs, c));
+            const half8_t qa = *reinterpret_cast<const half8_t*>(sm.Q + tile_off(t, c));
+            kk = mfma32(bs, at, kk);
+            if (kF32) {
+                kk = mfma32(*reinterpret_cast<const half8_t*>(klo_lds + tile_off(rs, c)), at, kk);
+                kk = mfma32(bs, *reinterpret_cast<const half8_t*>(klo_lds + tile_off(t, c)), kk);
             }
+            qk = mfma32(bs, qa, qk);
         }
-        // A is stored only for blocks (t/16, rb/16) on or below the diagonal; in the one block
-        // above it (mt == nt, rb in the upper half, t in the lower) the lane writes a slot of
-        // sm.bg instead (rewritten in phase 3), so no store needs a branch.  Entries with
-        // rb >= t inside stored diagonal blocks get zeros, which nothing reads.
-        const bool upper = mt == nt && ((lane >> 4) & 1);
+    }
+    lds_barrier();  // every wave's Q reads done: A goes over them
+    if (upper) {
+        // every (t < 32, s >= 32) entry is above the diagonal (the carry reads no Aqk there);
+        // this wave writes the per-token factors instead
+        const float x = sm.G[lane], xc = sm.G[kC - 1];
+        const float ex = __expf(x);
+        const float kn = kFused ? sm.kn[lane] : 1.f, qn = kFused ? sm.qn[lane] : 1.f;
+        float* wg = reinterpret_cast<float*>(wsc + kWsG);
+        store_dev(wg + lane, ex * qn);
+        store_dev(wg + kC + lane, ex * kn);
+        store_dev(wg + 2 * kC + lane, __expf(xc - x) * kn);
+        store_dev(wg + 3 * kC + lane, __expf(xc));
+    } else {
+        const float Gt = sm.G[t];
+        float bt = sm.bt[t], qf = 1.f;
+        if (kFused) {
+            bt *= sm.kn[t];
+            qf = sm.qn[t];
+        }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int q = r >> 2, e = r & 3;
-            const int t = 32 * mt + 8 * q + 4 * hi + e;
-            // the fused variant reads per row (holding the 32 values spills it)
-            const float Gt = kFused ? sm.G[t] : e == 0 ? g4[q].x : e == 1 ? g4[q].y : e == 2 ? g4[q].z : g4[q].w;
-            const float bt = kFused ? sm.bt[t] : e == 0 ? b4[q].x : e == 1 ? b4[q].y : e == 2 ? b4[q].z : b4[q].w;
-            const float dec = (rb <= t) ? __expf(Gt - Gs) : 0.f;
-            float aval = bt * kk[r] * dec, qval = qk[r] * dec;
-            if (kFused) {  // per-row reads here: 16-byte ones would hold 32 more registers
-                aval = bt * kk[r] * (dec * sm.kn[t] * kns);
-                qval = qk[r] * (dec * sm.qn[t] * kns);
+        for (int qd = 0; qd < 4; ++qd) {
+            const int s0 = 32 * nt + 8 * qd + 4 * hi;
+            const float4 g4 = *reinterpret_cast<const float4*>(sm.G + s0);
+            const float gs[4] = {g4.x, g4.y, g4.z, g4.w};
+            float ks[4] = {1.f, 1.f, 1.f, 1.f};
+            if (kFused) {
+                const float4 k4 = *reinterpret_cast<const float4*>(sm.kn + s0);
+                ks[0] = k4.x; ks[1] = k4.y; ks[2] = k4.z; ks[3] = k4.w;
             }
-            float* ap = (upper && r < 8) ? sm.bg + (lane & 63) : sm.x.s.A + tri_off(t, rb);
-            *ap = rb < t ? aval : 0.f;
-            sm.x.s.Aqk[t * kC + sp] = (half_t)qval;
+            float av[4];
+            half4_t qv;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float dec = s0 + e <= t ? __expf(Gt - gs[e]) * ks[e] : 0.f;
+                av[e] = s0 + e < t ? bt * kk[4 * qd + e] * dec : 0.f;
+                qv[e] = (half_t)(qk[4 * qd + e] * (dec * qf));
+            }
+            // blocks above the diagonal (t / 16 < s / 16) are not stored
+            if (mt != nt || qd < 2 || (lane & 16))
+                *reinterpret_cast<float4*>(sm.A + tri_off(t, s0)) = make_float4(av[0], av[1], av[2], av[3]);
+            store_dev8(wsc + kWsAqk + (size_t)((op_slot(t >> 4, nt) * 64 + qd * 16 + (t & 15)) * 16 + 8 * hi),
+                       __builtin_bit_cast(uint2, qv));
         }
     }
     lds_barrier();
 
-    // ---- 3. Aqk out (its staging shares LDS with Tm); wave 1: the decay block and the W
-    // column scale beta e^G (kn); Tm = (I + A)^-1 ----
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-        const int id = it * kThreads + tid;
-        store_dev(wsc + kWsAqk + (size_t)id * 16, *reinterpret_cast<const uint4*>(sm.x.s.Aqk + id * 8));
-    }
-    if (wave == 1) {
-        const float x = sm.G[lane], xc = sm.G[kC - 1];
-        const float ex = __expf(x);
-        const float kn = kFused ? sm.kn[lane] : 1.f, qn = kFused ? sm.qn[lane] : 1.f;
-        sm.bg[lane] = sm.bt[lane] * ex * kn;
-        float* wg = reinterpret_cast<float*>(wsc + kWsG);
-        store_dev(wg + lane, ex * qn);
-        store_dev(wg + kC + lane, __expf(xc - x) * kn);
-        store_dev(wg + 2 * kC + lane, lane == 0 ? __expf(xc) : 0.f);
-        store_dev(wg + 3 * kC + lane, 0.f);
-    }
-    lds_barrier();
+    // ---- 3. Tm = (I + A)^-1 ----
     if (wave == 0) {  // the four 16x16 diagonal blocks, one column per lane
         const int bi = lane >> 4, cj = lane & 15;
         float x[16];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            float acc = (t == cj) ? 1.f : 0.f;
+        for (int t = 0; t < 16; ++t) x[t] = t == cj ? 1.f : 0.f;
+        // row t of the block in 16-byte pieces; every row's earlier columns are known when it
+        // is reached, and its products go to one running sum (s ascending)
 #pragma unroll
-            for (int s = 0; s < t; ++s) acc = fmaf(-sm.x.s.A[tri_off(16 * bi + t, 16 * bi + s)], x[s], acc);
+        for (int t = 1; t < 16; ++t) {
+            float a[16];
+#pragma unroll
+            for (int s4 = 0; s4 < 16; s4 += 4) {
+                if (s4 >= t) break;
+                const float4 v = *reinterpret_cast<const float4*>(sm.A + tri_off(16 * bi + t, 16 * bi + s4));
+                a[s4] = v.x; a[s4 + 1] = v.y; a[s4 + 2] = v.z; a[s4 + 3] = v.w;
+            }
+            float acc = x[t];
+#pragma unroll
+            for (int s = 0; s < t; ++s) acc = fmaf(-a[s], x[s], acc);
             x[t] = acc;
         }
 #pragma unroll
-        for (int t = 0; t < 16; ++t) sm.x.s.Tm[tri_off(16 * bi + t, 16 * bi + cj)] = x[t];
+        for (int t = 0; t < 16; ++t) sm.Tm[tri_off(16 * bi + t, 16 * bi + cj)] = x[t];
     }
     lds_barrier();
     if (wave < 3) {  // block column j = wave: T_ij = -T_ii X, X = sum_{k=j}^{i-1} A_ik T_kj, i > j
@@ -457,147 +449,49 @@ gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k,
             for (int kb = j; kb < i; ++kb)
 #pragma unroll
                 for (int s4 = 0; s4 < 4; ++s4)
-                    x = mfma16f32(sm.x.s.A[tri_off(16 * i + r16, 16 * kb + 4 * s4 + k4)],
-                                  sm.x.s.Tm[tri_off(16 * kb + 4 * s4 + k4, 16 * j + r16)], x);
+                    x = mfma16f32(sm.A[tri_off(16 * i + r16, 16 * kb + 4 * s4 + k4)],
+                                  sm.Tm[tri_off(16 * kb + 4 * s4 + k4, 16 * j + r16)], x);
             float4_t t = {};
 #pragma unroll
             for (int s4 = 0; s4 < 4; ++s4)
-                t = mfma16f32(sm.x.s.Tm[tri_off(16 * i + r16, 16 * i + 4 * k4 + s4)], x[s4], t);
+                t = mfma16f32(sm.Tm[tri_off(16 * i + r16, 16 * i + 4 * k4 + s4)], x[s4], t);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) sm.x.s.Tm[tri_off(16 * i + 4 * k4 + r, 16 * j + r16)] = -t[r];
+            for (int r = 0; r < 4; ++r) sm.Tm[tri_off(16 * i + 4 * k4 + r, 16 * j + r16)] = -t[r];
             wave_lds_sync();
         }
     }
     lds_barrier();
 
-    // ---- 4. W = Tm diag(beta e^G) K and U = Tm diag(beta) V.  The Tm rows become fp16 A
-    // operands in registers; W's products run first, while Tm is still in LDS, then U's
-    // operand is taken as an exact pair of fp16 halves (hi + lo, two MFMAs per step) and V
-    // goes to LDS over A / Tm.  U is kept in fp32 (stored so): rounding its operand or its
-    // value to fp16 were each ~3e-4 of relative state error at T = 4096 ----
-    float16_t u_acc[2];
-    {
-        const int trow = 32 * mt + (lane & 31);
-        const int g16 = lane >> 4;
-        const int nks = mt == 0 ? 2 : 4;  // Tm[t < 32][s >= 32] = 0
-        // the 8 Tm values of this lane's operand slots at k-step ks, zero above the diagonal
-        auto tm_row = [&](int ks, float (&x)[8]) {
-            // block (trow/16, ks) lies above the diagonal for ks > trow/16: Tm is zero there
-            // and the masked read below goes to a stored block instead
-            const int base = tri_off(trow, 16 * min(ks, trow >> 4) + 8 * hi);
-            const float4 t0v = *reinterpret_cast<const float4*>(&sm.x.s.Tm[base]);
-            const float4 t1v = *reinterpret_cast<const float4*>(&sm.x.s.Tm[base ^ 4]);
-            const float tv[8] = {t0v.x, t0v.y, t0v.z, t0v.w, t1v.x, t1v.y, t1v.z, t1v.w};
+    // ---- 4. T' = Tm diag(beta) as an exact pair of fp16 halves, in the carry's operand order
+    // (slot (w, ks), lane (g, c): T'[16 w + c][32 ks + 8 g .. + 7]) ----
 #pragma unroll
-            for (int qd = 0; qd < 8; ++qd) x[qd] = (16 * ks + 8 * hi + qd <= trow) ? tv[qd] : 0.f;
-        };
-        {
-            // With fp32 I/O, W's A operand Tm diag(beta e^G) is taken as an exact pair of fp16
-            // halves (two MFMAs per step): with the carry's W S state operand also split, the
-            // state error of a slowly decaying gate halves (numpy model: 4.6e-5 -> 2.2e-5 at
-            // T = 2048).  The fp16-I/O path keeps one operand: the pair cost 3 % of a call at
-            // 32 heads, T = 4096 (A/B on one box).  One output tile at a time, its Tm operands
-            // re-read per tile: two accumulators and a second operand would not fit the 128
-            // registers of four workgroups per CU.
-            float16_t w_acc[2];
-#pragma unroll
-            for (int n2 = 0; n2 < 2; ++n2) {
-                const int ntw = 2 * (wave & 1) + n2;
-                w_acc[n2] = float16_t{};
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    if (ks >= nks) break;
-                    float x[8];
-                    tm_row(ks, x);
-                    half8_t awh, awl;
-#pragma unroll
-                    for (int qd = 0; qd < 8; ++qd) {
-                        const float y = x[qd] * sm.bg[16 * ks + 8 * hi + qd];
-                        awh[qd] = (half_t)y;
-                        awl[qd] = (half_t)(y - (float)awh[qd]);
-                    }
-                    const int row0 = 16 * ks + 8 * hi;
-                    const int col0 = 32 * ntw + 16 * (g16 & 1);
-                    const half8_t bk = cat8(tile_read_tr(sm.K, row0, col0), tile_read_tr(sm.K, row0 + 4, col0));
-                    w_acc[n2] = mfma32(awh, bk, w_acc[n2]);
-                    if (kF32) w_acc[n2] = mfma32(awl, bk, w_acc[n2]);
-                }
-            }
-            lds_barrier();  // every wave's K reads done: W is staged over K
-#pragma unroll
-            for (int n2 = 0; n2 < 2; ++n2) {
-                const int cp = perm32(32 * (2 * (wave & 1) + n2) + (lane & 31));
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int t = 32 * mt + 8 * (r >> 2) + 4 * hi + (r & 3);
-                    sm.K[t * kD + cp] = (half_t)w_acc[n2][r];
-                }
-            }
-        }
-        half8_t au[4], al[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            if (ks >= nks) break;
-            float x[8];
-            tm_row(ks, x);
-#pragma unroll
-            for (int qd = 0; qd < 8; ++qd) {
-                const float y = x[qd] * sm.bt[16 * ks + 8 * hi + qd];
-                au[ks][qd] = (half_t)y;
-                al[ks][qd] = (half_t)(y - (float)au[ks][qd]);
-            }
-        }
-        lds_barrier();
-#pragma unroll
-        for (int it = 0; it < 4; ++it) {  // V rows past T (loaded from the last row) are zero
-            const int id = it * kThreads + tid;
-            const bool past = t0 + (id >> 4) > lastt;
-            *reinterpret_cast<uint4*>(sm.x.V + tile_off(id >> 4, id & 15)) = past ? make_uint4(0, 0, 0, 0) : vreg[it];
-            if (kF32)
-                *reinterpret_cast<uint4*>(vlo_lds + tile_off(id >> 4, id & 15)) = past ? make_uint4(0, 0, 0, 0) : vlo[it];
-        }
-        lds_barrier();
-#pragma unroll
-        for (int n2 = 0; n2 < 2; ++n2) {
-            const int ntw = 2 * (wave & 1) + n2;
-            u_acc[n2] = float16_t{};
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                if (ks >= nks) break;
-                const int row0 = 16 * ks + 8 * hi;
-                const int col0 = 32 * ntw + 16 * (g16 & 1);
-                const half8_t bv = cat8(tile_read_tr(sm.x.V, row0, col0), tile_read_tr(sm.x.V, row0 + 4, col0));
-                u_acc[n2] = mfma32(au[ks], bv, u_acc[n2]);
-                u_acc[n2] = mfma32(al[ks], bv, u_acc[n2]);
-                if (kF32) {  // the low half of the fp32 V (lo x lo is below fp32 rounding)
-                    const half8_t bvl = cat8(tile_read_tr(vlo_lds, row0, col0), tile_read_tr(vlo_lds, row0 + 4, col0));
-                    u_acc[n2] = mfma32(au[ks], bvl, u_acc[n2]);
-                }
-            }
-        }
-    }
-
-    // ---- 5. U stored from registers in fp32 (registers 4a..4a+3 are tokens t0..t0+3 of one
-    // column: one 16-byte slot of the carry's layout); W from its staging, 16-byte stores ----
-#pragma unroll
-    for (int n2 = 0; n2 < 2; ++n2) {
-        const int col = 32 * (2 * (wave & 1) + n2) + (lane & 31);
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const int t0 = 32 * mt + 8 * a + 4 * hi;
-            const int slot = ((col >> 4) * 4 + (t0 >> 4)) * 64 + ((t0 >> 2) & 3) * 16 + (col & 15);
-            store_dev(wsc + kWsU + (size_t)slot * 16,
-                      make_uint4(__float_as_uint(u_acc[n2][4 * a]), __float_as_uint(u_acc[n2][4 * a + 1]),
-                                 __float_as_uint(u_acc[n2][4 * a + 2]), __float_as_uint(u_acc[n2][4 * a + 3])));
-        }
-    }
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
+    for (int it = 0; it < 2; ++it) {
         const int id = it * kThreads + tid;
-        store_dev(wsc + kWsW + (size_t)id * 16, *reinterpret_cast<const uint4*>(sm.K + id * 8));
+        if (id >= kTSlots * 64) break;
+        const int sl = id >> 6, l = id & 63;
+        const int w = sl < 2 ? sl : 2 + ((sl - 2) >> 1), ks = sl < 2 ? 0 : (sl - 2) & 1;
+        const int t = 16 * w + (l & 15), s0 = 32 * ks + 8 * (l >> 4);
+        // a block above the diagonal is zero; the read goes to a stored block instead
+        const int base = tri_off(t, 16 * min(s0 >> 4, t >> 4) + (s0 & 8));
+        const float4 t0v = *reinterpret_cast<const float4*>(&sm.Tm[base]);
+        const float4 t1v = *reinterpret_cast<const float4*>(&sm.Tm[base ^ 4]);
+        const float4 b0v = *reinterpret_cast<const float4*>(sm.bt + s0);
+        const float4 b1v = *reinterpret_cast<const float4*>(sm.bt + s0 + 4);
+        const float tv[8] = {t0v.x, t0v.y, t0v.z, t0v.w, t1v.x, t1v.y, t1v.z, t1v.w};
+        const float bv[8] = {b0v.x, b0v.y, b0v.z, b0v.w, b1v.x, b1v.y, b1v.z, b1v.w};
+        half8_t th, tl;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float y = rounded(s0 + e <= t ? tv[e] * bv[e] : 0.f);
+            th[e] = (half_t)y;
+            tl[e] = (half_t)(y - (float)th[e]);
+        }
+        const size_t o = (size_t)id * 16;
+        store_dev(wsc + kWsT + o, __builtin_bit_cast(uint4, th));
+        store_dev(wsc + kWsTlo + o, __builtin_bit_cast(uint4, tl));
     }
 
-    // ---- 6. publish (beside the carry only): every wave's device-scope stores complete, then
+    // ---- 5. publish (beside the carry only): every wave's device-scope stores complete, then
     // the chunk's flag.  In order the kernel boundary orders the stores before the carry, so
     // the workgroup ends without waiting for them ----
     if (flags) {
@@ -611,493 +505,112 @@ gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k,
 // ----------------------------------------------------------------------------------
 // Carry
 // ----------------------------------------------------------------------------------
-struct ChainSlot {                   // operands of the loop-carried part of one chunk
-    half_t K[kC * kD];               // K rows, swizzled (read transposed by the update)
-    half_t W[kC * kD];               // W rows (perm32 columns), swizzled
-    float U[kStrips * 4 * 64 * 4];   // this workgroup's two U strips (fp32), accumulator order
-    float E[kC];                     // e^{G_t} qn_t (the output's factor; unused here)
-    float Dg[kC];                    // e^{G_63 - G_t} kn_t
-    float Ec[2 * kC];                // e^{G_63} (the chunk's decay), then zeros
+// One workgroup of 8 waves per (b, h, 16 NC state columns), sequential over chunks.
+//
+// Chain waves 0-3 run the loop-carried part.  Wave w owns tokens 16 w .. + 15 of the chunk (rows
+// of K S and T' R) and state rows dk 32 w .. + 31 (fp32 accumulators) for all of the workgroup's
+// columns, so it reads a quarter of each operand; what the waves exchange goes through LDS in
+// operand order (16-byte lane-linear reads).  Per chunk, a barrier after each:
+//   1  X = K S, R = V - e^G X as fp16 hi + lo -> LDS
+//   2  Vnew = T' R (hi hi + lo hi + hi lo); Vnew and Vnew e^{G_63 - G} (hi + lo) -> LDS
+//   3  S = e^{G_63} S + K^T (hi + lo); S -> LDS as fp16
+// Helper waves 4-7 do everything that touches memory, in the same three intervals: wave w's
+// output tokens are 16 w .. + 15.
+//   1  the next chunk's K, V and factors from registers to LDS
+//   2  its T'; (Q S)^T for the wave's tokens
+//   3  O = e^G Q S + Aqk Vnew, stored
+// Every operand is loaded into registers two or three chunks before its use and its registers are reloaded as soon as they are free, a few loads in each interval: a wave that
+// issues loads stalls at issue while the CU's 64 B/clk load path is busy (~50 KB per chunk, 800
+// cycles), which in the chain waves cost 1.6 us per chunk instead of the chain's own time.
+template <typename TIO, int NC>
+struct CarrySlot {                      // a chunk's operands of the chain waves
+    static constexpr bool kF32 = std::is_same<TIO, float>::value;
+    half_t K[(kF32 ? 2 : 1) * kC * kD]; // K rows, swizzled (fp32 I/O: then their low halves)
+    uint4 T[kTSlots * 2 * 64];          // T' hi, lo in operand order
+    TIO V[kC * 16 * NC];                // [token][column index 4 NC (i / 4) ...] as in memory
+    float G[4 * kC];                    // the per-token factors
 };
-struct OutSlot {                     // operands of the output of one chunk
-    half_t Q[kC * kD];               // Q rows, swizzled
-    half_t A[kC * kC];               // Aqk rows (perm32 columns), 8-chunk swizzle
-    float E[kC];                     // e^{G_t} qn_t (followed in the workspace by e^{G_63 - G_t} kn_t)
-    float Dg[kC];
-};
+template <typename TIO, int NC>
 struct CarryLds {
-    ChainSlot cs[2];
-    OutSlot os[2];
-    uint4 XS[2][kStrips][6][64];     // chain -> output: S operands (4) and Vnew operands (2)
-    half_t OS[2][32 * 32];           // per output wave: its 32 tokens x 32 columns of O
-    int err[4];                      // per DMA wave: a ready wait timed out
+    static constexpr bool kF32 = std::is_same<TIO, float>::value;
+    CarrySlot<TIO, NC> c[2];
+    uint4 S[kF32 ? 2 : 1][NC][4][64];   // state operand, k-step, lane (fp32 I/O: hi, lo)
+    uint4 R[2][NC][2][64];              // R hi, lo
+    uint4 V[3][NC][2][64];              // Vnew e^{G_63 - G} hi, lo; Vnew
+    int err[4];                         // per helper wave: a ready wait timed out
 };
 
-// 16-B chunk swizzle of the [64][64] Aqk tile: 16 consecutive rows at one chunk are
-// conflict free (two rows share a 256-B bank period).
-__device__ __forceinline__ int aqk_off(int r, int c) {
-    return r * kC + ((c ^ ((r >> 1) & 7)) << 3);
+__device__ __forceinline__ uint4 bload4(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+// workspace loads beside the prep are device-scope (sc1), the counterpart of its stores
+template <bool kDev>
+__device__ __forceinline__ uint4 bload4w(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kDev ? 16 : 0));
+}
+template <bool kDev>
+__device__ __forceinline__ float bload1w(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, kDev ? 16 : 0));
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
 }
 
-typedef __attribute__((address_space(3))) void* lds_void_t;
-
-// Per-chunk copies into LDS: 66 one-KiB LDS-DMA instructions (global_load_lds_dwordx4,
-// lane l copies 16 bytes to M0 + 16*l).  Instruction n < 41 fills the chain slot at byte
-// 1024*n (K tile n < 16, W tile, fp32 U strips 32..39, decay block 40); n >= 41 fills the out
-// slot at byte 1024*(n-41) (Q tile, Aqk tile, E/Dg 65).  The structs' members are laid out in that
-// order so that the LDS offset is just 1024 * tile index.  The four DMA waves (4-7) take
-// n = w + 4j; each lane's source offset for its instructions is fixed for the whole loop
-// and computed once, so an instruction costs a scalar M0 write and the DMA itself.
-constexpr int kDmaN = 66, kDmaChain = 41;
-constexpr int kDmaEOut = 65;  // a 512-byte copy: lanes 0-31 only
-// With fp32 I/O the output waves load their operands from memory into registers and the out
-// slots hold instead the low halves of the chain chunk's K rows (K_lo, 16 KiB): instructions
-// 41 .. 56 copy them, swizzled like K, from the chunk's workspace.
-constexpr int kDmaNF32 = kDmaChain + 16;
-template <bool kF32> constexpr int dma_n() { return kF32 ? kDmaNF32 : kDmaN; }
-__device__ __forceinline__ unsigned dma_src_off_klo(int i, int lane) {
-    const int P = i * 64 + lane, row = P >> 4, cch = (P & 15) ^ swz(row);
-    return kWsKlo + row * kD * 2 + cch * 16;
+// 4 fp32 values as 4 fp16 highs and 4 fp16 lows.
+__device__ __forceinline__ void split4(const float4_t& x, uint2& hi, uint2& lo) {
+    half4_t h, l;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float y = rounded(x[r]);
+        h[r] = (half_t)y;
+        l[r] = (half_t)(y - (float)h[r]);
+    }
+    hi = __builtin_bit_cast(uint2, h);
+    lo = __builtin_bit_cast(uint2, l);
 }
 
-// Source byte offset of instruction n for this lane, from the instruction's base pointer:
-// the row base of the chunk's first token (K / Q tiles, rows at rowbytes apart, rows
-// past `lastrow` clamped to it: they only meet zero coefficients) or the chunk's workspace.
-__device__ __forceinline__ unsigned dma_src_off(int n, int lane, unsigned rowbytes, int pair, int lastrow) {
-    const int i = n < kDmaChain ? n : n - kDmaChain;
-    const bool chainslot = n < kDmaChain;
-    if (i < 16) {                                    // K or Q rows, swizzled 16-B chunks
-        const int P = i * 64 + lane, row = P >> 4, cch = (P & 15) ^ swz(row);
-        return (unsigned)min(row, lastrow) * rowbytes + cch * 16;
-    }
-    if (chainslot) {
-        if (i < 32) {                                // W rows, swizzled
-            const int P = (i - 16) * 64 + lane, row = P >> 4, cch = (P & 15) ^ swz(row);
-            return kWsW + (row * kD + cch * 8) * 2;
-        }
-        if (i < 40) return kWsU + pair * 8192 + (i - 32) * 1024 + lane * 16;  // own U strips
-        return kWsG + lane * 16;                     // the whole 1-KiB decay block
-    }
-    if (i < 24) {                                    // Aqk rows, 8-chunk swizzle
-        const int P = (i - 16) * 64 + lane, row = P >> 3, cch = (P & 7) ^ ((row >> 1) & 7);
-        return kWsAqk + (row * kC + cch * 8) * 2;
-    }
-    return kWsG + (lane & 31) * 16;
-}
+// Keeps the loads after it behind the products that make x.  Every reload must stay behind the
+// last use of what it replaces: with a use left below it the compiler takes other registers for
+// the new value and copies them at the loop's end, waiting for a load just issued.
+__device__ __forceinline__ void pin(float4_t& x) { asm volatile("" : "+v"(x)::"memory"); }
 
-// Issue instruction n: src = base + off (saddr form: 64-bit base in SGPRs, 32-bit VGPR
-// offset).  Written as inline asm on purpose: the compiler does not track LDS written by
-// DMA slot by slot and would wait for every DMA in flight before the first LDS read of the
-// other slot; the kernel orders the copies and the reads itself (dma_wait_barrier).
-// Workspace tiles (dev) are device-scope loads (sc1), the counterpart of the prep's stores.
-__device__ __forceinline__ void dma_issue(const void* base, unsigned off, unsigned lds_addr, bool half,
-                                          bool dev) {
-    if (!half || (threadIdx.x & 63) < 32) {
-        if (dev)
-            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 sc1" :: "v"(off), "s"(base),
-                         "{m0}"(lds_addr) : "memory");
-        else
-            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(base),
-                         "{m0}"(lds_addr) : "memory");
-    }
-}
-
-// Wait for this wave's copies (vmcnt counts them), then a barrier over LDS: after it every
-// wave sees every wave's copies.
-__device__ __forceinline__ void dma_wait_barrier() {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0); expcnt, lgkmcnt left at their maxima
-    lds_barrier();
-}
-
-// The loop of DMA wave W (0..3): instruction n = W + 4j is a constant in each unrolled
-// step, so its kind, base pointer and LDS address fold.  Iteration it copies the chain
-// operands of chunk it+1 into cs[(it+1)&1] and the output operands of chunk it into
-// os[it&1] (the prologue: chunk 0 into cs[0]), then waits for them and meets the barrier.
-// A chunk that ends past T recomputes its K / Q offsets with clamped rows.
-// kh / qh: the K / Q rows of chunk 0 (the inputs' rows, or with kF32 the fp16 copies in the
-// workspace, which the prep writes in this call and are therefore read device-scope), with
-// rowbytes between rows and chunk_bytes between chunks.
-template <int W, bool kF32>
-__device__ __forceinline__ void dma_role(const unsigned (&slot_lds)[4], const unsigned char* kh,
-                                         const unsigned char* qh, const unsigned char* wsh,
-                                         const unsigned* fl, unsigned wait_ticks,
-                                         int* err, unsigned rowbytes, size_t chunk_bytes, int pair,
-                                         int T, int nch) {
-    constexpr int kJ = (dma_n<kF32>() - W + 3) / 4;
-    const int lane = threadIdx.x & 63;
-    unsigned off[kJ];
-#pragma unroll
-    for (int j = 0; j < kJ; ++j) {
-        const int n = W + 4 * j;
-        off[j] = kF32 && n >= kDmaChain ? dma_src_off_klo(n - kDmaChain, lane)
-                                        : dma_src_off(n, lane, rowbytes, pair, kC - 1);
-    }
-    // slot_lds: cs[0], cs[1], os[0], os[1]
-    auto copies = [&](int pc, int po, int cn, int co) {
-        const bool do_c = cn < nch, do_o = co >= 0 && co < nch;
-        const int last_c = min(kC - 1, T - 1 - cn * kC), last_o = min(kC - 1, T - 1 - co * kC);
-        const unsigned char* kb = kh + (size_t)cn * chunk_bytes;
-        const unsigned char* wc = wsh + (size_t)cn * ws_chunk<kF32>();
-        const unsigned char* qb = qh + (size_t)co * chunk_bytes;
-        const unsigned char* wo = wsh + (size_t)co * ws_chunk<kF32>();
-        auto issue_all = [&](auto Ragged) {
-#pragma unroll
-            for (int j = 0; j < kJ; ++j) {
-                const int n = W + 4 * j;
-                const bool chainslot = n < kDmaChain;
-                const int i = chainslot ? n : n - kDmaChain;
-                if (kF32 && !chainslot) {  // K_lo rows of the chain chunk, into its parity's out slot
-                    if (do_c) dma_issue(wc, off[j], slot_lds[2 + pc] + 1024u * i, false, true);
-                    continue;
-                }
-                const bool rows = i < 16;
-                if (chainslot ? !do_c : !do_o) continue;
-                unsigned o = off[j];
-                if (decltype(Ragged)::value && rows)
-                    o = dma_src_off(n, lane, rowbytes, pair, chainslot ? last_c : last_o);
-                const unsigned char* base = chainslot ? (rows ? kb : wc) : (rows ? qb : wo);
-                const unsigned lds = (chainslot ? slot_lds[pc] : slot_lds[2 + po]) + 1024u * i;
-                dma_issue(base, o, lds, n == kDmaEOut, kF32 || !rows);
-            }
-        };
-        if ((do_c && last_c < kC - 1) || (do_o && last_o < kC - 1))
-            issue_all(std::true_type{});
-        else
-            issue_all(std::false_type{});
-    };
-    // fl[n] is chunk n's flag (device-scope loads, like the workspace copies that follow
-    // it).  The flag of the next chunk is loaded right after a chunk's copies are issued, so
-    // its round trip overlaps them and a chunk that is ready costs no wait.  After one
-    // timed-out wait, no more waits (the workgroup's results are then discarded).
-    auto peek = [&](int n) -> unsigned {
-        if (!fl) return 1u;  // in order after the prep: every chunk is ready
-        return n < nch ? __hip_atomic_load(fl + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-    };
-    // real-time counter (100 MHz), low 32 bits; readfirstlane keeps the wait loop uniform
-    auto now = []() { return __builtin_amdgcn_readfirstlane((unsigned)__builtin_amdgcn_s_memrealtime()); };
-    auto ready = [&](int n, unsigned v) {
-        v = __builtin_amdgcn_readfirstlane(v);
-        if (v != 0u || *err) return;
-        const unsigned t0 = now();
-        while (v == 0u) {
-            if (now() - t0 >= wait_ticks) {
-                *err = 1;
-                return;
-            }
-            __builtin_amdgcn_s_sleep(8);
-            v = __builtin_amdgcn_readfirstlane(
-                __hip_atomic_load(fl + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        }
-    };
-    *err = 0;
-    ready(0, peek(0));
-    copies(0, 0, 0, -1);
-    unsigned nxt = peek(1);
-    dma_wait_barrier();
-    for (int it = 0; it <= nch; it += 2) {
-        if (it + 1 < nch) ready(it + 1, nxt);
-        copies(1, 0, it + 1, it);
-        nxt = peek(it + 2);
-        dma_wait_barrier();
-        if (it + 1 > nch) break;
-        if (it + 2 < nch) ready(it + 2, nxt);
-        copies(0, 1, it + 2, it + 1);
-        nxt = peek(it + 3);
-        dma_wait_barrier();
-    }
-}
-
-
-// Per-lane LDS offsets (in halfs, within a tile) of the chain step's operand reads.  The
-// swizzle makes them lane-dependent, but row-tile and slot steps are constant, so with
-// these bases every read in the loop is a base register plus an immediate.
-struct ChainOffs {
-    int w[4];   // W operand, k-step kk, row tile 0 (row tile mt adds 16 * mt * kD)
-    int k[8];   // K^T operand, row tile m of S, token rows 4g.. (token block ks adds 32*ks*kD)
-};
-__device__ __forceinline__ ChainOffs chain_offs() {
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, i16 = lane & 15;
-    ChainOffs o;
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) o.w[kk] = tile_off(c, 4 * kk + g);
-    const int r = 4 * g + (i16 >> 2);  // token row this lane supplies to the transposed read
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const int col = 16 * m + 4 * (i16 & 3);
-        o.k[m] = tile_off(r, col >> 3) + (col & 7);
-    }
-    return o;
-}
-
-// Chain step for one chunk: strip S (fp32 accumulators) <- next state, and the S / Vnew
-// operands handed to the output waves in XS.  Every LDS read of the step (W and K^T
-// operands, U, decay factors) depends only on the chunk's slot, so all of them are issued
-// before the first MFMA and a scheduling barrier keeps them there: the MFMAs then find
-// their operands arriving in order instead of waiting on each small batch.
-// us: 1, or 0 for a transition map's chain (U = 0).
-// kLo (fp32 I/O): klo is the chunk's K_lo tile, and the update takes K as an exact hi + lo
-// pair (rounding the fp32 K to one fp16 operand there was ~2.3e-4 of relative state error on
-// the reference's own inputs, numpy model); W S takes the state as hi + lo too (see below).
-template <bool kLo>
-__device__ __forceinline__ void chain_step(float4_t (&S)[8], const ChainSlot& cs, uint4* xs, int sl,
-                                           const ChainOffs& off, float us, const half_t* klo) {
-    const int lane = threadIdx.x & 63, g = lane >> 4;
-    half8_t aW[4][4];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-            aW[mt][kk] = *reinterpret_cast<const half8_t*>(cs.W + off.w[kk] + 16 * mt * kD);
-    float4 u[4], d4[4];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-        u[mt] = *reinterpret_cast<const float4*>(cs.U + ((sl * 4 + mt) * 64 + lane) * 4);
-        d4[mt] = *reinterpret_cast<const float4*>(cs.Dg + 16 * mt + 4 * g);
-    }
-    const float eGC = cs.Ec[0];
-    // K^T operands of the state update, read transposed
-    half8_t aK[8][2];
-#pragma unroll
-    for (int m = 0; m < 8; ++m)
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-            aK[m][ks] = cat8(lds_read_tr16(cs.K + off.k[m] + 32 * ks * kD),
-                             lds_read_tr16(cs.K + off.k[m] + (32 * ks + 16) * kD));
-    __builtin_amdgcn_sched_barrier(0);
-
-    half8_t Sb[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-        Sb[kk] = half8_t{(half_t)S[2 * kk][0], (half_t)S[2 * kk][1], (half_t)S[2 * kk][2], (half_t)S[2 * kk][3],
-                         (half_t)S[2 * kk + 1][0], (half_t)S[2 * kk + 1][1], (half_t)S[2 * kk + 1][2], (half_t)S[2 * kk + 1][3]};
-    // W S, the four row-tile chains interleaved.  With fp32 I/O (kLo) the state operand is an
-    // exact pair of fp16 halves (hi + lo, a second MFMA per step reusing the W operand; with W's
-    // own A operand split in the prep, the state error of a slowly decaying gate halves, numpy
-    // model); the low halves are formed one k-step at a time, next to their MFMAs.  The fp16-I/O
-    // path keeps one operand: the pair put 16 MFMAs on the chunk step's dependency chain
-    // (+16 % per call at 32 heads, T = 4096, A/B on one box).
-    float4_t wsv[4] = {float4_t{}, float4_t{}, float4_t{}, float4_t{}};
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-        half8_t Sl;
-        if (kLo) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) Sl[e] = (half_t)(S[2 * kk + (e >> 2)][e & 3] - (float)Sb[kk][e]);
-        }
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            wsv[mt] = mfma16(aW[mt][kk], Sb[kk], wsv[mt]);
-            if (kLo) wsv[mt] = mfma16(aW[mt][kk], Sl, wsv[mt]);
-        }
-    }
-    // Vnew = U - W S (lane: column c, tokens 16mt + 4g + r); Vs = Vnew e^{G_C - G_t} as an
-    // exact pair of fp16 halves (hi + lo): its rounding to one fp16 operand was ~3e-4 of
-    // relative state error at T = 4096; the second MFMA per step reuses the K^T operand
-    half8_t Vn[2], Vs[2], Vl[2];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-        const float uu[4] = {u[mt].x, u[mt].y, u[mt].z, u[mt].w};
-        const float dg[4] = {d4[mt].x, d4[mt].y, d4[mt].z, d4[mt].w};
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float vn = fmaf(uu[r], us, -wsv[mt][r]);
-            Vn[mt >> 1][4 * (mt & 1) + r] = (half_t)vn;
-            const float vs = vn * dg[r];
-            const half_t vh = (half_t)vs;
-            Vs[mt >> 1][4 * (mt & 1) + r] = vh;
-            Vl[mt >> 1][4 * (mt & 1) + r] = (half_t)(vs - (float)vh);
-        }
-    }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) xs[kk * 64 + lane] = __builtin_bit_cast(uint4, Sb[kk]);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) xs[(4 + ks) * 64 + lane] = __builtin_bit_cast(uint4, Vn[ks]);
-    // S = e^{G_C} S + K^T (Vs hi + Vs lo)
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        S[m] *= eGC;
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            S[m] = mfma16(aK[m][ks], Vs[ks], S[m]);
-            S[m] = mfma16(aK[m][ks], Vl[ks], S[m]);
-        }
-    }
-    // + K_lo^T Vs hi, one row tile's operands read at a time (the registers of the hoisted K^T
-    // reads above are all in use)
-    if (kLo) {
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                const half8_t aKl = cat8(lds_read_tr16(klo + off.k[m] + 32 * ks * kD),
-                                         lds_read_tr16(klo + off.k[m] + (32 * ks + 16) * kD));
-                S[m] = mfma16(aKl, Vs[ks], S[m]);
-            }
-        }
-    }
-}
-
-// A operands of one output wave's chunk: Q (token tiles 2w, 2w+1, in the state operand's
-// k order), Aqk (perm32 columns) and the factors e^{G_t} qn_t of its D rows.
-struct OutOps {
-    half8_t aQ[2][4], aA[2][2];
-    float4 eg[2];
-};
-// from the chunk's out slot in LDS (fp16 I/O)
-__device__ __forceinline__ OutOps out_ops_lds(const OutSlot& os, int w) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    OutOps op;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int t = 16 * (2 * w + j) + c;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const half4_t lo = *reinterpret_cast<const half4_t*>(
-                os.Q + t * kD + (((4 * kk + (g >> 1)) ^ swz(t)) << 3) + 4 * (g & 1));
-            const half4_t up = *reinterpret_cast<const half4_t*>(
-                os.Q + t * kD + (((4 * kk + 2 + (g >> 1)) ^ swz(t)) << 3) + 4 * (g & 1));
-            op.aQ[j][kk] = cat8(lo, up);
-        }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-            op.aA[j][ks] = *reinterpret_cast<const half8_t*>(os.A + aqk_off(t, 4 * ks + g));
-        op.eg[j] = *reinterpret_cast<const float4*>(os.E + 16 * (2 * w + j) + 4 * g);
-    }
-    return op;
-}
-// from the chunk's workspace (fp32 I/O: the prep's fp16 Q rows, unswizzled)
-__device__ __forceinline__ OutOps out_ops_mem(const unsigned char* wsc, int w) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    const half_t* Q = reinterpret_cast<const half_t*>(wsc + kWsQ);
-    const half_t* A = reinterpret_cast<const half_t*>(wsc + kWsAqk);
-    const float* E = reinterpret_cast<const float*>(wsc + kWsG);
-    OutOps op;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int t = 16 * (2 * w + j) + c;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-            op.aQ[j][kk] = cat8(*reinterpret_cast<const half4_t*>(Q + t * kD + 32 * kk + 4 * g),
-                                *reinterpret_cast<const half4_t*>(Q + t * kD + 32 * kk + 16 + 4 * g));
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-            op.aA[j][ks] = *reinterpret_cast<const half8_t*>(A + t * kC + 8 * (4 * ks + g));
-        op.eg[j] = *reinterpret_cast<const float4*>(E + 16 * (2 * w + j) + 4 * g);
-    }
-    return op;
-}
-
-// Output for one chunk, token tiles {2w, 2w+1} of both strips: O = scale (e^G Q S + Aqk Vnew).
-// With TIO = float the values go straight to the fp32 output (o32: this wave's first token
-// row of the chunk and the workgroup's first column; rows past T are skipped) instead of
-// through the fp16 staging tile.
-template <typename TIO>
-__device__ __forceinline__ void out_step(const OutOps& op, const uint4 (*xs)[6][64], half_t* ostage,
-                                         int w, float scale, float* o32, size_t o32_row, int rows_left) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    float eg[2][4];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        eg[j][0] = op.eg[j].x; eg[j][1] = op.eg[j].y; eg[j][2] = op.eg[j].z; eg[j][3] = op.eg[j].w;
-    }
-    half8_t Sb[kStrips][4], Vn[kStrips][2];
-#pragma unroll
-    for (int s = 0; s < kStrips; ++s) {
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) Sb[s][kk] = __builtin_bit_cast(half8_t, xs[s][kk][lane]);
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) Vn[s][ks] = __builtin_bit_cast(half8_t, xs[s][4 + ks][lane]);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // every LDS read of the step ahead of the MFMAs
-    float4_t qs[2][kStrips], av[2][kStrips];
-#pragma unroll
-    for (int s = 0; s < kStrips; ++s) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            qs[j][s] = float4_t{};
-            av[j][s] = float4_t{};
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) qs[j][s] = mfma16(op.aQ[j][kk], Sb[s][kk], qs[j][s]);
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) av[j][s] = mfma16(op.aA[j][ks], Vn[s][ks], av[j][s]);
-        }
-    }
-    if (std::is_same<TIO, float>::value) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int tl = 16 * j + 4 * g + r;  // token within this wave's 32
-                if (tl < rows_left)
-#pragma unroll
-                    for (int s = 0; s < kStrips; ++s)
-                        o32[tl * o32_row + 16 * s + c] = scale * fmaf(eg[j][r], qs[j][s][r], av[j][s][r]);
-            }
-        return;
-    }
-    // O tile (32 tokens x 32 columns) staged in LDS; out_flush stores it
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int s = 0; s < kStrips; ++s)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                ostage[(16 * j + 4 * g + r) * 32 + 16 * s + c] =
-                    (half_t)(scale * fmaf(eg[j][r], qs[j][s][r], av[j][s][r]));
-}
-
-// 16-byte stores of a staged O tile (tokens t0 + 32w .. +31, columns pair*32 .. +31).
-// Called one iteration after out_step, so the stores drain behind a whole iteration of
-// work instead of in front of the next barrier.
-__device__ __forceinline__ void out_flush(const half_t* ostage, half_t* out, int b, int T, int Hv,
-                                          int h, int t0, int pair, int w, int Tloc) {
-    const int lane = threadIdx.x & 63;
-    wave_lds_sync();
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-        const int tl = 16 * hf + (lane >> 2);  // token within this wave's 32
-        const int tt = t0 + 32 * w + tl;
-        const uint4 v4 = *reinterpret_cast<const uint4*>(ostage + tl * 32 + 8 * (lane & 3));
-        if (tt < Tloc)
-            *reinterpret_cast<uint4*>(out + (((size_t)b * T + tt) * Hv + h) * kD + pair * 32 + 8 * (lane & 3)) = v4;
-    }
-    wave_lds_sync();
-}
-
-// TIO: the q / k / out element type.  With fp32 I/O the K / Q rows come from the prep's fp16
-// copies in the workspace and the output is stored in fp32 straight from registers.
-// job: the whole sequence (kJobPlain), or one launch of the sequence split (segments of the
+// TIO: the q / k / v / out element type.  NC: 16-column tiles of the workgroup.  kFlags: the
+// call runs beside the prep (or is its second launch) and waits on the chunks' ready flags.
+// job: the whole sequence (kJobPlain), or the maps launch of the sequence split (segments of the
 // workgroup's unit, its start state and where its end state goes are derived below).
-template <typename TIO>
-__global__ void __launch_bounds__(kCarryThreads, 1)
-gdn_chunk_carry(const TIO* __restrict__ q, const TIO* __restrict__ k,
-                const unsigned char* __restrict__ ws, const unsigned* __restrict__ flags,
-                unsigned* __restrict__ aborts, int mode, unsigned wait_ticks,
-                float* __restrict__ state,
-                TIO* __restrict__ out, int T, int Hq, int Hv, int nch_all, int BHv, float scale,
-                CarryJob job) {
+// One workgroup per CU: two waves per SIMD, one of each role.
+template <typename TIO, int NC, bool kFlags>
+__global__ void __launch_bounds__(kCarryThreads, 2)
+gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws, const unsigned* __restrict__ flags,
+                unsigned* __restrict__ aborts, int mode, unsigned wait_ticks, float* __restrict__ state,
+                TIO* __restrict__ out, int T, int Hq, int Hv, int nch_all, int BHv, float scale, CarryJob job) {
     constexpr bool kF32 = std::is_same<TIO, float>::value;
-    __shared__ CarryLds sm;
-    if (mode == kCarryRetry &&
-        __builtin_amdgcn_readfirstlane(__hip_atomic_load(aborts + blockIdx.x, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT)) == 0u)
-        return;  // this workgroup finished in the launch beside the prep
+    constexpr int kWgs = kD / (16 * NC);  // workgroups per head
+    __shared__ __align__(16) CarryLds<TIO, NC> sm;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: role branches are scalar
+    const bool chain = wave < 4;
+    const int w = wave & 3;
     const int g = lane >> 4, c = lane & 15;
-    // block id = (unit * 4 + pair) * BHv + bh: all column pairs of one head share an XCD when
-    // BHv % 8 == 0
-    const int unit = blockIdx.x / (4 * BHv);
-    const int pair = (blockIdx.x / BHv) & 3;
-    const int bh = blockIdx.x % BHv;
+    // Workgroups go round robin over the 8 XCDs.  A head's column parts share an XCD, whose L2 then
+    // fetches the head's operands once: the heads are padded to a multiple of 8 and the padding's
+    // workgroups end here.  (Not in a maps launch, whose units fill the device: there a head's
+    // share of one XCD's CUs would be too many.)
+    const int BHp = job.phase == kJobPlain ? (BHv + 7) & ~7 : BHv;
+    const int unit = blockIdx.x / (kWgs * BHp);
+    const int part = (blockIdx.x / BHp) % kWgs;
+    const int bh = blockIdx.x % BHp;
+    if (bh >= BHv) return;
+    const int wg = part * BHv + bh;  // its abort word (the launches that use one have one unit)
+    if (kFlags && mode == kCarryRetry &&
+        __builtin_amdgcn_readfirstlane(__hip_atomic_load(aborts + wg, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT)) == 0u)
+        return;  // this workgroup finished in the launch beside the prep
     const int b = bh / Hv, h = bh % Hv, hq = h % Hq;
-    const bool chain = wave < 2, outw = wave == 2 || wave == 3, dmaw = wave >= 4;
-    const int sl = wave & 1;  // chain wave: its strip; output wave: w = wave - 2
 
     // This workgroup's chunks [c0, c0 + nch), where its state starts (src: loaded; else zero,
     // or the identity for a transition map), where it ends (dst), where its outputs go (out,
-    // or a map's fp32 rows in the workspace), and the U scale (0 for a transition map).
+    // or a map's fp32 rows in the workspace), and the V scale (0 for a transition map).
     int seg = 0, c0 = 0, nch = nch_all;
     bool ident = false;
     float us = 1.f;
@@ -1125,145 +638,442 @@ gdn_chunk_carry(const TIO* __restrict__ q, const TIO* __restrict__ k,
         nch = seg == job.nseg - 1 ? nch_all - c0 : job.seg_len;
     }
     const int Tloc = T - c0 * kC;  // tokens from this workgroup's first chunk to the end of the sequence
-    const unsigned char* wsh = ws + ((size_t)bh * nch_all + c0) * ws_chunk<kF32>();
 
-    // Pipeline, iteration it.  Chain waves: process chunk it from cs[it&1].  Output waves:
-    // store the O tile of chunk it-2 staged in LDS, then compute the output of chunk it-1
-    // from os[(it-1)&1] and XS[(it-1)&1].  DMA waves: copy the chain operands of chunk it+1
-    // into cs[(it+1)&1] and the output operands of chunk it into os[it&1], then wait for
-    // the copies.  Then the workgroup meets at a barrier.
-    float4_t S[8];
-    // state layout [b*Hv + h][column][dk]: this lane's column, dk rows 16m + 4g + 0..3
-    const int col = (pair * kStrips + sl) * 16 + c;
-    const size_t soff = ((size_t)bh * kD + col) * kD, soff_seg = (size_t)col * kD;
-    const float* Sg = src == state ? state + soff : src + soff_seg;
+    // This lane's columns: with two tiles the columns interleave (tile ct, index i is column
+    // 8 (i / 4) + 4 ct + i % 4), so that the transposed output gives a lane 8 consecutive ones.
+    const int col0 = part * 16 * NC;
+    auto col = [&](int ct, int i) { return col0 + (NC == 1 ? i : 8 * (i >> 2) + 4 * ct + (i & 3)); };
+    const int nks = w < 2 ? 1 : 2;  // T' and Aqk key steps on or below the diagonal, from slot ts
+    const int ts = w < 2 ? w : 2 * w - 2;
+
     if (chain) {
+        // state layout [b*Hv + h][column][dk]: rows dk 32 w + 16 m + 4 g + 0..3
+        float4_t S[NC][2];
 #pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            if (src) {
-                const float4 v4 = *reinterpret_cast<const float4*>(Sg + 16 * m + 4 * g);
-                S[m] = float4_t{v4.x, v4.y, v4.z, v4.w};
-            } else {
+        for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) S[m][r] = ident && 16 * m + 4 * g + r == col ? 1.f : 0.f;
-            }
-        }
-    }
-    if (!dmaw) dma_wait_barrier();  // matches the DMA waves' prologue barrier
-    // Each role runs its own loop (one barrier per iteration in each), so no role's loop
-    // state occupies registers in another role's code.  `it` runs 0..nch; the loop is
-    // unrolled by two so slot indices are constants.
-    if (chain) {
-        const ChainOffs off = chain_offs();
-        for (int it = 0; it <= nch; it += 2) {
-            if (it < nch)
-                chain_step<kF32>(S, sm.cs[0], &sm.XS[0][sl][0][0], sl, off, us,
-                                 reinterpret_cast<const half_t*>(&sm.os[0]));
-            lds_barrier();  // chain waves issue no vector memory operations in the loop
-            if (it + 1 > nch) break;
-            if (it + 1 < nch)
-                chain_step<kF32>(S, sm.cs[1], &sm.XS[1][sl][0][0], sl, off, us,
-                                 reinterpret_cast<const half_t*>(&sm.os[1]));
-            lds_barrier();
-        }
-    } else if (outw) {
-        const int w = wave - 2;
-        const size_t orow = (size_t)Hv * kD;
-        // rows from this workgroup's first chunk on
-        half_t* out16 = reinterpret_cast<half_t*>(out) + (size_t)c0 * kC * orow;
-        // fp32 output (fp32 I/O, or a map's rows in the workspace): row of token t0 + 32 w of
-        // chunk ch, column pair * 32
-        const bool f32out = kF32 || obuf != nullptr;  // uniform
-        const size_t o32_row = obuf ? (size_t)kD : orow;
-        float* o32 = obuf ? obuf + (size_t)(32 * w) * kD + pair * 32
-                          : reinterpret_cast<float*>(out) + ((size_t)b * T + c0 * kC + 32 * w) * orow +
-                                (size_t)h * kD + pair * 32;
-        // fp32 I/O: the operands come from memory into registers, Q one chunk ahead (ops[ch & 1]
-        // holds chunk ch's), Aqk and e^G at the step (two full operand sets do not fit beside
-        // the chain's registers); otherwise from the chunk's out slot
-        OutOps ops[2];
-        if (kF32) ops[0] = out_ops_mem(wsh, w);
-        auto step = [&](int slot, int ch) {
-            if (kF32) {
-                const OutOps nx = out_ops_mem(wsh + (size_t)min(ch + 1, nch - 1) * ws_chunk<kF32>(), w);
-                if (ch + 1 < nch) {
+            for (int m = 0; m < 2; ++m) {
+                const int d0 = 32 * w + 16 * m + 4 * g;
+                if (src) {
+                    const float4 x = *reinterpret_cast<const float4*>(
+                        (src == state ? state + (size_t)bh * kSegSlotFloats : src) + (size_t)col(ct, c) * kD + d0);
+                    S[ct][m] = float4_t{x.x, x.y, x.z, x.w};
+                } else {
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int kk = 0; kk < 4; ++kk) ops[slot ^ 1].aQ[j][kk] = nx.aQ[j][kk];
+                    for (int r = 0; r < 4; ++r) S[ct][m][r] = ident && d0 + r == col(ct, c) ? 1.f : 0.f;
                 }
-                const OutOps cu = out_ops_mem(wsh + (size_t)ch * ws_chunk<kF32>(), w);
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-#pragma unroll
-                    for (int ks = 0; ks < 2; ++ks) ops[slot].aA[j][ks] = cu.aA[j][ks];
-                    ops[slot].eg[j] = cu.eg[j];
-                }
-            } else {
-                ops[slot] = out_ops_lds(sm.os[slot], w);
             }
-            if (f32out)
-                out_step<float>(ops[slot], sm.XS[slot], sm.OS[w], w, scale, o32 + (size_t)ch * kC * o32_row,
-                                o32_row, Tloc - ch * kC - 32 * w);
-            else
-                out_step<TIO>(ops[slot], sm.XS[slot], sm.OS[w], w, scale, o32, o32_row, 0);
+        // where this lane's 4 consecutive rows of a D tile go in the operand of the next product:
+        // row 16 m' + 4 g + r of a 32-row k-step is slot (g' = 2 m' + g / 2, 4 (g % 2) + r)
+        auto put = [&](uint4* op, int m, const uint2& x) {
+            reinterpret_cast<uint2*>(op)[2 * ((2 * m + (g >> 1)) * 16 + c) + (g & 1)] = x;
         };
-        for (int it = 0; it <= nch; it += 2) {
-            if (!f32out && it >= 2) out_flush(sm.OS[w], out16, b, T, Hv, h, (it - 2) * kC, pair, w, Tloc);
-            if (it >= 1) step(1, it - 1);
-            lds_barrier();  // the O stores need not complete before the barrier
-            if (it + 1 > nch) break;
-            if (!f32out && it >= 1) out_flush(sm.OS[w], out16, b, T, Hv, h, (it - 1) * kC, pair, w, Tloc);
-            step(0, it);
-            lds_barrier();
-        }
-    } else {
-        // the inputs' K / Q rows, or with fp32 I/O the prep's fp16 copies in the workspace
-        const unsigned rowbytes = kF32 ? (unsigned)kD * 2 : (unsigned)Hq * kD * 2;
-        const size_t chunk_bytes = kF32 ? (size_t)kWsChunkF32 : (size_t)kC * rowbytes;
-        const unsigned char* kh = kF32 ? wsh + kWsK
-                                       : reinterpret_cast<const unsigned char*>(k + ((size_t)b * T * Hq + hq) * kD) +
-                                             (size_t)c0 * chunk_bytes;
-        const unsigned char* qh = kF32 ? wsh + kWsQ
-                                       : reinterpret_cast<const unsigned char*>(q + ((size_t)b * T * Hq + hq) * kD) +
-                                             (size_t)c0 * chunk_bytes;
-        const unsigned slot_lds[4] = {(unsigned)(uintptr_t)(lds_void_t)(void*)&sm.cs[0],
-                                      (unsigned)(uintptr_t)(lds_void_t)(void*)&sm.cs[1],
-                                      (unsigned)(uintptr_t)(lds_void_t)(void*)&sm.os[0],
-                                      (unsigned)(uintptr_t)(lds_void_t)(void*)&sm.os[1]};
-        const unsigned* fl = flags ? flags + (size_t)bh * nch_all + c0 : nullptr;
-        int* err = &sm.err[wave - 4];
-        switch (wave) {
-            case 4: dma_role<0, kF32>(slot_lds, kh, qh, wsh, fl, wait_ticks, err, rowbytes, chunk_bytes, pair, Tloc, nch); break;
-            case 5: dma_role<1, kF32>(slot_lds, kh, qh, wsh, fl, wait_ticks, err, rowbytes, chunk_bytes, pair, Tloc, nch); break;
-            case 6: dma_role<2, kF32>(slot_lds, kh, qh, wsh, fl, wait_ticks, err, rowbytes, chunk_bytes, pair, Tloc, nch); break;
-            default: dma_role<3, kF32>(slot_lds, kh, qh, wsh, fl, wait_ticks, err, rowbytes, chunk_bytes, pair, Tloc, nch); break;
-        }
-    }
-    if (chain) {
-        // a timed-out wait means some chunk operands were read before they were published:
-        // beside the prep, leave the state for the second launch; otherwise poison it
-        const bool lost = (sm.err[0] | sm.err[1] | sm.err[2] | sm.err[3]) != 0;
-        // the abort word (cleared at the start of the call) sends this workgroup into the
-        // second launch
-        if (mode == kCarryBeside && tid == 0 && lost)
-            __hip_atomic_store(aborts + blockIdx.x, 1u, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        // in order after the prep the abort words were not cleared: the first unit's
-        // workgroups zero theirs (a workgroup that runs in order never gives up)
-        if (mode == kCarryInOrder && tid == 0 && blockIdx.x < 4 * BHv)
-            __hip_atomic_store(aborts + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (dst && !(lost && mode == kCarryBeside)) {
-            const float nan = __builtin_nanf("");
-            float* Dg = dst == state ? state + soff : dst + soff_seg;
+        auto put_state = [&]() {
 #pragma unroll
-            for (int m = 0; m < 8; ++m)
-                *reinterpret_cast<float4*>(Dg + 16 * m + 4 * g) =
-                    lost ? make_float4(nan, nan, nan, nan) : make_float4(S[m][0], S[m][1], S[m][2], S[m][3]);
+            for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    uint2 hi, lo;
+                    split4(S[ct][m], hi, lo);
+                    put(sm.S[0][ct][w], m, hi);
+                    if (kF32) put(sm.S[kF32 ? 1 : 0][ct][w], m, lo);
+                }
+        };
+        // step 1's operands that do not depend on the state, read ahead of the barrier before it
+        half8_t kA[4], kAl[4];
+        float v[NC][4], ek[4];
+        half4_t v4[NC];
+        auto ahead = [&](const CarrySlot<TIO, NC>& cs) __attribute__((always_inline)) {
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                kA[kk] = *reinterpret_cast<const half8_t*>(cs.K + tile_off(16 * w + c, 4 * kk + g));
+                if (kF32) kAl[kk] = *reinterpret_cast<const half8_t*>(cs.K + kC * kD + tile_off(16 * w + c, 4 * kk + g));
+            }
+            // V of tokens 16 w + 4 g + r at this lane's columns (fp16: read transposed, the lane
+            // supplying 4 columns of one token)
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct)
+                if constexpr (kF32) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[ct][r] = cs.V[(16 * w + 4 * g + r) * 16 * NC + col(ct, c) - col0];
+                } else {
+                    v4[ct] = lds_read_tr16(cs.V + (16 * w + 4 * g + (c >> 2)) * 16 * NC + col(ct, 4 * (c & 3)) - col0);
+                }
+            const float4 e = *reinterpret_cast<const float4*>(cs.G + kC + 16 * w + 4 * g);
+            ek[0] = e.x; ek[1] = e.y; ek[2] = e.z; ek[3] = e.w;
+        };
+        auto step = [&](const CarrySlot<TIO, NC>& cs, const CarrySlot<TIO, NC>& nx, int ch) __attribute__((always_inline)) {
+            // ---- 1. X = K S; R = V - e^G X ----
+            half8_t Sh[NC][4], Sl[NC][4];
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct) {
+                    Sh[ct][kk] = __builtin_bit_cast(half8_t, sm.S[0][ct][kk][lane]);
+                    if (kF32) Sl[ct][kk] = __builtin_bit_cast(half8_t, sm.S[kF32 ? 1 : 0][ct][kk][lane]);
+                }
+            // T' operands of step 2: their LDS time runs under step 1
+            half8_t th[2], tl[2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                th[ks] = __builtin_bit_cast(half8_t, cs.T[(ts + min(ks, nks - 1)) * 64 + lane]);
+                tl[ks] = __builtin_bit_cast(half8_t, cs.T[(kTSlots + ts + min(ks, nks - 1)) * 64 + lane]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct) {
+                float4_t x[2] = {};
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    x[kk & 1] = mfma16(kA[kk], Sh[ct][kk], x[kk & 1]);
+                    if (kF32) {
+                        x[kk & 1] = mfma16(kA[kk], Sl[ct][kk], x[kk & 1]);
+                        x[kk & 1] = mfma16(kAl[kk], Sh[ct][kk], x[kk & 1]);
+                    }
+                }
+                float4_t r4;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) r4[r] = fmaf(-ek[r], x[0][r] + x[1][r], us * (kF32 ? v[ct][r] : (float)v4[ct][r]));
+                uint2 hi, lo;
+                split4(r4, hi, lo);
+                put(sm.R[0][ct][w >> 1], w & 1, hi);
+                put(sm.R[1][ct][w >> 1], w & 1, lo);
+            }
+            lds_barrier();
+            // ---- 2. Vnew = T' R ----
+            half8_t Rh[NC][2], Rl[NC][2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct) {
+                    Rh[ct][ks] = __builtin_bit_cast(half8_t, sm.R[0][ct][ks][lane]);
+                    Rl[ct][ks] = __builtin_bit_cast(half8_t, sm.R[1][ct][ks][lane]);
+                }
+            // K^T operands and factors of step 3 (and e^{G_63 - G}): under step 2
+            half8_t aK[2][2], aKl[2][2];
+            const float4 d4 = *reinterpret_cast<const float4*>(cs.G + 2 * kC + 16 * w + 4 * g);
+            const float ec = ch < nch ? cs.G[3 * kC] : 1.f;
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    aK[m][ks] = cat8(tile_read_tr(cs.K, 32 * ks + 8 * g, 32 * w + 16 * m),
+                                     tile_read_tr(cs.K, 32 * ks + 8 * g + 4, 32 * w + 16 * m));
+                    if (kF32)
+                        aKl[m][ks] = cat8(tile_read_tr(cs.K + kC * kD, 32 * ks + 8 * g, 32 * w + 16 * m),
+                                          tile_read_tr(cs.K + kC * kD, 32 * ks + 8 * g + 4, 32 * w + 16 * m));
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            const float dg[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct) {
+                float4_t vn[3] = {};
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    if (ks >= nks) break;  // uniform
+                    vn[0] = mfma16(th[ks], Rh[ct][ks], vn[0]);
+                    vn[1] = mfma16(tl[ks], Rh[ct][ks], vn[1]);
+                    vn[2] = mfma16(th[ks], Rl[ct][ks], vn[2]);
+                }
+                float4_t vs;
+                half4_t vh;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float x = vn[0][r] + (vn[1][r] + vn[2][r]);
+                    vs[r] = x * dg[r];
+                    vh[r] = (half_t)x;
+                }
+                uint2 hi, lo;
+                split4(vs, hi, lo);
+                put(sm.V[0][ct][w >> 1], w & 1, hi);
+                put(sm.V[1][ct][w >> 1], w & 1, lo);
+                put(sm.V[2][ct][w >> 1], w & 1, __builtin_bit_cast(uint2, vh));
+            }
+            lds_barrier();
+            // ---- 3. S = e^{G_63} S + K^T Vs ----
+            half8_t Vh[NC][2], Vl[NC][2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct) {
+                    Vh[ct][ks] = __builtin_bit_cast(half8_t, sm.V[0][ct][ks][lane]);
+                    Vl[ct][ks] = __builtin_bit_cast(half8_t, sm.V[1][ct][ks][lane]);
+                }
+            ahead(nx);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) S[ct][m] *= ec;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) S[ct][m] = mfma16(aK[m][ks], Vh[ct][ks], S[ct][m]);
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) {
+                        S[ct][m] = mfma16(aK[m][ks], Vl[ct][ks], S[ct][m]);
+                        if (kF32) S[ct][m] = mfma16(aKl[m][ks], Vh[ct][ks], S[ct][m]);
+                    }
+            put_state();
+            lds_barrier();
+        };
+        put_state();
+        lds_barrier();  // S written; the helpers' copy of chunk 0 is in its slot
+        ahead(sm.c[0]);
+        // an odd count runs a chunk past the last one, whose operands read as zero and leave the
+        // state as it is
+        for (int ch = 0; ch < nch; ch += 2) {
+            step(sm.c[0], sm.c[1], ch);
+            step(sm.c[1], sm.c[0], ch + 1);
         }
-    } else if (outw && !kF32 && !obuf) {
-        out_flush(sm.OS[wave - 2], reinterpret_cast<half_t*>(out) + (size_t)c0 * kC * Hv * kD, b, T, Hv, h,
-                  (nch - 1) * kC, pair, wave - 2, Tloc);
+        bool lost = false;
+        if constexpr (kFlags) {
+            // a timed-out wait means some chunk operands were read before they were published:
+            // beside the prep, leave the state for the second launch (sent there by the abort word,
+            // cleared at the start of the call); otherwise poison it
+            lds_barrier();  // the helpers' err words
+            lost = (sm.err[0] | sm.err[1] | sm.err[2] | sm.err[3]) != 0;
+            if (mode == kCarryBeside && tid == 0 && lost)
+                __hip_atomic_store(aborts + wg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (tid == 0 && unit == 0 && part < kAbortWgs) {
+            // in order after the prep the abort words were not cleared: the first unit's workgroups
+            // zero theirs (a workgroup that runs in order never gives up)
+            __hip_atomic_store(aborts + wg, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (lost && mode == kCarryBeside) return;
+        const float nan = __builtin_nanf("");
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                *reinterpret_cast<float4*>((dst == state ? state + (size_t)bh * kSegSlotFloats : dst) +
+                                           (size_t)col(ct, c) * kD + 32 * w + 16 * m + 4 * g) =
+                    lost ? make_float4(nan, nan, nan, nan)
+                         : make_float4(S[ct][m][0], S[ct][m][1], S[ct][m][2], S[ct][m][3]);
+        return;
+    }
+
+    // ---- helper waves ----
+    // A buffer descriptor per tensor and chunk ends with the sequence's last token (none past the
+    // last chunk), so rows past the end read as zero and their stores are dropped.  Per-lane
+    // offsets are fixed.
+    constexpr unsigned kE = sizeof(TIO);
+    const unsigned vrow = (unsigned)Hv * kD * kE;  // bytes between tokens
+    const TIO* vh = v + (((size_t)b * T + (size_t)c0 * kC) * Hv + h) * kD;
+    const unsigned char* wsh = ws + ((size_t)bh * nch_all + c0) * ws_chunk<kF32>();
+    const unsigned char* wsq = ws + (((size_t)b * Hv + hq) * nch_all + c0) * ws_chunk<kF32>();  // the QK head's rows
+    // V: 4 lanes a token, 4 NC columns a lane
+    const unsigned voff = (unsigned)(16 * w + (lane >> 2)) * vrow + (unsigned)(col0 + 4 * NC * (lane & 3)) * kE;
+    const unsigned lane16 = (unsigned)lane * 16;
+    auto span = [&](int ch, unsigned row, unsigned last) {  // bytes of a chunk's rows
+        return ch < nch ? (unsigned)(min(kC, Tloc - ch * kC) - 1) * row + last : 0u;
+    };
+    auto rsrc_ws = [&](const unsigned char* p, int ch) {
+        return rsrc_of(p + (size_t)ch * ws_chunk<kF32>(), ch < nch ? (kF32 ? kWsUsedF32 : kWsUsed) : 0);
+    };
+    struct In {                 // what goes to the chain waves
+        uint4 k[4], kl[kF32 ? 4 : 1], t[3];
+        uint4 v[NC * (kF32 ? 2 : 1)];  // 8 bytes of it with fp16 I/O and NC = 1
+        float gf;
+    };
+    struct Own {                // what stays: operands of this wave's tokens
+        uint4 q[4], a[2];
+    };
+    auto load_t = [&](In& x, int ch) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t wr = rsrc_ws(wsh, ch);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) x.t[j] = bload4w<kFlags>(wr, kWsT + (unsigned)(3 * w + j) * 1024 + lane16);
+    };
+    auto load_kv = [&](In& x, int ch) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t qr = rsrc_ws(wsq, ch);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x.k[j] = bload4w<kFlags>(qr, kWsK + (unsigned)(4 * w + j) * 1024 + lane16);
+            if (kF32) x.kl[kF32 ? j : 0] = bload4w<kFlags>(qr, kWsKlo + (unsigned)(4 * w + j) * 1024 + lane16);
+        }
+        x.gf = bload1w<kFlags>(rsrc_ws(wsh, ch), kWsG + 4 * (kC * w + lane));
+        const __amdgpu_buffer_rsrc_t vr = rsrc_of(vh + (size_t)ch * kC * Hv * kD, span(ch, vrow, kD * kE));
+        if constexpr (NC * kE == 2) {
+            const u32x2_t y = __builtin_amdgcn_raw_buffer_load_b64(vr, voff, 0, 0);
+            x.v[0] = make_uint4(y[0], y[1], 0, 0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < (int)(NC * kE) / 4; ++i) x.v[i] = bload4(vr, voff + 16 * i);
+        }
+    };
+    auto load_q = [&](Own& x, int ch) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t qr = rsrc_ws(wsq, ch);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) x.q[kk] = bload4w<kFlags>(qr, kWsQ + (unsigned)(4 * w + kk) * 1024 + lane16);
+    };
+    auto load_a = [&](Own& x, int ch) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t wr = rsrc_ws(wsh, ch);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) x.a[ks] = bload4w<kFlags>(wr, kWsAqk + (unsigned)(ts + min(ks, nks - 1)) * 1024 + lane16);
+    };
+    // (the empty asm at the end of each keeps the reloads that follow behind these uses)
+    auto put_t = [&](CarrySlot<TIO, NC>& cs, const In& x) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) cs.T[(3 * w + j) * 64 + lane] = x.t[j];
+        asm volatile("" ::: "memory");
+    };
+    auto put_kv = [&](CarrySlot<TIO, NC>& cs, const In& x) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int off = tile_off(16 * w + 4 * j + (lane >> 4), lane & 15);
+            *reinterpret_cast<uint4*>(cs.K + off) = x.k[j];
+            if (kF32) *reinterpret_cast<uint4*>(cs.K + kC * kD + off) = x.kl[kF32 ? j : 0];
+        }
+        TIO* vp = cs.V + (16 * w + (lane >> 2)) * 16 * NC + 4 * NC * (lane & 3);
+        if constexpr (NC * kE == 2) {
+            *reinterpret_cast<uint2*>(vp) = make_uint2(x.v[0].x, x.v[0].y);
+        } else {
+#pragma unroll
+            for (int i = 0; i < (int)(NC * kE) / 4; ++i) reinterpret_cast<uint4*>(vp)[i] = x.v[i];
+        }
+        cs.G[kC * w + lane] = x.gf;
+        asm volatile("" ::: "memory");
+    };
+
+    // Ready flags (kFlags): a wave waits for a chunk's flag before it loads the chunk's workspace.
+    // After one timed-out wait, no more waits (the workgroup's results are then discarded).
+    const unsigned* fl = kFlags ? flags + (size_t)bh * nch_all + c0 : nullptr;
+    const unsigned* flq = kFlags ? flags + ((size_t)b * Hv + hq) * nch_all + c0 : nullptr;
+    bool gave_up = false;
+    auto ready = [&](int n) {
+        if constexpr (kFlags) {
+            auto look = [&]() {
+                const unsigned f = __hip_atomic_load(fl + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const unsigned fq = __hip_atomic_load(flq + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return __builtin_amdgcn_readfirstlane(f & fq);
+            };
+            // real-time counter (100 MHz), low 32 bits; readfirstlane keeps the wait loop uniform
+            auto now = []() { return __builtin_amdgcn_readfirstlane((unsigned)__builtin_amdgcn_s_memrealtime()); };
+            if (n < nch && !gave_up && look() == 0u) {
+                const unsigned t0 = now();
+                while (true) {
+                    if (now() - t0 >= wait_ticks) {
+                        gave_up = true;
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(8);
+                    if (look() != 0u) break;
+                }
+            }
+            asm volatile("" ::: "memory");  // no load of the chunk's workspace above the wait
+        }
+    };
+
+    // Output rows: fp32 (fp32 I/O, or a map's rows in the workspace) or the caller's type.
+    const unsigned orow = obuf ? (unsigned)kD * 4 : vrow;
+    unsigned char* ob = obuf ? reinterpret_cast<unsigned char*>(obuf)
+                             : reinterpret_cast<unsigned char*>(out + (((size_t)b * T + (size_t)c0 * kC) * Hv + h) * kD);
+    const bool o32 = kF32 || obuf != nullptr;  // uniform
+    const unsigned ooff = (unsigned)(16 * w + c) * orow + (unsigned)(col0 + 4 * NC * g) * (o32 ? 4 : 2);
+
+    // in: the next chunk's operands; o: this chunk's
+    auto step = [&](In& in, Own& o, CarrySlot<TIO, NC>& cs, CarrySlot<TIO, NC>& nx, int ch) __attribute__((always_inline)) {
+        // ---- 1. the next chunk's K, V and factors to the chain waves ----
+        put_kv(nx, in);
+        ready(ch + 3);
+        load_kv(in, ch + 3);
+        lds_barrier();
+        // ---- 2. its T'; (Q S)^T: rows are columns of the state, so a lane ends with consecutive
+        // output columns of one token ----
+        half8_t Sh[NC][4];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct) Sh[ct][kk] = __builtin_bit_cast(half8_t, sm.S[0][ct][kk][lane]);
+        const float eq = cs.G[16 * w + c];
+        put_t(nx, in);
+        load_t(in, ch + 3);
+        float4_t qs[NC];
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) qs[ct] = float4_t{};
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct)
+                qs[ct] = mfma16(Sh[ct][kk], __builtin_bit_cast(half8_t, o.q[kk]), qs[ct]);
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) pin(qs[ct]);
+        load_q(o, ch + 2);
+        lds_barrier();
+        // ---- 3. O ----
+        half8_t Vn[NC][2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct) Vn[ct][ks] = __builtin_bit_cast(half8_t, sm.V[2][ct][ks][lane]);
+        float4_t ov[NC];
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) {
+            float4_t av = {};
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                if (ks >= nks) break;  // uniform
+                av = mfma16(Vn[ct][ks], __builtin_bit_cast(half8_t, o.a[ks]), av);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ov[ct][r] = scale * fmaf(eq, qs[ct][r], av[r]);
+            pin(ov[ct]);
+        }
+        const __amdgpu_buffer_rsrc_t orr =
+            rsrc_of(ob + (size_t)ch * kC * orow, span(ch, orow, (unsigned)kD * (o32 ? 4 : 2)));
+        if (o32) {
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, ov[ct]), orr, ooff + 16 * ct, 0, 0);
+        } else {
+            half4_t oh[NC];
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) oh[ct][r] = (half_t)ov[ct][r];
+            if constexpr (NC == 2)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, cat8(oh[0], oh[NC - 1])), orr, ooff, 0, 0);
+            else
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, oh[0]), orr, ooff, 0, 0);
+        }
+        load_a(o, ch + 2);
+        lds_barrier();
+    };
+
+    In in0, in1;
+    Own a0, a1;
+    auto load_in = [&](In& x, int ch) __attribute__((always_inline)) {
+        ready(ch);
+        load_kv(x, ch);
+        load_t(x, ch);
+    };
+    load_in(in0, 0);
+    load_q(a0, 0);
+    load_a(a0, 0);
+    load_in(in1, 1);
+    load_q(a1, 1);
+    load_a(a1, 1);
+    put_kv(sm.c[0], in0);
+    put_t(sm.c[0], in0);
+    load_in(in0, 2);
+    lds_barrier();
+    // chunks 0 .. 2's operands are waited for here: with loads in flight at its entry the loop's
+    // own waits would be as strict as the entry's order asks for; and there is no exit between
+    // the two steps, which would leave the loop's header a path with one step's loads only
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    for (int ch = 0; ch < nch; ch += 2) {
+        step(in1, a0, sm.c[0], sm.c[1], ch);
+        step(in0, a1, sm.c[1], sm.c[0], ch + 1);
+    }
+    if constexpr (kFlags) {
+        if (lane == 0) sm.err[w] = gave_up;
+        lds_barrier();
     }
 }
 
@@ -1494,7 +1304,7 @@ SegPlan seg_plan(int BHv, int nch, int req) {
 // flags and the abort words, rounded up to 256 B.
 size_t seg_offset(size_t BHv, size_t nch, bool f32) {
     const size_t end = BHv * nch * ((f32 ? kWsChunkF32 : kWsChunk) + sizeof(unsigned)) +
-                       BHv * (kD / (16 * kStrips)) * sizeof(unsigned);
+                       BHv * kAbortWgs * sizeof(unsigned);
     return (end + 255) & ~(size_t)255;
 }
 }  // namespace
@@ -1506,7 +1316,7 @@ namespace {
 size_t ws_bytes_for(size_t BHv, size_t nch, int T, bool f32, const SegPlan& plan) {
     if (plan.nseg == 1)
         return BHv * nch * ((f32 ? kWsChunkF32 : kWsChunk) + sizeof(unsigned)) +
-               BHv * (kD / (16 * kStrips)) * sizeof(unsigned);
+               BHv * kAbortWgs * sizeof(unsigned);
     const size_t Tr = (size_t)T - (size_t)plan.seg_len * kC;
     return seg_offset(BHv, nch, f32) + BHv * plan.nseg * kSegSlots * kSegSlotFloats * sizeof(float) +
            2 * BHv * Tr * kD * sizeof(float);
@@ -1559,9 +1369,10 @@ hipError_t launch_chunked(const void* q, const void* k, const void* v, const flo
                           hipStream_t stream, size_t ws_budget = SIZE_MAX, int nseg = 0) {
     const int nch = (T + kC - 1) / kC;
     const int BHv = B * Hv;
-    const int carry_wgs = BHv * (kD / (16 * kStrips));
+    const int carry_wgs = BHv * kAbortWgs;
     auto Q = static_cast<const TIO*>(q);
     auto K = static_cast<const TIO*>(k);
+    auto V = static_cast<const TIO*>(v);
     auto W = static_cast<unsigned char*>(ws);
     unsigned* flags = reinterpret_cast<unsigned*>(W + (size_t)BHv * nch * ws_chunk<std::is_same<TIO, float>::value>());
     unsigned* aborts = flags + (size_t)BHv * nch;
@@ -1574,15 +1385,24 @@ hipError_t launch_chunked(const void* q, const void* k, const void* v, const flo
     // In order (the prep, then the carry, on one stream) no ready flags are written or read.
     auto prep = [&](hipStream_t st, bool publish) {
         hipLaunchKernelGGL((gdn_chunk_prep<kFused, TIO>), dim3(BHv * nch), dim3(kThreads), 0, st, Q, K,
-                           static_cast<const TIO*>(v), g_log, beta, gates, W, publish ? flags : nullptr, T,
+                           g_log, beta, gates, W, publish ? flags : nullptr, T,
                            Hq, Hv, nch, BHv);
         return hipGetLastError();
     };
     auto carry = [&](int mode, unsigned ticks, int units = 1, CarryJob job = CarryJob{}) {
-        hipLaunchKernelGGL(gdn_chunk_carry<TIO>, dim3(units * carry_wgs), dim3(kCarryThreads), 0, stream, Q, K,
-                           W, mode == kCarryInOrder ? nullptr : flags, aborts, mode, ticks, state, static_cast<TIO*>(out), T, Hq, Hv, nch, BHv,
-                           scale, job);
-        return hipGetLastError();
+        auto launch = [&](auto kernel, int wgs) {
+            hipLaunchKernelGGL(kernel, dim3(units == 1 ? wgs * ((BHv + 7) & ~7) : units * wgs * BHv), dim3(kCarryThreads), 0, stream, V, W,
+                               mode == kCarryInOrder ? nullptr : flags, aborts, mode, ticks, state,
+                               static_cast<TIO*>(out), T, Hq, Hv, nch, BHv, scale, job);
+            return hipGetLastError();
+        };
+        if (mode != kCarryInOrder) return launch(gdn_chunk_carry<TIO, 2, true>, kAbortWgs);
+        // A workgroup takes a CU.  16 columns each while every workgroup then has a CU of its own,
+        // else 32: a chunk step of 32 columns is ~1.25 steps of 16, and a second round costs a
+        // whole one.  (us per carry, 16 / 32 columns: 32 heads, T = 4096 74 / 88; 48 heads, T = 1000
+        // 36 / 27; fp32 I/O, 48 heads, T = 512 30 / 22; maps of 4 heads, T = 4096 23 / 18.)
+        if (units * 2 * kAbortWgs * BHv <= kSplitCUs) return launch(gdn_chunk_carry<TIO, 1, false>, 2 * kAbortWgs);
+        return launch(gdn_chunk_carry<TIO, 2, false>, kAbortWgs);
     };
 
     // Sequence split: in order on the caller's stream (the maps need every chunk's operands)
@@ -1729,7 +1549,7 @@ hipError_t gdn_chunked_noalloc(const void* q, const void* k, const void* v, cons
 hipError_t gdn_chunked_redo_count(const void* ws, int B, int T, int Hv, bool f32, int* count,
                                   hipStream_t stream) {
     const size_t nch = (size_t)(T + kC - 1) / kC;
-    const size_t n = (size_t)B * Hv * (kD / (16 * kStrips));
+    const size_t n = (size_t)B * Hv * kAbortWgs;
     const unsigned char* aborts = static_cast<const unsigned char*>(ws) +
                                   (size_t)B * Hv * nch * ((f32 ? kWsChunkF32 : kWsChunk) + sizeof(unsigned));
     unsigned* host = static_cast<unsigned*>(std::malloc(n * sizeof(unsigned)));
