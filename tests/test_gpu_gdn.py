@@ -442,6 +442,23 @@ def test_chunked_column_tiles(dev, orc, hq, hv, T, io):
     _check(o, s, o_ref, s_ref, *(TOL["chunked"] if io == "f16" else (2e-3, 2e-5)), label=f"{io} Hq={hq} Hv={hv} T={T}")
 
 
+@pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("T", [5, 6, 7, 8, 9, 15, 16, 17, 24, 33])
+def test_recurrent_token_blocks(dev, orc, T, io):
+    """The token-serial kernel's two forms around their line (6 tokens) and at the remainders of
+    the staged form's blocks of 8: bit for bit T decode steps, whose lanes and sums both share."""
+    import torch
+    rng = np.random.default_rng(700 + T)
+    B, Hq, Hv = 2, 3, 5
+    q, k, v, g, beta, st = _inputs(rng, B, T, Hq, Hv, sstd=0.02)
+    q, k, v = _as(io, q, k, v)
+    o, s = _gpu(dev, "recurrent", q, k, v, g, beta, st)
+    tq, tk, tv, tg, tb, ts = _dev(dev, q, k, v, g, beta, st)
+    steps = [tsa.gdn_decode_step(*(x[:, t].contiguous() for x in (tq, tk, tv, tg, tb)), ts) for t in range(T)]
+    assert np.array_equal(torch.stack(steps, 1).float().cpu().numpy(), o) and np.array_equal(ts.cpu().numpy(), s)
+    _check(o, s, *orc.gdn_serial(q, k, v, g, beta, st), *TOL["recurrent"], label=f"recurrent {io} T={T}")
+
+
 def _ws_fill(ws, kind):
     import torch
     if kind == "ones":      # every flag and abort word reads 1 ("ready", "redo")

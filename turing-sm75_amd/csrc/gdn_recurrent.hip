@@ -14,7 +14,8 @@
 //   * the state is read and written with nontemporal loads/stores: it is touched once
 //     per launch, and keeping it out of the caches measured 4.6 -> 5.6 TB/s for the
 //     in-place read-modify-write stream of a 16 x 32 head decode step;
-//   * T > 1: a 256-thread workgroup owns 32 columns of one (b, h) for all T tokens;
+//   * T > 1: a 256-thread workgroup owns 32 columns of one (b, h) for all T tokens (from 6 tokens
+//     on with the tokens staged through LDS, gdn_serial_kernel);
 //     decode (T = 1): a one-wave workgroup owns 8 columns, so a decode step of 16 x 32
 //     heads is 8192 independent workgroups.
 // The reference's token-serial family (serial/smem/occ/occ2/occ4/occ4p/occ8,
@@ -109,6 +110,122 @@ gdn_recurrent_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
             s[it][3] = fmaf(g, s[it][3], kr[4 * it + 3] * d);
         }
         if (j == 0) out[(bt * Hv + h) * kD + col] = (TIO)(scale * fmaf(g, sq, d * kq));
+    }
+#pragma unroll
+    for (int it = 0; it < 4; ++it) __builtin_nontemporal_store(s[it], Sc + it * 8 + j);
+}
+
+// Token-serial form for longer T: the same columns, lanes and sums, with the tokens taken in blocks
+// of 8 whose k, q, v and gates the workgroup stages through LDS as fp32, each value loaded and
+// converted once per workgroup.  The loads of block n + 2 are in flight while block n is
+// computed.  k . q is the same for every column: each wave's 8 lane groups take one token of the
+// block each and hand the sums round by readlane.  What bounds it is one wave per SIMD's chain of
+// ~90 vector instructions and 8 broadcast LDS reads a token: 0.58 -> 0.27 us a token at 48 heads,
+// fp32 I/O (T = 512: 299 -> 139 us).  Unrolled without the end-of-sequence test per token (LDS
+// reads of the next token ahead, 130 registers) it measured 136 us there and 339 instead of 314
+// at 256 heads.
+constexpr int kStagedMinT = 6;
+constexpr int kTB = 8;  // tokens per block: 32 threads of 4 elements load one token's row
+template <typename TIO>
+__global__ void __launch_bounds__(kThreads)
+gdn_serial_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
+                  const TIO* __restrict__ v, const float* __restrict__ g_log,
+                  const float* __restrict__ beta, float* __restrict__ state,
+                  TIO* __restrict__ out, int T, int Hq, int Hv, float scale) {
+    struct Block {
+        float4_t k[kTB][kD / 4], q[kTB][kD / 4];
+        float v[kTB][kColsPerBlock], g[kTB], be[kTB];
+    };
+    __shared__ Block blk[2];
+    const int bh = blockIdx.x / kBlocksPerHead;
+    const int cb = blockIdx.x % kBlocksPerHead;
+    const int b = bh / Hv, h = bh % Hv, hq = h % Hq;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int cl = tid >> 3, col = cb * kColsPerBlock + cl;
+    const int j = tid & 7;
+
+    float4_t* Sc = reinterpret_cast<float4_t*>(state + ((size_t)bh * kD + col) * kD);
+    float4_t s[4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it) s[it] = __builtin_nontemporal_load(Sc + it * 8 + j);
+
+    // this thread's share of a block: 4 elements of a token's k and q, one of its v (tokens past
+    // the end: the last one's, unused)
+    const int lt = tid >> 5, le = tid & 31;
+    struct Share {
+        float4_t k, q;
+        float v, g, be;
+    };
+    auto load = [&](Share& x, int t0) {
+        const size_t bt = (size_t)b * T + min(t0 + lt, T - 1);
+        x.k = load4(k + (bt * Hq + hq) * kD + 4 * le);
+        x.q = load4(q + (bt * Hq + hq) * kD + 4 * le);
+        x.v = (float)v[(bt * Hv + h) * kD + cb * kColsPerBlock + le];
+        x.g = g_log[bt * Hv + h];
+        x.be = beta[bt * Hv + h];
+    };
+    auto put = [&](Block& bl, const Share& x) {
+        bl.k[lt][le] = x.k;
+        bl.q[lt][le] = x.q;
+        bl.v[lt][le] = x.v;
+        if (le == 0) {
+            bl.g[lt] = __expf(x.g);
+            bl.be[lt] = x.be;
+        }
+    };
+    auto compute = [&](const Block& bl, int t0) {
+        // lane group i: k . q of the block's token i
+        float kq8 = 0.f;
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            const float4_t kr = bl.k[lane >> 3][it * 8 + j], qr = bl.q[lane >> 3][it * 8 + j];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) kq8 = fmaf(kr[e], qr[e], kq8);
+        }
+        kq8 = sum8(kq8);
+        TIO* o = out + (((size_t)b * T + t0) * Hv + h) * kD + col;
+#pragma unroll
+        for (int i = 0; i < kTB; ++i) {
+            if (t0 + i >= T) break;
+            float4_t kr[4], qr[4];
+#pragma unroll
+            for (int it = 0; it < 4; ++it) kr[it] = bl.k[i][it * 8 + j];
+#pragma unroll
+            for (int it = 0; it < 4; ++it) qr[it] = bl.q[i][it * 8 + j];
+            const float vc = bl.v[i][cl], g = bl.g[i], be = bl.be[i];
+            const float kq = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, kq8), 8 * i));
+            float kv = 0.f, sq = 0.f;
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    kv = fmaf(s[it][e], kr[it][e], kv);
+                    sq = fmaf(s[it][e], qr[it][e], sq);
+                }
+            kv = sum8(kv);
+            sq = sum8(sq);
+            const float d = (vc - g * kv) * be;
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[it][e] = fmaf(g, s[it][e], kr[it][e] * d);
+            if (j == 0) o[(size_t)i * Hv * kD] = (TIO)(scale * fmaf(g, sq, d * kq));
+        }
+    };
+    Share x;
+    load(x, 0);
+    put(blk[0], x);
+    load(x, kTB);
+    lds_barrier();
+    for (int t0 = 0; t0 < T; t0 += 2 * kTB) {
+        put(blk[1], x);
+        load(x, t0 + 2 * kTB);
+        compute(blk[0], t0);
+        lds_barrier();
+        put(blk[0], x);
+        load(x, t0 + 3 * kTB);
+        compute(blk[1], t0 + kTB);
+        lds_barrier();
     }
 #pragma unroll
     for (int it = 0; it < 4; ++it) __builtin_nontemporal_store(s[it], Sc + it * 8 + j);
@@ -276,6 +393,14 @@ hipError_t launch_recurrent(const void* q, const void* k, const void* v, const f
         return hipGetLastError();
     }
     const unsigned blocks = (unsigned)(B * Hv * kBlocksPerHead);
+    // From 6 tokens on the staged form, below it the direct one (us per call, direct / staged: 48
+    // heads, fp32 I/O, T = 2 3.3 / 4.3, 4 4.3 / 4.7, 6 5.5 / 5.3, 8 6.6 / 5.7, 31 20.0 / 11.8; four
+    // sequences, fp16, T = 4 7.6 / 8.1, 6 9.3 / 8.9, 8 11.1 / 9.9, 31 33.3 / 21.8).
+    if (T >= kStagedMinT) {
+        hipLaunchKernelGGL(gdn_serial_kernel<TIO>, dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
+                           g_log, beta, state, O, T, Hq, Hv, scale);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(gdn_recurrent_kernel<TIO>, dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
                        g_log, beta, state, O, T, Hq, Hv, scale);
     return hipGetLastError();
