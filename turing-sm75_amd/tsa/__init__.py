@@ -18,6 +18,7 @@ import ctypes
 import math
 import os
 import re
+import struct
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 PKG_ROOT = os.path.dirname(_HERE)
@@ -122,32 +123,47 @@ def _check(code: int) -> None:
         raise TsaError(code, strerror(code))
 
 
+# What every call does on the host is longer than a small call's kernel (a decode step of one
+# sequence: 4 us on the GPU), so the checks and conversions below avoid what only costs time:
+# no Stream object for the current stream, pointers as plain ints (ctypes converts them by the
+# declared argument types), torch looked up once, a workspace sized only when one is made.
+_torch = None
+
+
+def _t():
+    global _torch
+    if _torch is None:
+        import torch
+        _torch = torch
+    return _torch
+
+
 def _stream(stream):
-    import torch
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        torch = _torch or _t()
+        if not torch.cuda.is_initialized():
+            return torch.cuda.current_stream().cuda_stream
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return stream.cuda_stream
 
 
 def _need(t, dtype, ndim, name):
-    import torch
-    if not isinstance(t, torch.Tensor):
+    if not isinstance(t, (_torch or _t()).Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
-    if t.dtype != dtype or t.dim() != ndim or not t.is_cuda or not t.is_contiguous():
+    if t.dtype is not dtype or t.dim() != ndim or not t.is_cuda or not t.is_contiguous():
         raise ValueError(f"{name}: expected a contiguous {ndim}-d {dtype} CUDA tensor, got "
                          f"{tuple(t.shape)} {t.dtype} on {t.device}")
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _out(out, like, name="out"):
     """The output tensor: a new one shaped like `like`, or the caller's, which must have
     exactly that shape (a smaller one would be written past its end)."""
-    import torch
     if out is None:
-        return torch.empty_like(like)
+        return (_torch or _t()).empty_like(like)
     _need(out, like.dtype, like.dim(), name)
     if out.shape != like.shape:
         raise ValueError(f"{name}: expected shape {tuple(like.shape)}, got {tuple(out.shape)}")
@@ -169,7 +185,7 @@ def _scratch(nbytes, device, stream):
 def attn_fwd(q, k, v, out=None, scale=None, causal=True, stream=None, naive=False, valu=False):
     """O = softmax(scale Q K^T [+ causal mask]) V on the MFMA kernel (or the naive one, or the
     VALU opponent with valu=True)."""
-    import torch
+    torch = _torch or _t()
     for name, t in (("q", q), ("k", k), ("v", v)):
         _need(t, torch.float16, 4, name)
     if k.shape != q.shape or v.shape != q.shape:
@@ -193,7 +209,7 @@ def attn_fwd(q, k, v, out=None, scale=None, causal=True, stream=None, naive=Fals
 def attn_gqa_fwd(q, k, v, gate=None, out=None, scale=None, causal=True, stream=None, naive=False):
     """Gated grouped-query attention: q, gate [B, Hq, S, D]; k, v [B, Hkv, S, D] with
     Hq % Hkv == 0; O = softmax(scale Q K^T [+ causal mask]) V, times sigmoid(gate) if given."""
-    import torch
+    torch = _torch or _t()
     for name, t in (("q", q), ("k", k), ("v", v)):
         _need(t, torch.float16, 4, name)
     B, Hq, S, D = q.shape
@@ -213,7 +229,7 @@ def attn_gqa_fwd(q, k, v, gate=None, out=None, scale=None, causal=True, stream=N
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     fn = load().tsa_attn_gqa_naive if naive else load().tsa_attn_gqa_fwd
-    gp = _ptr(gate) if gate is not None else ctypes.c_void_p(0)
+    gp = _ptr(gate) if gate is not None else None
     _check(fn(_ptr(q), _ptr(k), _ptr(v), gp, _ptr(out), B, Hq, Hkv, S, D, float(scale),
               int(bool(causal)), _stream(stream)))
     return out
@@ -225,7 +241,7 @@ def attn_gqa_fwd(q, k, v, gate=None, out=None, scale=None, causal=True, stream=N
 def _gdn_shapes(q, k, v, g_log, beta, state, batched_t: bool):
     """Shapes of a GDN call; q, k, v are all fp16 (the library's I/O type) or all fp32 (the
     *_f32 entry points, the reference's own I/O)."""
-    import torch
+    torch = _torch or _t()
     nd = 4 if batched_t else 3
     io = q.dtype if isinstance(q, torch.Tensor) and q.dtype in (torch.float16, torch.float32) else torch.float16
     for name, t in (("q", q), ("k", k), ("v", v)):
@@ -269,15 +285,14 @@ def gdn_chunked_fwd(q, k, v, g_log, beta, state, out=None, scale=None, chunk=64,
     chunks the library splits the sequence into segments run side by side (same results to
     fp32 rounding).  nseg (through tsa_gdn_chunked_plan_fwd) asks for an explicit plan: 0 =
     the library's, 1 = no split, n >= 2 = n segments."""
-    import torch
+    torch = _torch or _t()
     B, T, Hq, Hv, dk, dv = _gdn_shapes(q, k, v, g_log, beta, state, True)
     out = _out(out, v)
     if scale is None:
         scale = 1.0 / math.sqrt(dk)
     f32 = q.dtype == torch.float32
-    need = gdn_chunked_workspace_bytes(B, T, Hq, Hv, dk, dv, chunk, f32=f32, nseg=nseg)
     if ws is None:
-        ws = _scratch(need, q.device, stream)
+        ws = _scratch(gdn_chunked_workspace_bytes(B, T, Hq, Hv, dk, dv, chunk, f32=f32, nseg=nseg), q.device, stream)
     args = (_ptr(q), _ptr(k), _ptr(v), _ptr(g_log), _ptr(beta), _ptr(state), _ptr(out),
             B, T, Hq, Hv, dk, dv, chunk, float(scale))
     tail = (_ptr(ws), ws.numel() * ws.element_size(), _stream(stream))
@@ -303,7 +318,7 @@ def gdn_recurrent_fwd(q, k, v, g_log, beta, state, out=None, scale=None, stream=
                       naive=False):
     """Token-serial recurrence over T tokens (or the naive check kernel); state in place.
     fp32 q/k/v select the *_f32 entry points."""
-    import torch
+    torch = _torch or _t()
     B, T, Hq, Hv, dk, dv = _gdn_shapes(q, k, v, g_log, beta, state, True)
     out = _out(out, v)
     if scale is None:
@@ -318,7 +333,7 @@ def gdn_recurrent_fwd(q, k, v, g_log, beta, state, out=None, scale=None, stream=
 def gdn_decode_step(q, k, v, g_log, beta, state, out=None, scale=None, stream=None):
     """One token per sequence: q/k [B, Hq, dk], v [B, Hv, dv]; state in place (fp16 or fp32
     q/k/v/out)."""
-    import torch
+    torch = _torch or _t()
     B, _, Hq, Hv, dk, dv = _gdn_shapes(q, k, v, g_log, beta, state, False)
     out = _out(out, v)
     if scale is None:
@@ -338,7 +353,7 @@ def gdn_naive(q, k, v, g_log, beta, state, out=None, scale=None, stream=None):
 # ---- the layer's pre / post ops (q, k l2 norm; beta = sigmoid(b); g_log = softplus(a +
 # dt_bias) * A; gated RMSNorm of the output), fused or as passes of their own ----
 def _gates(a, b, dt_bias, A, lead, Hv):
-    import torch
+    torch = _torch or _t()
     for name, t in (("a", a), ("b", b)):
         _need(t, torch.float32, len(lead) + 1, name)
         if tuple(t.shape) != tuple(lead) + (Hv,):
@@ -353,16 +368,15 @@ def gdn_chunked_fused_fwd(q, k, v, a, b, dt_bias, A, state, out=None, scale=None
                           chunk=64, ws=None, stream=None):
     """Chunked prefill from raw q, k [B,T,Hq,dk] and raw gate projections a, b [B,T,Hv]
     (fp16 q / k / v / out)."""
-    import torch
+    torch = _torch or _t()
     _need(q, torch.float16, 4, "q")
     B, T, Hq, Hv, dk, dv = _gdn_shapes(q, k, v, a, b, state, True)
     _gates(a, b, dt_bias, A, (B, T), Hv)
     out = _out(out, v)
     if scale is None:
         scale = 1.0 / math.sqrt(dk)
-    need = gdn_chunked_workspace_bytes(B, T, Hq, Hv, dk, dv, chunk)
     if ws is None:
-        ws = _scratch(need, q.device, stream)
+        ws = _scratch(gdn_chunked_workspace_bytes(B, T, Hq, Hv, dk, dv, chunk), q.device, stream)
     _check(load().tsa_gdn_chunked_fused_fwd(
         _ptr(q), _ptr(k), _ptr(v), _ptr(a), _ptr(b), _ptr(dt_bias), _ptr(A), _ptr(state),
         _ptr(out), B, T, Hq, Hv, dk, dv, chunk, float(scale), float(eps), _ptr(ws),
@@ -374,7 +388,7 @@ def gdn_decode_fused_step(q, k, v, a, b, dt_bias, A, state, out=None, scale=None
                           stream=None):
     """One decode step from raw q, k [B,Hq,dk] and raw gate projections a, b [B,Hv] (fp16
     q / k / v / out)."""
-    import torch
+    torch = _torch or _t()
     _need(q, torch.float16, 3, "q")
     B, _, Hq, Hv, dk, dv = _gdn_shapes(q, k, v, a, b, state, False)
     _gates(a, b, dt_bias, A, (B,), Hv)
@@ -389,7 +403,7 @@ def gdn_decode_fused_step(q, k, v, a, b, dt_bias, A, state, out=None, scale=None
 
 def gdn_preprocess(q, k, a, b, dt_bias, A, eps=1e-6, stream=None):
     """The pre-ops as a pass: returns (q_n, k_n, g_log, beta) for raw q, k [B,T,Hq,dk]."""
-    import torch
+    torch = _torch or _t()
     _need(q, torch.float16, 4, "q")
     _need(k, torch.float16, 4, "k")
     if k.shape != q.shape:
@@ -407,7 +421,7 @@ def gdn_preprocess(q, k, a, b, dt_bias, A, eps=1e-6, stream=None):
 
 def gdn_gated_rmsnorm(x, z, w, out=None, eps=1e-6, stream=None):
     """y = x / sqrt(mean(x^2) + eps) * w * silu(z) over dv; x, z [B,T,Hv,dv] fp16, w [dv]."""
-    import torch
+    torch = _torch or _t()
     _need(x, torch.float16, 4, "x")
     _need(z, torch.float16, 4, "z")
     _need(w, torch.float32, 1, "w")
@@ -425,23 +439,31 @@ def gdn_gated_rmsnorm(x, z, w, out=None, eps=1e-6, stream=None):
 def ggml_view(t) -> TsaTensor:
     """The ggml view of a torch tensor of up to 4 dims: ne / nb are its shape / strides in
     reverse order (ne[0] = the innermost dimension), padded with 1s."""
-    import torch
-    if t.dtype not in (torch.float32, torch.float16):
+    torch = _torch or _t()
+    return TsaTensor.from_buffer(bytearray(_pack_view(t)))
+
+
+# a tsa_tensor as bytes: data, type, ne[4], nb[4]
+_VIEW = struct.Struct("@Pi4x4q4N")
+assert _VIEW.size == ctypes.sizeof(TsaTensor)
+
+
+def _pack_view(t) -> bytes:
+    torch = _torch or _t()
+    if t.dtype is torch.float32:
+        kind, es = TSA_TYPE_F32, 4
+    elif t.dtype is torch.float16:
+        kind, es = TSA_TYPE_F16, 2
+    else:
         raise ValueError(f"ggml views are fp32 or fp16, got {t.dtype}")
-    if t.dim() > 4 or not t.is_cuda:
+    nd = t.dim()
+    if nd > 4 or not t.is_cuda:
         raise ValueError("a ggml view is a CUDA tensor of at most 4 dims")
-    ne = list(reversed(t.shape)) + [1] * (4 - t.dim())
-    es = t.element_size()
-    nb = [st * es for st in reversed(t.stride())]
+    ne, nb = list(t.shape[::-1]), [st * es for st in t.stride()[::-1]]
     while len(nb) < 4:
-        nb.append(nb[-1] * ne[len(nb) - 1] if nb else es)
-    v = TsaTensor()
-    v.data = t.data_ptr()
-    v.type = TSA_TYPE_F16 if t.dtype == torch.float16 else TSA_TYPE_F32
-    for i in range(4):
-        v.ne[i] = int(ne[i])
-        v.nb[i] = int(nb[i])
-    return v
+        nb.append(nb[-1] * ne[-1] if nb else es)
+        ne.append(1)
+    return _VIEW.pack(t.data_ptr(), kind, *ne, *nb)
 
 
 def ggml_gdn_workspace_bytes(q, v) -> int:
@@ -453,15 +475,15 @@ def ggml_gated_delta_net(q, k, v, g_log, beta, state, out, state_out=None, scale
     """Torch tensors in the kernels' index order ([B, T, H, S] for q / k / v / out,
     [B, T, Hv] for g_log / beta, [B, Hv, S, S] for the states), any strides / fp32 or fp16:
     passed as ggml views.  state_out defaults to state (in place)."""
-    import torch
+    torch = _torch or _t()
     if state_out is None:
         state_out = state
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[-1])
-    views = [ggml_view(x) for x in (q, k, v, g_log, beta, state, out, state_out)]
-    need = int(load().tsa_ggml_gdn_workspace_bytes(ctypes.byref(views[0]), ctypes.byref(views[2])))
     if ws is None:
-        ws = _scratch(need, q.device, stream)
-    _check(load().tsa_ggml_gated_delta_net(*[ctypes.byref(x) for x in views], float(scale),
-                                           _ptr(ws), ws.numel() * ws.element_size(), _stream(stream)))
+        ws = _scratch(ggml_gdn_workspace_bytes(q, v), q.device, stream)
+    views = (TsaTensor * 8).from_buffer(bytearray(b"".join(
+        [_pack_view(x) for x in (q, k, v, g_log, beta, state, out, state_out)])))
+    _check(load().tsa_ggml_gated_delta_net(*views, float(scale), _ptr(ws), ws.numel() * ws.element_size(),
+                                           _stream(stream)))
     return out
