@@ -133,3 +133,48 @@ def test_against_oracle(dev, orc):
     es = float(np.abs(ts.cpu().numpy() - s_ref).max() / np.abs(s_ref).max())
     print(f"ggml adapter T={T} Hv={Hv}: out max-abs {eo:.2e}  state rel {es:.2e}")
     assert eo < 2e-3 and es < 3e-4
+
+
+@pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("form", ["fused", "head_major", "batch_inner", "broadcast", "offset", "odd_rows", "over_input"])
+@pytest.mark.parametrize("T", [1, 5, 20, 40, 1100])
+def test_rows_read_where_they_lie(dev, form, io, T):
+    """q, k and v in every form the kernels read without a gather -- column blocks of one
+    projection, heads outside tokens, sequences inside tokens, one head's rows for all heads
+    (stride 0) -- and in forms that still take one (rows off a 16-byte boundary, an odd token
+    stride, an output laid over the inputs' memory), from a state that is read in one buffer and
+    written to another: bit for bit the dense call, at T of every kernel (1100: the sequence
+    split)."""
+    import torch
+    B, Hk, Hv = 2, 2, 4
+    q, k, v, g, beta, st = _data(np.random.default_rng(T), B, T, Hk, Hv)
+    if form == "broadcast":
+        q, k, v = (np.repeat(x[:, :, :1], x.shape[2], 2) for x in (q, k, v))
+    f32 = io == "f32"
+    o_ref, s_ref = _direct(dev, q, k, v, g, beta, st, f32=f32)
+    dt = torch.float32 if f32 else torch.float16
+    tq, tk, tv = (_t(dev, x).to(dt) for x in (q, k, v))
+    W = (2 * Hk + Hv) * D
+    extra = {"offset": 8, "odd_rows": 3}.get(form, 0)
+    if form in ("fused", "offset", "odd_rows", "over_input"):
+        lead = 1 if form == "offset" else 0
+        proj = torch.zeros(B, T, W + extra, device=dev, dtype=dt)
+        x = proj[:, :, lead:lead + W]
+        x[:] = torch.cat([tq.flatten(2), tk.flatten(2), tv.flatten(2)], 2)
+        tq, tk, tv = (x[:, :, a:b].unflatten(2, (-1, D)) for a, b in
+                      ((0, Hk * D), (Hk * D, 2 * Hk * D), (2 * Hk * D, W)))
+    elif form == "head_major":
+        tq, tk, tv = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (tq, tk, tv))
+    elif form == "batch_inner":
+        tq, tk, tv = (x.transpose(0, 1).contiguous().transpose(0, 1) for x in (tq, tk, tv))
+    else:
+        tq, tk, tv = (x[:, :, :1].contiguous().expand(-1, -1, x.shape[2], -1) for x in (tq, tk, tv))
+    ts_in, ts_out = _t(dev, st), torch.full((B, Hv, D, D), -3.0, device=dev)
+    if form == "over_input":   # a dense output at the start of the projection's own memory
+        out = proj.flatten()[:B * T * Hv * D].view(B, T, Hv, D)
+    else:
+        out = torch.empty(B, T, Hv, D, device=dev, dtype=dt)
+    tsa.ggml_gated_delta_net(tq, tk, tv, _t(dev, g), _t(dev, beta), ts_in, out, ts_out)
+    torch.cuda.synchronize()
+    assert torch.equal(out.cpu(), o_ref) and torch.equal(ts_out.cpu(), s_ref)
+    assert torch.equal(ts_in.cpu(), torch.from_numpy(st))

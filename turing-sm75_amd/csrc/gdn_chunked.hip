@@ -247,7 +247,7 @@ template <bool kFused, typename TIO>
 __global__ void __launch_bounds__(kThreads, prep_wgs_per_cu<TIO>())
 gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k, const float* __restrict__ g_log,
                const float* __restrict__ beta, GdnRawGates gates, unsigned char* __restrict__ ws,
-               unsigned* __restrict__ flags, int T, int Hq, int Hv, int nch, int BHv) {
+               unsigned* __restrict__ flags, int T, int Hq, int Hv, int nch, int BHv, GdnStrides st) {
     __shared__ __align__(16) PrepLds sm;
     __shared__ __align__(16) half_t klo_lds[std::is_same<TIO, float>::value ? kC * kD : 8];  // low halves of the K rows
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hi = lane >> 5;
@@ -277,9 +277,9 @@ gdn_chunk_prep(const TIO* __restrict__ q, const TIO* __restrict__ k, const float
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
         const int id = it * kThreads + tid;
-        const size_t o = (((size_t)b * T + min(t0 + (id >> 4), lastt)) * Hq + hq) * kD + (id & 15) * 8;
-        load8hl(k + o, kreg[it], klo[it]);
-        qreg[it] = load8h(q + o);
+        const int t = min(t0 + (id >> 4), lastt);
+        load8hl(k + b * st.k.b + t * st.k.t + hq * st.k.h + (id & 15) * 8, kreg[it], klo[it]);
+        qreg[it] = load8h(q + b * st.q.b + t * st.q.t + hq * st.q.h + (id & 15) * 8);
     }
     const bool copies = h < Hq;  // this workgroup leaves its QK head's rows to the carry
 #pragma unroll
@@ -582,8 +582,9 @@ __device__ __forceinline__ void pin(float4_t& x) { asm volatile("" : "+v"(x)::"m
 template <typename TIO, int NC, bool kFlags>
 __global__ void __launch_bounds__(kCarryThreads, 2)
 gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws, const unsigned* __restrict__ flags,
-                unsigned* __restrict__ aborts, int mode, unsigned wait_ticks, float* __restrict__ state,
-                TIO* __restrict__ out, int T, int Hq, int Hv, int nch_all, int BHv, float scale, CarryJob job) {
+                unsigned* __restrict__ aborts, int mode, unsigned wait_ticks, const float* state_in, float* state,
+                TIO* __restrict__ out, int T, int Hq, int Hv, int nch_all, int BHv, float scale, CarryJob job,
+                RowStride vs) {
     constexpr bool kF32 = std::is_same<TIO, float>::value;
     constexpr int kWgs = kD / (16 * NC);  // workgroups per head
     __shared__ __align__(16) CarryLds<TIO, NC> sm;
@@ -614,7 +615,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
     int seg = 0, c0 = 0, nch = nch_all;
     bool ident = false;
     float us = 1.f;
-    const float* src = state;
+    const float* src = state_in;
     float* dst = state;
     float* obuf = nullptr;  // a map's fp32 output rows (from segment 1's first token), or out
     // this head's slots (no slots in the plain job)
@@ -656,7 +657,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
                 const int d0 = 32 * w + 16 * m + 4 * g;
                 if (src) {
                     const float4 x = *reinterpret_cast<const float4*>(
-                        (src == state ? state + (size_t)bh * kSegSlotFloats : src) + (size_t)col(ct, c) * kD + d0);
+                        (src == state_in ? state_in + (size_t)bh * kSegSlotFloats : src) + (size_t)col(ct, c) * kD + d0);
                     S[ct][m] = float4_t{x.x, x.y, x.z, x.w};
                 } else {
 #pragma unroll
@@ -864,8 +865,8 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
     // last chunk), so rows past the end read as zero and their stores are dropped.  Per-lane
     // offsets are fixed.
     constexpr unsigned kE = sizeof(TIO);
-    const unsigned vrow = (unsigned)Hv * kD * kE;  // bytes between tokens
-    const TIO* vh = v + (((size_t)b * T + (size_t)c0 * kC) * Hv + h) * kD;
+    const unsigned vrow = (unsigned)vs.t * kE;  // bytes between tokens of V
+    const TIO* vh = v + b * vs.b + (long long)c0 * kC * vs.t + h * vs.h;
     const unsigned char* wsh = ws + ((size_t)bh * nch_all + c0) * ws_chunk<kF32>();
     const unsigned char* wsq = ws + (((size_t)b * Hv + hq) * nch_all + c0) * ws_chunk<kF32>();  // the QK head's rows
     // V: 4 lanes a token, 4 NC columns a lane
@@ -898,7 +899,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
             if (kF32) x.kl[kF32 ? j : 0] = bload4w<kFlags>(qr, kWsKlo + (unsigned)(4 * w + j) * 1024 + lane16);
         }
         x.gf = bload1w<kFlags>(rsrc_ws(wsh, ch), kWsG + 4 * (kC * w + lane));
-        const __amdgpu_buffer_rsrc_t vr = rsrc_of(vh + (size_t)ch * kC * Hv * kD, span(ch, vrow, kD * kE));
+        const __amdgpu_buffer_rsrc_t vr = rsrc_of(vh + (long long)ch * kC * vs.t, span(ch, vrow, kD * kE));
         if constexpr (NC * kE == 2) {
             const u32x2_t y = __builtin_amdgcn_raw_buffer_load_b64(vr, voff, 0, 0);
             x.v[0] = make_uint4(y[0], y[1], 0, 0);
@@ -971,7 +972,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
     };
 
     // Output rows: fp32 (fp32 I/O, or a map's rows in the workspace) or the caller's type.
-    const unsigned orow = obuf ? (unsigned)kD * 4 : vrow;
+    const unsigned orow = obuf ? (unsigned)kD * 4 : (unsigned)Hv * kD * kE;
     unsigned char* ob = obuf ? reinterpret_cast<unsigned char*>(obuf)
                              : reinterpret_cast<unsigned char*>(out + (((size_t)b * T + (size_t)c0 * kC) * Hv + h) * kD);
     const bool o32 = kF32 || obuf != nullptr;  // uniform
@@ -1364,9 +1365,9 @@ bool overlap_requested() { return env_long("TSA_GDN_OVERLAP", 0, 1) != 0; }
 
 template <bool kFused, typename TIO>
 hipError_t launch_chunked(const void* q, const void* k, const void* v, const float* g_log,
-                          const float* beta, const GdnRawGates& gates, float* state, void* out,
-                          int B, int T, int Hq, int Hv, float scale, void* ws, bool may_overlap,
-                          hipStream_t stream, size_t ws_budget = SIZE_MAX, int nseg = 0) {
+                          const float* beta, const GdnRawGates& gates, const float* state_in, float* state,
+                          void* out, int B, int T, int Hq, int Hv, float scale, void* ws, bool may_overlap,
+                          hipStream_t stream, const GdnStrides& st, size_t ws_budget = SIZE_MAX, int nseg = 0) {
     const int nch = (T + kC - 1) / kC;
     const int BHv = B * Hv;
     const int carry_wgs = BHv * kAbortWgs;
@@ -1383,17 +1384,17 @@ hipError_t launch_chunked(const void* q, const void* k, const void* v, const flo
         return hipGetLastError();
     };
     // In order (the prep, then the carry, on one stream) no ready flags are written or read.
-    auto prep = [&](hipStream_t st, bool publish) {
-        hipLaunchKernelGGL((gdn_chunk_prep<kFused, TIO>), dim3(BHv * nch), dim3(kThreads), 0, st, Q, K,
+    auto prep = [&](hipStream_t on, bool publish) {
+        hipLaunchKernelGGL((gdn_chunk_prep<kFused, TIO>), dim3(BHv * nch), dim3(kThreads), 0, on, Q, K,
                            g_log, beta, gates, W, publish ? flags : nullptr, T,
-                           Hq, Hv, nch, BHv);
+                           Hq, Hv, nch, BHv, st);
         return hipGetLastError();
     };
     auto carry = [&](int mode, unsigned ticks, int units = 1, CarryJob job = CarryJob{}) {
         auto launch = [&](auto kernel, int wgs) {
             hipLaunchKernelGGL(kernel, dim3(units == 1 ? wgs * ((BHv + 7) & ~7) : units * wgs * BHv), dim3(kCarryThreads), 0, stream, V, W,
-                               mode == kCarryInOrder ? nullptr : flags, aborts, mode, ticks, state,
-                               static_cast<TIO*>(out), T, Hq, Hv, nch, BHv, scale, job);
+                               mode == kCarryInOrder ? nullptr : flags, aborts, mode, ticks, state_in,
+                               state, static_cast<TIO*>(out), T, Hq, Hv, nch, BHv, scale, job, st.v);
             return hipGetLastError();
         };
         if (mode != kCarryInOrder) return launch(gdn_chunk_carry<TIO, 2, true>, kAbortWgs);
@@ -1542,8 +1543,8 @@ hipError_t gdn_chunked_noalloc(const void* q, const void* k, const void* v, cons
     const hipError_t e = scratch_address(stream, &ws);
     if (e != hipSuccess) return e;
     // in order on the caller's stream: no side stream or event is ever created here
-    return launch_chunked<false, half_t>(q, k, v, g_log, beta, GdnRawGates{}, state, out, B, T, Hq, Hv,
-                                         scale, ws, false, stream, kScratchBytes);
+    return launch_chunked<false, half_t>(q, k, v, g_log, beta, GdnRawGates{}, state, state, out, B, T, Hq, Hv,
+                                         scale, ws, false, stream, gdn_dense(T, Hq, Hv), kScratchBytes);
 }
 
 hipError_t gdn_chunked_redo_count(const void* ws, int B, int T, int Hv, bool f32, int* count,
@@ -1568,18 +1569,30 @@ hipError_t gdn_chunked_redo_count(const void* ws, int B, int T, int Hv, bool f32
 hipError_t gdn_chunked(const void* q, const void* k, const void* v, const float* g_log,
                        const float* beta, float* state, void* out, int B, int T, int Hq, int Hv,
                        float scale, void* ws, bool f32, hipStream_t stream, int nseg) {
+    const GdnStrides st = gdn_dense(T, Hq, Hv);
     if (f32)
-        return launch_chunked<false, float>(q, k, v, g_log, beta, GdnRawGates{}, state, out, B, T, Hq,
-                                            Hv, scale, ws, true, stream, SIZE_MAX, nseg);
-    return launch_chunked<false, half_t>(q, k, v, g_log, beta, GdnRawGates{}, state, out, B, T, Hq, Hv,
-                                         scale, ws, true, stream, SIZE_MAX, nseg);
+        return launch_chunked<false, float>(q, k, v, g_log, beta, GdnRawGates{}, state, state, out, B, T, Hq,
+                                            Hv, scale, ws, true, stream, st, SIZE_MAX, nseg);
+    return launch_chunked<false, half_t>(q, k, v, g_log, beta, GdnRawGates{}, state, state, out, B, T, Hq,
+                                         Hv, scale, ws, true, stream, st, SIZE_MAX, nseg);
+}
+
+hipError_t gdn_chunked_strided(const void* q, const void* k, const void* v, const GdnStrides& st,
+                               const float* g_log, const float* beta, const float* state_in, float* state,
+                               void* out, int B, int T, int Hq, int Hv, float scale, void* ws, bool f32,
+                               hipStream_t stream) {
+    if (f32)
+        return launch_chunked<false, float>(q, k, v, g_log, beta, GdnRawGates{}, state_in, state, out, B, T, Hq,
+                                            Hv, scale, ws, true, stream, st);
+    return launch_chunked<false, half_t>(q, k, v, g_log, beta, GdnRawGates{}, state_in, state, out, B, T, Hq,
+                                         Hv, scale, ws, true, stream, st);
 }
 
 hipError_t gdn_chunked_fused(const void* q, const void* k, const void* v, const GdnRawGates& gates,
                              float* state, void* out, int B, int T, int Hq, int Hv, float scale,
                              void* ws, hipStream_t stream) {
-    return launch_chunked<true, half_t>(q, k, v, nullptr, nullptr, gates, state, out, B, T, Hq, Hv,
-                                        scale, ws, true, stream);
+    return launch_chunked<true, half_t>(q, k, v, nullptr, nullptr, gates, state, state, out, B, T, Hq, Hv,
+                                        scale, ws, true, stream, gdn_dense(T, Hq, Hv));
 }
 
 }  // namespace tsa

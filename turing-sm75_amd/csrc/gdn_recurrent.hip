@@ -61,8 +61,8 @@ template <typename TIO>
 __global__ void __launch_bounds__(kThreads)
 gdn_recurrent_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
                      const TIO* __restrict__ v, const float* __restrict__ g_log,
-                     const float* __restrict__ beta, float* __restrict__ state,
-                     TIO* __restrict__ out, int T, int Hq, int Hv, float scale) {
+                     const float* __restrict__ beta, const float* state_in, float* state,
+                     TIO* __restrict__ out, int T, int Hq, int Hv, float scale, GdnStrides st) {
     const int bh = blockIdx.x / kBlocksPerHead;
     const int cb = blockIdx.x % kBlocksPerHead;
     const int b = bh / Hv, h = bh % Hv, hq = h % Hq;
@@ -70,19 +70,20 @@ gdn_recurrent_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     const int col = cb * kColsPerBlock + (tid >> 3);
     const int j = tid & 7;
 
+    const float4_t* Si = reinterpret_cast<const float4_t*>(state_in + ((size_t)bh * kD + col) * kD);
     float4_t* Sc = reinterpret_cast<float4_t*>(state + ((size_t)bh * kD + col) * kD);
     float4_t s[4];
 #pragma unroll
-    for (int it = 0; it < 4; ++it) s[it] = __builtin_nontemporal_load(Sc + it * 8 + j);
+    for (int it = 0; it < 4; ++it) s[it] = __builtin_nontemporal_load(Si + it * 8 + j);
 
     for (int t = 0; t < T; ++t) {
         const size_t bt = (size_t)b * T + t;
         float kr[16], qr[16];
-        load_row16(k + (bt * Hq + hq) * kD, j, kr);
-        load_row16(q + (bt * Hq + hq) * kD, j, qr);
+        load_row16(k + b * st.k.b + t * st.k.t + hq * st.k.h, j, kr);
+        load_row16(q + b * st.q.b + t * st.q.t + hq * st.q.h, j, qr);
         const float gl = g_log[bt * Hv + h];
         const float be = beta[bt * Hv + h];
-        const float vc = (float)v[(bt * Hv + h) * kD + col];
+        const float vc = (float)v[b * st.v.b + t * st.v.t + h * st.v.h + col];
         float kv = 0.f, sq = 0.f, kq = 0.f;
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
@@ -130,8 +131,8 @@ template <typename TIO>
 __global__ void __launch_bounds__(kThreads)
 gdn_serial_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
                   const TIO* __restrict__ v, const float* __restrict__ g_log,
-                  const float* __restrict__ beta, float* __restrict__ state,
-                  TIO* __restrict__ out, int T, int Hq, int Hv, float scale) {
+                  const float* __restrict__ beta, const float* state_in, float* state,
+                  TIO* __restrict__ out, int T, int Hq, int Hv, float scale, GdnStrides st) {
     struct Block {
         float4_t k[kTB][kD / 4], q[kTB][kD / 4];
         float v[kTB][kColsPerBlock], g[kTB], be[kTB];
@@ -144,10 +145,11 @@ gdn_serial_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     const int cl = tid >> 3, col = cb * kColsPerBlock + cl;
     const int j = tid & 7;
 
+    const float4_t* Si = reinterpret_cast<const float4_t*>(state_in + ((size_t)bh * kD + col) * kD);
     float4_t* Sc = reinterpret_cast<float4_t*>(state + ((size_t)bh * kD + col) * kD);
     float4_t s[4];
 #pragma unroll
-    for (int it = 0; it < 4; ++it) s[it] = __builtin_nontemporal_load(Sc + it * 8 + j);
+    for (int it = 0; it < 4; ++it) s[it] = __builtin_nontemporal_load(Si + it * 8 + j);
 
     // this thread's share of a block: 4 elements of a token's k and q, one of its v (tokens past
     // the end: the last one's, unused)
@@ -157,10 +159,11 @@ gdn_serial_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
         float v, g, be;
     };
     auto load = [&](Share& x, int t0) {
-        const size_t bt = (size_t)b * T + min(t0 + lt, T - 1);
-        x.k = load4(k + (bt * Hq + hq) * kD + 4 * le);
-        x.q = load4(q + (bt * Hq + hq) * kD + 4 * le);
-        x.v = (float)v[(bt * Hv + h) * kD + cb * kColsPerBlock + le];
+        const int t = min(t0 + lt, T - 1);
+        const size_t bt = (size_t)b * T + t;
+        x.k = load4(k + b * st.k.b + t * st.k.t + hq * st.k.h + 4 * le);
+        x.q = load4(q + b * st.q.b + t * st.q.t + hq * st.q.h + 4 * le);
+        x.v = (float)v[b * st.v.b + t * st.v.t + h * st.v.h + cb * kColsPerBlock + le];
         x.g = g_log[bt * Hv + h];
         x.be = beta[bt * Hv + h];
     };
@@ -256,8 +259,8 @@ template <int kCols, int kLpc, bool kFused, typename TIO>
 __global__ void __launch_bounds__(kLpc * kCols)
 gdn_decode_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
                   const TIO* __restrict__ v, const float* __restrict__ g_log,
-                  const float* __restrict__ beta, GdnRawGates gates, float* __restrict__ state,
-                  TIO* __restrict__ out, int Hq, int Hv, float scale) {
+                  const float* __restrict__ beta, GdnRawGates gates, const float* state_in, float* state,
+                  TIO* __restrict__ out, int Hq, int Hv, float scale, GdnStrides st) {
     static_assert(kLpc * kCols >= 64, "wave 0 loads the q / k rows");
     constexpr int kWgPerHead = kD / kCols;
     constexpr int kR = 32 / kLpc;  // float4 chunks of the column per lane
@@ -270,11 +273,12 @@ gdn_decode_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
 
     typedef typename std::conditional<std::is_same<TIO, float>::value, float4_t, half4_t>::type row4_t;
     __shared__ row4_t kq_rows[2][kD / 4];
+    const float4_t* Si = reinterpret_cast<const float4_t*>(state_in + ((size_t)bh * kD + col) * kD);
     float4_t* Sc = reinterpret_cast<float4_t*>(state + ((size_t)bh * kD + col) * kD);
     float4_t s[kR];
 #pragma unroll
     for (int it = 0; it < kR; ++it)
-        s[it] = __builtin_nontemporal_load(Sc + it * kLpc + j);
+        s[it] = __builtin_nontemporal_load(Si + it * kLpc + j);
     // Wait for the state before issuing the q / k / v loads.  Measured over 16 x 32 heads with
     // 16 replicas cycled: 11.3 vs 12.2 us per step with the small loads issued under the
     // state loads (and 9.4 vs 10.4 us on a cache-resident state).
@@ -282,10 +286,10 @@ gdn_decode_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0); expcnt, lgkmcnt left at their maxima
     __builtin_amdgcn_sched_barrier(0);
     if (tid < 64) {  // wave 0 -- lanes 0-31: k row, 32-63: q row, 4 elements each
-        const TIO* row = (tid < 32 ? k : q) + (bt * Hq + hq) * kD;
+        const TIO* row = tid < 32 ? k + b * st.k.b + hq * st.k.h : q + b * st.q.b + hq * st.q.h;
         kq_rows[tid >> 5][tid & 31] = *reinterpret_cast<const row4_t*>(row + 4 * (tid & 31));
     }
-    const float vc = (float)v[vrow + col];
+    const float vc = (float)v[b * st.v.b + h * st.v.h + col];
     float g, be;
     if (kFused) {
         g = __expf(gdn_softplus(gates.a[bt * Hv + h] + gates.dt_bias[h]) * gates.A[h]);
@@ -378,9 +382,9 @@ gdn_naive_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
 }
 
 template <typename TIO>
-hipError_t launch_recurrent(const void* q, const void* k, const void* v, const float* g_log,
-                            const float* beta, float* state, void* out, int B, int T, int Hq,
-                            int Hv, float scale, hipStream_t stream) {
+hipError_t launch_recurrent(const void* q, const void* k, const void* v, const GdnStrides& st,
+                            const float* g_log, const float* beta, const float* state_in, float* state,
+                            void* out, int B, int T, int Hq, int Hv, float scale, hipStream_t stream) {
     auto Q = static_cast<const TIO*>(q);
     auto K = static_cast<const TIO*>(k);
     auto V = static_cast<const TIO*>(v);
@@ -389,7 +393,7 @@ hipError_t launch_recurrent(const void* q, const void* k, const void* v, const f
         const unsigned blocks = (unsigned)(B * Hv * (kD / kDecodeCols));
         hipLaunchKernelGGL((gdn_decode_kernel<kDecodeCols, kDecodeLpc, false, TIO>), dim3(blocks),
                            dim3(kDecodeLpc * kDecodeCols), 0, stream, Q, K, V, g_log, beta,
-                           GdnRawGates{}, state, O, Hq, Hv, scale);
+                           GdnRawGates{}, state_in, state, O, Hq, Hv, scale, st);
         return hipGetLastError();
     }
     const unsigned blocks = (unsigned)(B * Hv * kBlocksPerHead);
@@ -398,11 +402,11 @@ hipError_t launch_recurrent(const void* q, const void* k, const void* v, const f
     // sequences, fp16, T = 4 7.6 / 8.1, 6 9.3 / 8.9, 8 11.1 / 9.9, 31 33.3 / 21.8).
     if (T >= kStagedMinT) {
         hipLaunchKernelGGL(gdn_serial_kernel<TIO>, dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
-                           g_log, beta, state, O, T, Hq, Hv, scale);
+                           g_log, beta, state_in, state, O, T, Hq, Hv, scale, st);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(gdn_recurrent_kernel<TIO>, dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
-                       g_log, beta, state, O, T, Hq, Hv, scale);
+                       g_log, beta, state_in, state, O, T, Hq, Hv, scale, st);
     return hipGetLastError();
 }
 
@@ -424,8 +428,16 @@ hipError_t launch_naive(const void* q, const void* k, const void* v, const float
 hipError_t gdn_recurrent(const void* q, const void* k, const void* v, const float* g_log,
                          const float* beta, float* state, void* out, int B, int T, int Hq,
                          int Hv, float scale, bool f32, hipStream_t stream) {
-    return f32 ? launch_recurrent<float>(q, k, v, g_log, beta, state, out, B, T, Hq, Hv, scale, stream)
-               : launch_recurrent<half_t>(q, k, v, g_log, beta, state, out, B, T, Hq, Hv, scale, stream);
+    return gdn_recurrent_strided(q, k, v, gdn_dense(T, Hq, Hv), g_log, beta, state, state, out, B, T, Hq, Hv, scale,
+                                 f32, stream);
+}
+
+hipError_t gdn_recurrent_strided(const void* q, const void* k, const void* v, const GdnStrides& st,
+                                 const float* g_log, const float* beta, const float* state_in, float* state,
+                                 void* out, int B, int T, int Hq, int Hv, float scale, bool f32,
+                                 hipStream_t stream) {
+    return f32 ? launch_recurrent<float>(q, k, v, st, g_log, beta, state_in, state, out, B, T, Hq, Hv, scale, stream)
+               : launch_recurrent<half_t>(q, k, v, st, g_log, beta, state_in, state, out, B, T, Hq, Hv, scale, stream);
 }
 
 hipError_t gdn_decode_fused(const void* q, const void* k, const void* v, const GdnRawGates& gates,
@@ -435,7 +447,7 @@ hipError_t gdn_decode_fused(const void* q, const void* k, const void* v, const G
     hipLaunchKernelGGL((gdn_decode_kernel<kDecodeCols, kDecodeLpc, true, half_t>), dim3(blocks),
                        dim3(kDecodeLpc * kDecodeCols), 0, stream, static_cast<const half_t*>(q),
                        static_cast<const half_t*>(k), static_cast<const half_t*>(v), nullptr, nullptr,
-                       gates, state, static_cast<half_t*>(out), Hq, Hv, scale);
+                       gates, state, state, static_cast<half_t*>(out), Hq, Hv, scale, gdn_dense(1, Hq, Hv));
     return hipGetLastError();
 }
 

@@ -11,10 +11,11 @@
 // with S = 128.  q / k / v / out may be fp32 (ggml's op) or fp16 and any strides (views
 // into a fused projection); g_log, beta and the states are fp32.  When any of q / k / v / out
 // is fp32 the kernels run with fp32 I/O (fp16 operands are widened, exactly), so fp32
-// operands are never narrowed; when all four are fp16 they run with fp16 I/O.  Operands
-// already in the kernels' dense layout are used in place; the others are gathered into the
-// caller's workspace (and the output scattered back) by strided copy kernels.  state_out
-// may be the same buffer as state (in place).
+// operands are never narrowed; when all four are fp16 they run with fp16 I/O.  q, k
+// and v rows of the kernels' I/O type are read where they lie (any token, head and sequence
+// strides) and a dense state is read where it lies and written to state_out; what else is not in
+// the kernels' dense layout is gathered into the caller's workspace (and the output scattered
+// back) by strided copy kernels.  state_out may be the same buffer as state (in place).
 //
 // Dispatch on the tokens per sequence T: one token -> the decode kernel; T below
 // kChunkedMinT -> the token-serial kernel (state on chip for all T); otherwise the chunked
@@ -63,6 +64,16 @@ tsa::View4 dense_view(const int64_t (&ne)[4], size_t e) {
         stride *= ne[i];
     }
     return v;
+}
+
+// The memory of two views meets.
+bool overlap(const tsa_tensor& a, const tsa_tensor& b) {
+    auto end = [](const tsa_tensor& t) {
+        uintptr_t e = (uintptr_t)t.data + esize(t.type);
+        for (int i = 0; i < 4; ++i) e += (size_t)(t.ne[i] - 1) * t.nb[i];
+        return e;
+    };
+    return (uintptr_t)a.data < end(b) && (uintptr_t)b.data < end(a);
 }
 
 bool same_ne(const tsa_tensor& t, int64_t a, int64_t b, int64_t c, int64_t d) {
@@ -159,6 +170,29 @@ extern "C" int tsa_ggml_gated_delta_net(const tsa_tensor* q, const tsa_tensor* k
     hipError_t e = hipSuccess;
     auto ok = [&]() { return e == hipSuccess; };
 
+    // Rows of q, k and v where they lie, when the kernels can read them there: the I/O type,
+    // consecutive elements, 16-byte aligned rows, and a chunk's 64 tokens within a buffer
+    // descriptor's reach.  Gathering them first was a launch per operand, longer than the decode
+    // kernel's own time at a few sequences (8 sequences, 48 heads, one token: 3 x 2.4-2.8 us beside
+    // its 8.2).
+    // Not where the result would be written over them.
+    auto in_place = [&](const tsa_tensor& t) {
+        const size_t es = f32 ? 4 : 2;
+        if (!dense(t) && (overlap(t, *out) || overlap(t, *state_out))) return false;
+        if ((t.type == TSA_TYPE_F32) != f32 || t.nb[0] != es || ((uintptr_t)t.data & 15)) return false;
+        for (int i = 1; i < 4; ++i)
+            if (t.nb[i] % 16 || t.nb[i] > (size_t)INT64_MAX) return false;
+        return t.nb[2] <= (size_t)INT_MAX / 64;
+    };
+    // its strides, or those of the dense copy
+    auto strides = [&](const tsa_tensor& t) {
+        const long long es = f32 ? 4 : 2;
+        if (in_place(t)) return tsa::RowStride{(long long)t.nb[3] / es, (long long)t.nb[2] / es, (long long)t.nb[1] / es};
+        const long long row = t.ne[0] * t.ne[1];
+        return tsa::RowStride{row * t.ne[2], row, t.ne[0]};
+    };
+    const tsa::GdnStrides rows{strides(*q), strides(*k), strides(*v)};
+
     // operands in the kernels' layout: used in place when already dense, else gathered
     auto operand = [&](const tsa_tensor& t, size_t off, bool f16) -> void* {
         if (dense(t) && (t.type == TSA_TYPE_F16) == f16) return t.data;
@@ -167,25 +201,30 @@ extern "C" int tsa_ggml_gated_delta_net(const tsa_tensor* q, const tsa_tensor* k
                                   dense_view(t.ne, f16 ? 2 : 4), st);
         return dst;
     };
-    const void* qd = operand(*q, p.q, !f32);
-    const void* kd = operand(*k, p.k, !f32);
-    const void* vd = operand(*v, p.v, !f32);
+    const void* qd = in_place(*q) ? q->data : operand(*q, p.q, !f32);
+    const void* kd = in_place(*k) ? k->data : operand(*k, p.k, !f32);
+    const void* vd = in_place(*v) ? v->data : operand(*v, p.v, !f32);
     const float* gd = static_cast<const float*>(operand(*g, p.g, false));
     const float* bd = static_cast<const float*>(operand(*beta, p.beta, false));
-    // the state the kernels update in place: state_out itself when it is dense, else scratch
+    // the state the kernels write: state_out itself when it is dense, else scratch; they read
+    // state where it lies when that is dense (a copy first was 8 us at 8 sequences of 48 heads)
     float* sd = dense(*state_out) ? static_cast<float*>(state_out->data)
                                   : reinterpret_cast<float*>(w + p.state);
-    if (ok() && !(state->data == static_cast<void*>(sd) && dense(*state)))
-        e = tsa::copy4d(state->data, 0, view_of(*state), sd, 0, dense_view(state->ne, 4), st);
+    const float* si = static_cast<const float*>(state->data);
+    if (!dense(*state) || ((uintptr_t)state->data & 15) ||
+        (si != sd && (overlap(*state, *state_out) || overlap(*state, *out)))) {
+        if (ok()) e = tsa::copy4d(state->data, 0, view_of(*state), sd, 0, dense_view(state->ne, 4), st);
+        si = sd;
+    }
     const bool out_direct = dense(*out) && (out->type == TSA_TYPE_F32) == f32;
     void* od = out_direct ? out->data : static_cast<void*>(w + p.out);
     if (!ok()) return TSA_ERR_LAUNCH;
 
     const int B = (int)p.B, T = (int)p.T, Hk = (int)p.Hk, Hv = (int)p.Hv;
     if (T >= kChunkedMinT)
-        e = tsa::gdn_chunked(qd, kd, vd, gd, bd, sd, od, B, T, Hk, Hv, scale, w + p.chunk, f32, st);
+        e = tsa::gdn_chunked_strided(qd, kd, vd, rows, gd, bd, si, sd, od, B, T, Hk, Hv, scale, w + p.chunk, f32, st);
     else  // T == 1 takes the decode kernel inside gdn_recurrent
-        e = tsa::gdn_recurrent(qd, kd, vd, gd, bd, sd, od, B, T, Hk, Hv, scale, f32, st);
+        e = tsa::gdn_recurrent_strided(qd, kd, vd, rows, gd, bd, si, sd, od, B, T, Hk, Hv, scale, f32, st);
     if (ok() && !out_direct)
         e = tsa::copy4d(od, f32 ? 0 : 1, dense_view(out->ne, f32 ? 4 : 2), out->data,
                         out->type == TSA_TYPE_F16, view_of(*out), st);

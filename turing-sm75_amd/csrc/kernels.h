@@ -27,6 +27,19 @@ struct GdnRawGates {
     float eps;
 };
 
+// Where the rows of q, k and v lie: element strides between sequences, tokens and heads.  A row's
+// dk (dv) elements are consecutive, and rows start at multiples of 16 bytes.
+struct RowStride {
+    long long b, t, h;
+};
+struct GdnStrides {
+    RowStride q, k, v;
+};
+inline GdnStrides gdn_dense(int T, int Hq, int Hv) {
+    const RowStride qk{(long long)T * Hq * 128, (long long)Hq * 128, 128}, v{(long long)T * Hv * 128, (long long)Hv * 128, 128};
+    return {qk, qk, v};
+}
+
 // f32: q / k / v / out are fp32 (the reference's own I/O; a larger workspace), else fp16.
 // nseg: the sequence-split plan, 0 = the library's (a function of the shapes), 1 = no split,
 // n >= 2 = n segments (fewer when the sequence has fewer chunks).
@@ -34,6 +47,11 @@ size_t gdn_chunked_ws_bytes(int B, int T, int Hv, bool f32 = false, int nseg = 0
 hipError_t gdn_chunked(const void* q, const void* k, const void* v, const float* g_log,
                        const float* beta, float* state, void* out, int B, int T, int Hq, int Hv,
                        float scale, void* ws, bool f32, hipStream_t stream, int nseg = 0);
+// The same on rows that lie anywhere; state_in is read, state (which may be state_in) written.
+hipError_t gdn_chunked_strided(const void* q, const void* k, const void* v, const GdnStrides& strides,
+                               const float* g_log, const float* beta, const float* state_in, float* state,
+                               void* out, int B, int T, int Hq, int Hv, float scale, void* ws, bool f32,
+                               hipStream_t stream);
 // The chunked prefill without a caller workspace: the library's fixed device scratch array
 // (gdn_chunked_noalloc_max_bytes() bytes per GPU) stands in for it; no allocation, no side
 // stream.  The caller checks gdn_chunked_ws_bytes(...) against the maximum.
@@ -51,6 +69,11 @@ hipError_t gdn_chunked_redo_count(const void* ws, int B, int T, int Hv, bool f32
 hipError_t gdn_recurrent(const void* q, const void* k, const void* v, const float* g_log,
                          const float* beta, float* state, void* out, int B, int T, int Hq,
                          int Hv, float scale, bool f32, hipStream_t stream);
+// The same on rows that lie anywhere; state_in is read, state (which may be state_in) written.
+hipError_t gdn_recurrent_strided(const void* q, const void* k, const void* v, const GdnStrides& strides,
+                                 const float* g_log, const float* beta, const float* state_in, float* state,
+                                 void* out, int B, int T, int Hq, int Hv, float scale, bool f32,
+                                 hipStream_t stream);
 hipError_t gdn_chunked_fused(const void* q, const void* k, const void* v, const GdnRawGates& gates,
                              float* state, void* out, int B, int T, int Hq, int Hv, float scale,
                              void* ws, hipStream_t stream);
