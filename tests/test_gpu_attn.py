@@ -246,3 +246,28 @@ def test_valu_reference_driver_inputs(dev, orc):
     qkv = orc.mt_normal_half(42, 0.0, 0.5, n, 3).view(np.float16).reshape((3,) + shape)
     q, k, v = qkv[0], qkv[1], qkv[2]
     assert _err(_run(dev, q, k, v, True, valu=True), orc.attn_naive(q, k, v, True)) < TIGHT
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [
+    # D <= 128: 32-row query tiles around the lines of the split-key forms
+    (1, 1, 1, 1, 64), (1, 4, 4, 33, 64), (1, 16, 16, 1024, 64), (1, 16, 16, 1025, 64), (1, 32, 32, 2048, 64),
+    (1, 1, 1, 31, 128), (1, 8, 8, 1024, 128), (1, 8, 2, 1025, 128), (1, 16, 16, 3584, 128), (1, 16, 8, 3585, 128),
+    # around the one-per-CU and two-per-CU counts of whole tiles
+    (1, 16, 16, 3900, 128), (1, 40, 40, 1500, 128),
+    # D = 256: 128-row tiles from S = 129, and both sides of the count of 256-row ones
+    (1, 6, 1, 128, 256), (1, 6, 1, 129, 256), (1, 24, 4, 2048, 256), (1, 24, 4, 2049, 256), (1, 8, 4, 4097, 256)])
+def test_split_keys_dispatch(dev, B, Hq, Hkv, S, D, causal):
+    """Every form of the forward around the sizes where the dispatch changes, with odd lengths,
+    grouped heads and the gate, every row against the on-device naive kernel (fp32 dots, exact
+    two-pass softmax).  fp16 P and O: 2^-11 relative each against |O| <= ~2 here, 2e-3 absolute."""
+    import torch
+    g = torch.Generator(device=dev).manual_seed(S * 7 + D)
+    mk = lambda h: torch.randn(B, h, S, D, device=dev, generator=g).half()
+    q, k, v, gate = mk(Hq), mk(Hkv), mk(Hkv), mk(Hq)
+    o = tsa.attn_gqa_fwd(q, k, v, gate, causal=causal).float()
+    ref = tsa.attn_gqa_fwd(q, k, v, gate, causal=causal, naive=True).float()
+    torch.cuda.synchronize()
+    err = float((o - ref).abs().max())
+    print(f"B={B} {Hq}/{Hkv} S={S} D={D} causal={causal}: max-abs {err:.2e}")
+    assert torch.isfinite(o).all() and err < 2e-3 * max(1.0, float(ref.abs().max()))

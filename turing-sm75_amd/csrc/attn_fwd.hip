@@ -76,11 +76,17 @@ __device__ __forceinline__ int chunk_pos(int r, int c) {
 // 1.22 -> 0.49 GB of HBM traffic per launch); without groups XCD x runs heads x, x + 8, ...
 // (0.48 vs 0.56 GB at B=1 H=32 S=8192 D=128).  Causal runs issue the longest (highest) query
 // tiles first.
+// With two workgroups per CU (two) and no more workgroups than that, a CU's second one starts
+// with its first and the sum of the two decides: the later workgroups then go lightest first
+// (32 heads, S = 2001, D = 128: 52.5 -> 51.0 us).
 __device__ __forceinline__ void map_block(int bid, int BH, int n_qt, bool causal, int group,
-                                          int& bh, int& qt) {
+                                          int& bh, int& qt, bool two = false) {
     int rank;
     if ((BH & 7) == 0) {
-        const int xcd = bid & 7, slot = bid >> 3, hpx = BH >> 3;
+        constexpr int kCus = 32;  // per XCD
+        const int xcd = bid & 7, hpx = BH >> 3, slots = hpx * n_qt;
+        int slot = bid >> 3;
+        if (two && causal && slot >= kCus && slots <= 2 * kCus) slot = slots - 1 - (slot - kCus);
         bh = group > 1 ? xcd * hpx + slot % hpx : (slot % hpx) * 8 + xcd;
         rank = slot / hpx;
     } else {
@@ -107,9 +113,9 @@ __device__ __forceinline__ half4_t lds_read_tr16_at(unsigned addr) {
 // a tile of 64 rows x D halfs is kTile instructions, K then V, and wave w of kW issues
 // instructions w + kW j.  LDS chunk position p of row r holds source chunk p ^ swz(r), so
 // the tile lands in the same swizzled layout the operand reads expect.
-template <int D, int kW = 4>
+template <int D, int kW = 4, int kRows = kKRows>
 struct Dma {
-    static constexpr int kTile = kKRows * D * 2 / 1024;  // instructions per K (or V) tile
+    static constexpr int kTile = kRows * D * 2 / 1024;   // instructions per K (or V) tile
     static constexpr int kPerWave = 2 * kTile / kW;      // for kW waves per workgroup
     static constexpr int kChunks = D / 8;
     static_assert(kTile % kW == 0, "each wave copies whole groups of K and V blocks");
@@ -137,7 +143,7 @@ __device__ __forceinline__ void dma_issue(const void* base, unsigned off, unsign
 // (blk = w mod 4 fixes it), at D = 256 (two rows per block) when kW is a multiple of 8
 // (blk = w mod 8) -- block blk of a full tile sits at off0 + 1024 (blk - w): one register
 // for all copies.
-template <int D, int kPart, int kW>
+template <int D, int kPart, int kW, int kRowsT = kKRows>
 __device__ __forceinline__ void copy_tile(unsigned off0, int wave, const half_t* Kh, const half_t* Vh,
                                           int k0, int S, unsigned lds_buf) {
     static_assert(D <= 128 || kW % 8 == 0, "a wave's copy blocks must share one swizzle pattern");
@@ -146,8 +152,8 @@ __device__ __forceinline__ void copy_tile(unsigned off0, int wave, const half_t*
     const int lastrow = S - 1 - k0;
     auto issue_all = [&](auto Ragged) {  // a ragged last tile clamps its rows to S - 1
 #pragma unroll
-        for (int j = kPart * Dma<D, kW>::kPerWave / 2; j < (kPart + 1) * Dma<D, kW>::kPerWave / 2; ++j) {
-            constexpr int kT = Dma<D>::kTile;  // a multiple of kW, and wave < kW
+        for (int j = kPart * Dma<D, kW, kRowsT>::kPerWave / 2; j < (kPart + 1) * Dma<D, kW, kRowsT>::kPerWave / 2; ++j) {
+            constexpr int kT = Dma<D, kW, kRowsT>::kTile;  // a multiple of kW, and wave < kW
             const bool isv = kW * j >= kT;
             const int dblk = kW * j - (isv ? kT : 0);  // blk - wave
             unsigned o;
@@ -163,10 +169,10 @@ __device__ __forceinline__ void copy_tile(unsigned off0, int wave, const half_t*
                 o = (unsigned)min(row, lastrow) * kRowB + o0 % kRowB;
             }
             dma_issue(isv ? (const void*)vb : (const void*)kb, o,
-                      lds_buf + (unsigned)(isv ? kKRows * D * 2 : 0) + 1024u * (unsigned)(wave + dblk));
+                      lds_buf + (unsigned)(isv ? kRowsT * D * 2 : 0) + 1024u * (unsigned)(wave + dblk));
         }
     };
-    if (lastrow >= kKRows - 1)
+    if (lastrow >= kRowsT - 1)
         issue_all(std::false_type{});
     else
         issue_all(std::true_type{});
@@ -174,6 +180,34 @@ __device__ __forceinline__ void copy_tile(unsigned off0, int wave, const half_t*
 __device__ __forceinline__ void dma_wait_barrier() {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's copies have landed
     lds_barrier();
+}
+
+// Epilogue: O = O^T / l (times sigmoid(gate)), 4 consecutive d per store.  O, gate: the head's rows.
+template <int D>
+__device__ __forceinline__ void store_o(const float16_t (&o)[Cfg<D>::kDBlocks], float l, half_t* __restrict__ O,
+                                        const half_t* __restrict__ gate, int my_q, int S, int hi) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    if (my_q < S) {
+        half_t* orow = O + (size_t)my_q * D;
+        const half_t* grow = gate ? gate + (size_t)my_q * D : nullptr;
+#pragma unroll
+        for (int db = 0; db < Cfg<D>::kDBlocks; ++db)
+#pragma unroll
+            for (int rg = 0; rg < 4; ++rg) {
+                const int d0 = 32 * db + 8 * rg + 4 * hi;
+                float f[4] = {inv, inv, inv, inv};
+                if (grow) {
+                    const half4_t g4 = *reinterpret_cast<const half4_t*>(grow + d0);
+                    // sigmoid by the hardware reciprocal (1 ulp): an IEEE division per element
+                    // was ~10 VALU ops, 128 of them per lane at D = 256 in every workgroup's tail
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) f[e] = inv * __builtin_amdgcn_rcpf(1.f + __expf(-(float)g4[e]));
+                }
+                const half4_t v4 = {(half_t)(o[db][4 * rg] * f[0]), (half_t)(o[db][4 * rg + 1] * f[1]),
+                                    (half_t)(o[db][4 * rg + 2] * f[2]), (half_t)(o[db][4 * rg + 3] * f[3])};
+                *reinterpret_cast<half4_t*>(orow + d0) = v4;
+            }
+    }
 }
 
 // kW waves per workgroup, 32 query rows each: kW = 4 at D <= 128 (two workgroups per CU,
@@ -193,7 +227,7 @@ attn_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hi = lane >> 5;  // which half of the wave
     int bh, qt;
-    map_block(blockIdx.x, BH, n_qt, kCausal, group, bh, qt);
+    map_block(blockIdx.x, BH, n_qt, kCausal, group, bh, qt, D <= 128);
     const size_t head = (size_t)bh * S * D;  // Q, O, gate: query head bh = b * Hq + h
     const size_t kvhead = (size_t)((bh / Hq) * (Hq / group) + (bh % Hq) / group) * S * D;
     const int q0 = qt * (32 * kW);
@@ -472,30 +506,215 @@ attn_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         }
     }
 
-    // ---- epilogue: O = O^T / l (times sigmoid(gate)), 4 consecutive d per store ----
+    store_o<D>(o, sum_xor32(l), O + head, gate ? gate + head : nullptr, my_q, S, hi);
+}
+
+// ---------------------------------------------------------------------------------
+// The same forward with a workgroup's keys split over its waves, for grids that leave the device
+// idle or end in a long tail: kQG * kKG waves own 32 kQG query rows, and wave (qg, kg) takes the
+// kg-th kKT keys of every tile of kKG kKT keys, with a running max, sum and O of its own that
+// meet in LDS at the end.  A workgroup then does its rows in 1 / kKG of the steps: the longest
+// workgroup of a causal grid, which sets the time when there are no more workgroups than fit the
+// device, is that much shorter, and small grids have kKG times the waves.  The 32-key halves, their
+// operand read-ahead and the copies are those of attn_fwd_kernel's D = 256 form.
+// ---------------------------------------------------------------------------------
+template <int D, bool kCausal, int kQG, int kKG, int kKT>
+__global__ void __launch_bounds__(64 * kQG * kKG, 2)
+attn_ksplit_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
+                   const half_t* __restrict__ V, const half_t* __restrict__ gate,
+                   half_t* __restrict__ O, int S, int BH, int n_qt, int Hq, int group,
+                   float c2 /* scale * log2(e) */) {
+    using C = Cfg<D>;
+    constexpr int kW = kQG * kKG, kRows = kKG * kKT;  // waves; keys per tile
+    constexpr int kBuf = 2 * kRows * D;               // halfs per buffer (K, V)
+    static_assert(2 * kBuf * 2 >= (kKG - 1) * kQG * 32 * D * 4, "the partial O's fit the tile buffers");
+    static_assert((kW * 1024 / (2 * D)) % 16 == 0, "a wave's copy blocks must share one swizzle pattern");
+    __shared__ __align__(1024) half_t lds[2 * kBuf];
+    __shared__ float2 ml[kKG][kQG][64];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int qg = wave % kQG, kg = wave / kQG;
+    const int hi = lane >> 5;
+    int bh, qt;
+    map_block(blockIdx.x, BH, n_qt, kCausal, group, bh, qt);
+    const size_t head = (size_t)bh * S * D;
+    const size_t kvhead = (size_t)((bh / Hq) * (Hq / group) + (bh % Hq) / group) * S * D;
+    const int q0 = qt * (32 * kQG);
+    const int qw0 = q0 + 32 * qg;
+    const int my_q = qw0 + (lane & 31);
+
+    half8_t qf[C::kKSteps];
+#pragma unroll
+    for (int kk = 0; kk < C::kKSteps; ++kk) {
+        if (my_q < S)
+            qf[kk] = *reinterpret_cast<const half8_t*>(Q + head + (size_t)my_q * D + 16 * kk + 8 * hi);
+        else
+            qf[kk] = half8_t{};
+    }
+    const int kv_end = kCausal ? min(S, q0 + 32 * kQG) : S;
+    const int n_tiles = (kv_end + kRows - 1) / kRows;
+    const int wave_kv_end = kCausal ? min(S, qw0 + 32) : S;
+
+    float16_t o[C::kDBlocks];
+#pragma unroll
+    for (int i = 0; i < C::kDBlocks; ++i) o[i] = float16_t{};
+    float m = -INFINITY, l = 0.f;
+
+    const int krow = lane & 31, ksw = swz<D>(krow);
+    const int g16 = lane >> 4, i16 = lane & 15;
+    const int vj = i16 >> 2, vm = i16 & 3;
+    const int vchunk = 2 * (g16 & 1) + (vm >> 1), vsub = 4 * (vm & 1);
+    const unsigned off = dma_off<D>(wave, lane, kRows - 1);
+    const unsigned lds0 = (unsigned)(uintptr_t)(lds_void_t)(void*)lds;
+    constexpr unsigned kBufB = kBuf * 2, kRowB = 2 * D;
+    // this wave's share of a tile starts kKT kg rows in (a multiple of 16: the swizzle is the same)
+    const unsigned goff = (unsigned)(kKT * kg) * kRowB;
+    unsigned ka = lds0 + goff + krow * kRowB + 16u * (unsigned)(hi ^ ksw);
+    unsigned va[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int r = 4 * hi + vj + 8 * e;
+        va[e] = lds0 + goff + kRows * kRowB + r * kRowB + 16u * (unsigned)chunk_pos<D>(r, vchunk) + 2u * vsub;
+    }
+    const half_t* Kh = K + kvhead;
+    const half_t* Vh = V + kvhead;
+    copy_tile<D, 0, kW, kRows>(off, wave, Kh, Vh, 0, S, lds0);
+    copy_tile<D, 1, kW, kRows>(off, wave, Kh, Vh, 0, S, lds0);
+    dma_wait_barrier();
+
+    for (int t = 0; t < n_tiles; ++t) {
+        const unsigned ubase = (unsigned)(t & 1) * kBufB, nbuf = lds0 + (unsigned)((t + 1) & 1) * kBufB;
+        const bool more = t + 1 < n_tiles;
+        if (more) copy_tile<D, 0, kW, kRows>(off, wave, Kh, Vh, (t + 1) * kRows, S, nbuf);
+        bool copied = false;
+#pragma unroll
+        for (int kb = 0; kb < kKT / 32; ++kb) {
+            const int kb0 = t * kRows + kKT * kg + 32 * kb;  // first key of this half
+            if (kb0 >= wave_kv_end) break;
+            asm volatile("" : "+v"(ka), "+v"(va[0]), "+v"(va[1]));
+            constexpr int kPreK = 3;
+            float16_t sh = float16_t{};
+            half8_t kop[C::kKSteps];
+            auto read_k = [&](int kk) {
+                kop[kk] = lds_read_b128((ka ^ (32u * kk)) + ubase + (unsigned)(32 * kb) * kRowB);
+            };
+#pragma unroll
+            for (int kk = 0; kk < kPreK; ++kk) read_k(kk);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kk = 0; kk < C::kKSteps; ++kk) {
+                if (kk + kPreK < C::kKSteps) read_k(kk + kPreK);
+                sh = mfma32(kop[kk], qf[kk], sh);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if ((kCausal && kb0 + 31 > qw0) || kb0 + 32 > S) {
+                const int base = kb0 + 4 * hi;
+                const int lim_q = kCausal ? my_q - base : INT_MAX;
+                const int lim_s = S - base;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int c = 8 * (r >> 2) + (r & 3);
+                    if (c > lim_q || c >= lim_s) sh[r] = -INFINITY;
+                }
+            }
+            float mx = sh[0];
+#pragma unroll
+            for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sh[r]);
+            mx = max_xor32(mx);
+            if (__builtin_amdgcn_ballot_w64((mx - m) * c2 > 8.f)) {
+                const float m_new = fmaxf(m, mx);
+                const float alpha = m_new == -INFINITY ? 1.f : fast_exp2((m - m_new) * c2);
+                m = m_new;
+                l *= alpha;
+#pragma unroll
+                for (int db = 0; db < C::kDBlocks; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+            }
+            const float mc = m == -INFINITY ? 0.f : m * c2;
+            half8_t p[2];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) p[r >> 3][r & 7] = (half_t)fast_exp2(fmaf(sh[r], c2, -mc));
+            const half2_t one2 = {(half_t)1.f, (half_t)1.f};
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    l = __builtin_amdgcn_fdot2(half2_t{p[i][2 * u], p[i][2 * u + 1]}, one2, l, false);
+            auto read_v = [&](int ks, int db) {
+                const unsigned a = ubase + (unsigned)(32 * D * ks);
+                const half4_t lo = lds_read_tr16_at((va[0] ^ (64u * db)) + a);
+                const half4_t up = lds_read_tr16_at((va[1] ^ (64u * db)) + a);
+                return half8_t{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
+            };
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+            constexpr int kSteps = 2 * C::kDBlocks, kPreV = 2;
+            half8_t vbuf[kSteps];
+#pragma unroll
+            for (int i = 0; i < kPreV; ++i) vbuf[i] = read_v(2 * kb + i / C::kDBlocks, i % C::kDBlocks);
+#pragma unroll
+            for (int i = 0; i < kSteps; ++i) {
+                const int ks = i / C::kDBlocks, db = i % C::kDBlocks;
+                if (i + kPreV < kSteps)
+                    vbuf[i + kPreV] = read_v(2 * kb + (i + kPreV) / C::kDBlocks, (i + kPreV) % C::kDBlocks);
+                if (kb == 0 && i == C::kDBlocks && more) {
+                    copy_tile<D, 1, kW, kRows>(off, wave, Kh, Vh, (t + 1) * kRows, S, nbuf);
+                    copied = true;
+                }
+                o[db] = mfma32(vbuf[i], p[ks], o[db]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        if (more && !copied) copy_tile<D, 1, kW, kRows>(off, wave, Kh, Vh, (t + 1) * kRows, S, nbuf);
+        dma_wait_barrier();
+    }
+
+    // ---- merge: the partial O's of the key groups past the first, lane for lane, through the tile
+    // buffers (every wave is past its last read of them) ----
     l = sum_xor32(l);
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    if (my_q < S) {
-        half_t* orow = O + head + (size_t)my_q * D;
-        const half_t* grow = gate ? gate + head + (size_t)my_q * D : nullptr;
+    float4* part = reinterpret_cast<float4*>(lds);
+    constexpr int kPart4 = C::kDBlocks * 4 * 64;  // float4s per wave's O
+    if (kg > 0) {
+        float4* w = part + (size_t)((kg - 1) * kQG + qg) * kPart4;
 #pragma unroll
         for (int db = 0; db < C::kDBlocks; ++db)
 #pragma unroll
-            for (int rg = 0; rg < 4; ++rg) {
-                const int d0 = 32 * db + 8 * rg + 4 * hi;
-                float f[4] = {inv, inv, inv, inv};
-                if (grow) {
-                    const half4_t g4 = *reinterpret_cast<const half4_t*>(grow + d0);
-                    // sigmoid by the hardware reciprocal (1 ulp): an IEEE division per element
-                    // was ~10 VALU ops, 128 of them per lane at D = 256 in every workgroup's tail
+            for (int r = 0; r < 4; ++r)
+                w[(db * 4 + r) * 64 + lane] = make_float4(o[db][4 * r], o[db][4 * r + 1], o[db][4 * r + 2], o[db][4 * r + 3]);
+        ml[kg][qg][lane] = make_float2(m, l);
+    }
+    lds_barrier();
+    if (kg > 0) return;
+    // (a group without keys for the row has m = -inf and factor 0; group 0 holds key 0, which every
+    // row sees)
+#pragma unroll 1
+    for (int i = 1; i < kKG; ++i) {
+        const float2 x = ml[i][qg][lane];
+        const float mt = fmaxf(m, x.x);
+        const float f0 = m == -INFINITY ? 0.f : fast_exp2((m - mt) * c2);
+        const float f1 = x.x == -INFINITY ? 0.f : fast_exp2((x.x - mt) * c2);
+        m = mt;
+        l = fmaf(x.y, f1, l * f0);
+        const float4* w = part + (size_t)((i - 1) * kQG + qg) * kPart4 + lane;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) f[e] = inv * __builtin_amdgcn_rcpf(1.f + __expf(-(float)g4[e]));
-                }
-                const half4_t v4 = {(half_t)(o[db][4 * rg] * f[0]), (half_t)(o[db][4 * rg + 1] * f[1]),
-                                    (half_t)(o[db][4 * rg + 2] * f[2]), (half_t)(o[db][4 * rg + 3] * f[3])};
-                *reinterpret_cast<half4_t*>(orow + d0) = v4;
+        for (int db = 0; db < C::kDBlocks; ++db)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float4 y = w[(db * 4 + r) * 64];
+                float a0 = fmaf(y.x, f1, o[db][4 * r] * f0), a1 = fmaf(y.y, f1, o[db][4 * r + 1] * f0);
+                float a2 = fmaf(y.z, f1, o[db][4 * r + 2] * f0), a3 = fmaf(y.w, f1, o[db][4 * r + 3] * f0);
+                // keeps the next read behind these sums: the reads hoisted together spill
+                asm volatile("" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)::"memory");
+                o[db][4 * r] = a0;
+                o[db][4 * r + 1] = a1;
+                o[db][4 * r + 2] = a2;
+                o[db][4 * r + 3] = a3;
             }
     }
+    store_o<D>(o, l, O + head, gate ? gate + head : nullptr, my_q, S, hi);
 }
 
 template <int D, bool kCausal>
@@ -503,6 +722,28 @@ hipError_t launch(const half_t* q, const half_t* k, const half_t* v, const half_
                   int B, int Hq, int Hkv, int S, float scale, hipStream_t stream) {
     constexpr int kW = D == 256 ? 8 : 4;
     const int BH = B * Hq;
+    // The split-key form where whole query tiles leave the device idle, by the number of 32-row query
+    // tiles (D <= 128) or of 256-row ones (D = 256).  us per call, whole tiles / split, causal unless
+    // noted: D = 64 128 tiles 17.5 / 9.3, 512 18.5 / 10.8, 1024 18.5 / 13.9, 2000 63.8 / 53.6, 4000
+    // 91.9 / 95.4; D = 128 32 tiles 9.9 / 7.6, 252 39.9 / 26.1, 512 23.7 / 18.1, 1024 24.0 / 21.5, 1504
+    // 36.8 / 33.5, 2016 51.0 / 52.8, 4000 142 / 167; D = 256 12 tiles 58.6 / 42.6, 72 45.0 / 36.8, 144 86.6 / 64.8, 288 161 /
+    // 173.  At D = 256 a split tile moves its K and V for half the queries (10 TB/s from L2 at
+    // that rate), so without a mask's uneven tiles it pays only while its workgroups fit the CUs.
+    auto split = [&](auto kernel, int rows, int waves) {
+        const int n = (S + rows - 1) / rows;
+        hipLaunchKernelGGL(kernel, dim3(BH * n), dim3(64 * waves), 0, stream, q, k, v, gate, o, S, BH, n, Hq,
+                           Hq / Hkv, scale * kLog2e);
+        return hipGetLastError();
+    };
+    if constexpr (D == 256) {
+        const long long tiles = (long long)BH * ((S + 255) / 256), half = (long long)BH * ((S + 127) / 128);
+        if (S > 128 && (kCausal ? tiles <= 192 : half <= 256))
+            return split(attn_ksplit_kernel<D, kCausal, 4, 2, 32>, 128, 8);
+    } else {
+        const long long tiles = (long long)BH * ((S + 31) / 32);
+        if (tiles <= (D == 64 ? 512 : 256)) return split(attn_ksplit_kernel<D, kCausal, 1, 4, 32>, 32, 4);
+        if (tiles <= (D == 64 ? 2048 : 1792)) return split(attn_ksplit_kernel<D, kCausal, 2, 2, D == 64 ? 64 : 32>, 64, 4);
+    }
     const int n_qt = (S + 32 * kW - 1) / (32 * kW);
     hipLaunchKernelGGL((attn_fwd_kernel<D, kCausal, kW>), dim3(BH * n_qt), dim3(64 * kW), 0,
                        stream, q, k, v, gate, o, S, BH, n_qt, Hq, Hq / Hkv, scale * kLog2e);
