@@ -256,7 +256,8 @@ def test_valu_reference_driver_inputs(dev, orc):
     # around the one-per-CU and two-per-CU counts of whole tiles
     (1, 16, 16, 3900, 128), (1, 40, 40, 1500, 128),
     # D = 256: 128-row tiles from S = 129, and both sides of the count of 256-row ones
-    (1, 6, 1, 128, 256), (1, 6, 1, 129, 256), (1, 24, 4, 2048, 256), (1, 24, 4, 2049, 256), (1, 8, 4, 4097, 256)])
+    (1, 6, 1, 128, 256), (1, 6, 1, 129, 256), (1, 24, 4, 2048, 256), (1, 24, 4, 2049, 256), (1, 8, 4, 4097, 256), (1, 40, 8, 2000, 256),
+    (1, 40, 8, 2049, 256)])
 def test_split_keys_dispatch(dev, B, Hq, Hkv, S, D, causal):
     """Every form of the forward around the sizes where the dispatch changes, with odd lengths,
     grouped heads and the gate, every row against the on-device naive kernel (fp32 dots, exact

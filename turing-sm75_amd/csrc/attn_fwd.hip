@@ -146,7 +146,8 @@ __device__ __forceinline__ void dma_issue(const void* base, unsigned off, unsign
 template <int D, int kPart, int kW, int kRowsT = kKRows>
 __device__ __forceinline__ void copy_tile(unsigned off0, int wave, const half_t* Kh, const half_t* Vh,
                                           int k0, int S, unsigned lds_buf) {
-    static_assert(D <= 128 || kW % 8 == 0, "a wave's copy blocks must share one swizzle pattern");
+    constexpr int kStep = kW * 1024 / (2 * D);  // rows from one of a wave's blocks to its next
+    static_assert(kStep % 8 == 0, "a wave's copy blocks share one swizzle pattern up to its row bit 3");
     const half_t* kb = Kh + (size_t)k0 * D;
     const half_t* vb = Vh + (size_t)k0 * D;
     const int lastrow = S - 1 - k0;
@@ -156,14 +157,16 @@ __device__ __forceinline__ void copy_tile(unsigned off0, int wave, const half_t*
             constexpr int kT = Dma<D, kW, kRowsT>::kTile;  // a multiple of kW, and wave < kW
             const bool isv = kW * j >= kT;
             const int dblk = kW * j - (isv ? kT : 0);  // blk - wave
+            // an odd number of 8-row steps flips row bit 3, which the swizzle has as bit 1 of the chunk
+            const unsigned flip = kStep % 16 == 8 && ((dblk / kW) & 1) ? 32u : 0u;
             unsigned o;
             if constexpr (!decltype(Ragged)::value) {
-                o = off0 + 1024u * (unsigned)dblk;
+                o = (off0 ^ flip) + 1024u * (unsigned)dblk;
             } else {  // the same offset with its row clamped to S - 1
                 constexpr unsigned kRowB = 2 * D, kRows = 1024 / kRowB;
                 // the empty asm keeps this arithmetic inside the ragged branch (hoisted, its
                 // values take registers for the whole loop)
-                unsigned o0 = off0;
+                unsigned o0 = off0 ^ flip;
                 asm volatile("" : "+v"(o0));
                 const int row = (int)(o0 / kRowB) + (int)kRows * dblk;
                 o = (unsigned)min(row, lastrow) * kRowB + o0 % kRowB;
@@ -516,7 +519,8 @@ attn_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 // meet in LDS at the end.  A workgroup then does its rows in 1 / kKG of the steps: the longest
 // workgroup of a causal grid, which sets the time when there are no more workgroups than fit the
 // device, is that much shorter, and small grids have kKG times the waves.  The 32-key halves, their
-// operand read-ahead and the copies are those of attn_fwd_kernel's D = 256 form.
+// operand read-ahead and the copies are those of attn_fwd_kernel's D = 256 form.  (kKG = 1: no split, a shorter
+// query tile.)
 // ---------------------------------------------------------------------------------
 template <int D, bool kCausal, int kQG, int kKG, int kKT>
 __global__ void __launch_bounds__(64 * kQG * kKG, 2)
@@ -528,16 +532,15 @@ attn_ksplit_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     constexpr int kW = kQG * kKG, kRows = kKG * kKT;  // waves; keys per tile
     constexpr int kBuf = 2 * kRows * D;               // halfs per buffer (K, V)
     static_assert(2 * kBuf * 2 >= (kKG - 1) * kQG * 32 * D * 4, "the partial O's fit the tile buffers");
-    static_assert((kW * 1024 / (2 * D)) % 16 == 0, "a wave's copy blocks must share one swizzle pattern");
     __shared__ __align__(1024) half_t lds[2 * kBuf];
-    __shared__ float2 ml[kKG][kQG][64];
+    __shared__ float2 ml[kKG][kKG > 1 ? kQG : 1][kKG > 1 ? 64 : 1];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int qg = wave % kQG, kg = wave / kQG;
+    const int qg = kKG == 1 ? wave : wave % kQG, kg = kKG == 1 ? 0 : wave / kQG;
     const int hi = lane >> 5;
     int bh, qt;
-    map_block(blockIdx.x, BH, n_qt, kCausal, group, bh, qt);
+    map_block(blockIdx.x, BH, n_qt, kCausal, group, bh, qt, kKG == 1);
     const size_t head = (size_t)bh * S * D;
     const size_t kvhead = (size_t)((bh / Hq) * (Hq / group) + (bh % Hq) / group) * S * D;
     const int q0 = qt * (32 * kQG);
@@ -677,42 +680,44 @@ attn_ksplit_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     l = sum_xor32(l);
     float4* part = reinterpret_cast<float4*>(lds);
     constexpr int kPart4 = C::kDBlocks * 4 * 64;  // float4s per wave's O
-    if (kg > 0) {
-        float4* w = part + (size_t)((kg - 1) * kQG + qg) * kPart4;
+    if constexpr (kKG > 1) {
+        if (kg > 0) {
+            float4* w = part + (size_t)((kg - 1) * kQG + qg) * kPart4;
 #pragma unroll
-        for (int db = 0; db < C::kDBlocks; ++db)
+            for (int db = 0; db < C::kDBlocks; ++db)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                w[(db * 4 + r) * 64 + lane] = make_float4(o[db][4 * r], o[db][4 * r + 1], o[db][4 * r + 2], o[db][4 * r + 3]);
-        ml[kg][qg][lane] = make_float2(m, l);
-    }
-    lds_barrier();
-    if (kg > 0) return;
-    // (a group without keys for the row has m = -inf and factor 0; group 0 holds key 0, which every
-    // row sees)
+                for (int r = 0; r < 4; ++r)
+                    w[(db * 4 + r) * 64 + lane] = make_float4(o[db][4 * r], o[db][4 * r + 1], o[db][4 * r + 2], o[db][4 * r + 3]);
+            ml[kg][qg][lane] = make_float2(m, l);
+        }
+        lds_barrier();
+        if (kg > 0) return;
+        // (a group without keys for the row has m = -inf and factor 0; group 0 holds key 0, which every
+        // row sees)
 #pragma unroll 1
-    for (int i = 1; i < kKG; ++i) {
-        const float2 x = ml[i][qg][lane];
-        const float mt = fmaxf(m, x.x);
-        const float f0 = m == -INFINITY ? 0.f : fast_exp2((m - mt) * c2);
-        const float f1 = x.x == -INFINITY ? 0.f : fast_exp2((x.x - mt) * c2);
-        m = mt;
-        l = fmaf(x.y, f1, l * f0);
-        const float4* w = part + (size_t)((i - 1) * kQG + qg) * kPart4 + lane;
+        for (int i = 1; i < kKG; ++i) {
+            const float2 x = ml[i][qg][lane];
+            const float mt = fmaxf(m, x.x);
+            const float f0 = m == -INFINITY ? 0.f : fast_exp2((m - mt) * c2);
+            const float f1 = x.x == -INFINITY ? 0.f : fast_exp2((x.x - mt) * c2);
+            m = mt;
+            l = fmaf(x.y, f1, l * f0);
+            const float4* w = part + (size_t)((i - 1) * kQG + qg) * kPart4 + lane;
 #pragma unroll
-        for (int db = 0; db < C::kDBlocks; ++db)
+            for (int db = 0; db < C::kDBlocks; ++db)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float4 y = w[(db * 4 + r) * 64];
-                float a0 = fmaf(y.x, f1, o[db][4 * r] * f0), a1 = fmaf(y.y, f1, o[db][4 * r + 1] * f0);
-                float a2 = fmaf(y.z, f1, o[db][4 * r + 2] * f0), a3 = fmaf(y.w, f1, o[db][4 * r + 3] * f0);
-                // keeps the next read behind these sums: the reads hoisted together spill
-                asm volatile("" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)::"memory");
-                o[db][4 * r] = a0;
-                o[db][4 * r + 1] = a1;
-                o[db][4 * r + 2] = a2;
-                o[db][4 * r + 3] = a3;
-            }
+                for (int r = 0; r < 4; ++r) {
+                    const float4 y = w[(db * 4 + r) * 64];
+                    float a0 = fmaf(y.x, f1, o[db][4 * r] * f0), a1 = fmaf(y.y, f1, o[db][4 * r + 1] * f0);
+                    float a2 = fmaf(y.z, f1, o[db][4 * r + 2] * f0), a3 = fmaf(y.w, f1, o[db][4 * r + 3] * f0);
+                    // keeps the next read behind these sums: the reads hoisted together spill
+                    asm volatile("" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)::"memory");
+                    o[db][4 * r] = a0;
+                    o[db][4 * r + 1] = a1;
+                    o[db][4 * r + 2] = a2;
+                    o[db][4 * r + 3] = a3;
+                }
+        }
     }
     store_o<D>(o, l, O + head, gate ? gate + head : nullptr, my_q, S, hi);
 }
@@ -739,6 +744,11 @@ hipError_t launch(const half_t* q, const half_t* k, const half_t* v, const half_
         const long long tiles = (long long)BH * ((S + 255) / 256), half = (long long)BH * ((S + 127) / 128);
         if (S > 128 && (kCausal ? tiles <= 192 : half <= 256))
             return split(attn_ksplit_kernel<D, kCausal, 4, 2, 32>, 128, 8);
+        // Somewhat more tiles than CUs leave a second round nearly empty: half tiles, two workgroups
+        // per CU, 32-key steps and no split there (the same keys in the same order, so the same
+        // values; us, whole / half tiles, causal 216 tiles 119 / 106, 256 194 / 182, 264 137 / 126, 288
+        // 157.4 / 159.2; no mask 264 289 / 180, 288 337 / 319; from 384 on within 4 % either way).
+        if (tiles > 192 && tiles <= (kCausal ? 272 : 320)) return split(attn_ksplit_kernel<D, kCausal, 4, 1, 32>, 128, 4);
     } else {
         const long long tiles = (long long)BH * ((S + 31) / 32);
         if (tiles <= (D == 64 ? 512 : 256)) return split(attn_ksplit_kernel<D, kCausal, 1, 4, 32>, 32, 4);
