@@ -240,7 +240,9 @@ size_t tsa_ggml_gdn_workspace_bytes(const tsa_tensor* q, const tsa_tensor* v);
  * any strides); g_log, beta [Hv, T, B, 1] and state, state_out [S, S, Hv, B] fp32
  * (state_out may be state itself, the same view).  S = 128; V-head h reads QK head h % Hk.
  * Dispatches on T: the decode step (T = 1), the token-serial kernel, or the chunked
- * prefill.  Dense fp16 / fp32 operands are used in place; others are gathered into ws. */
+ * prefill.  q, k and v rows of the call's type are read where they lie (consecutive elements,
+ * 16-byte aligned rows, any other strides), and so is a dense state; others are gathered into
+ * ws. */
 int tsa_ggml_gated_delta_net(const tsa_tensor* q, const tsa_tensor* k, const tsa_tensor* v,
                              const tsa_tensor* g_log, const tsa_tensor* beta,
                              const tsa_tensor* state, const tsa_tensor* out,
