@@ -443,6 +443,29 @@ def test_chunked_column_tiles(dev, orc, hq, hv, T, io):
 
 
 @pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("hv,T,nseg", [(4, 1, None), (4, 64, None), (4, 128, None), (4, 180, None), (40, 180, None),
+                                       (2, 374, 2)])
+def test_chunked_state_above_the_fp16_range(dev, orc, hv, T, nseg, io):
+    """A final state with entries above 65504, which only the last token writes (k = 4 on one
+    coordinate, v = 2e4, beta = 1: 8e4): the fp32 state is finite and no later chunk reads it, at
+    one, two and three chunks, in both widths of the carry and in a split of two segments of
+    three chunks."""
+    rng = np.random.default_rng(2100 + T)
+    q, k, v, g, beta, st = _inputs(rng, 1, T, 2, hv, sstd=0.02)
+    k[:, -1] = 0
+    k[:, -1, :, 5] = 4
+    v[:, -1] = 2e4
+    beta[:, -1], g[:, -1] = 1.0, 0.0
+    q, k, v = _as(io, q, k, v)
+    o, s = _gpu(dev, "chunked", q, k, v, g, beta, st, nseg=nseg)
+    o_ref, s_ref = orc.gdn_serial(q, k, v, g, beta, st)
+    assert np.abs(s_ref).max() > 65520 and np.isfinite(s).all()
+    es, eo = _rel(s, s_ref), _rel(o, o_ref)
+    print(f"{io} Hv={hv} T={T}: state rel {es:.2e}  out rel {eo:.2e}")
+    assert es < TOL["chunked"][1] and eo < 1e-3
+
+
+@pytest.mark.parametrize("io", ["f16", "f32"])
 @pytest.mark.parametrize("T", [5, 6, 7, 8, 9, 15, 16, 17, 24, 33])
 def test_recurrent_token_blocks(dev, orc, T, io):
     """The token-serial kernel's two forms around their line (6 tokens) and at the remainders of

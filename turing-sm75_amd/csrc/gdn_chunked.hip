@@ -703,7 +703,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
             const float4 e = *reinterpret_cast<const float4*>(cs.G + kC + 16 * w + 4 * g);
             ek[0] = e.x; ek[1] = e.y; ek[2] = e.z; ek[3] = e.w;
         };
-        auto step = [&](const CarrySlot<TIO, NC>& cs, const CarrySlot<TIO, NC>& nx, int ch) __attribute__((always_inline)) {
+        auto step = [&](const CarrySlot<TIO, NC>& cs, const CarrySlot<TIO, NC>& nx) __attribute__((always_inline)) {
             // ---- 1. X = K S; R = V - e^G X ----
             half8_t Sh[NC][4], Sl[NC][4];
 #pragma unroll
@@ -753,7 +753,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
             // K^T operands and factors of step 3 (and e^{G_63 - G}): under step 2
             half8_t aK[2][2], aKl[2][2];
             const float4 d4 = *reinterpret_cast<const float4*>(cs.G + 2 * kC + 16 * w + 4 * g);
-            const float ec = ch < nch ? cs.G[3 * kC] : 1.f;
+            const float ec = cs.G[3 * kC];
 #pragma unroll
             for (int m = 0; m < 2; ++m)
 #pragma unroll
@@ -827,11 +827,18 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
         put_state();
         lds_barrier();  // S written; the helpers' copy of chunk 0 is in its slot
         ahead(sm.c[0]);
-        // an odd count runs a chunk past the last one, whose operands read as zero and leave the
-        // state as it is
-        for (int ch = 0; ch < nch; ch += 2) {
-            step(sm.c[0], sm.c[1], ch);
-            step(sm.c[1], sm.c[0], ch + 1);
+        // With an odd count the helper waves take a chunk past the last one, whose operands read as
+        // zero; the chain waves only meet its barriers.  (Its products would not leave the state as it
+        // is: an entry above the fp16 range is infinite in the operand, and 0 * inf is NaN.)
+        for (int ch = 0; ch + 1 < nch; ch += 2) {
+            step(sm.c[0], sm.c[1]);
+            step(sm.c[1], sm.c[0]);
+        }
+        if (nch & 1) {
+            step(sm.c[0], sm.c[1]);
+            lds_barrier();
+            lds_barrier();
+            lds_barrier();
         }
         bool lost = false;
         if constexpr (kFlags) {
