@@ -465,6 +465,37 @@ def test_chunked_state_above_the_fp16_range(dev, orc, hv, T, nseg, io):
     assert es < TOL["chunked"][1] and eo < 1e-3
 
 
+@pytest.mark.parametrize("io,hv,T", [("f16", 266400, 70), ("f32", 133200, 64)])
+def test_chunked_rows_past_32_bit_offsets(dev, io, hv, T):
+    """Heads whose 63 token rows of V and the output lie more than 2^32 bytes apart, two chunks and
+    one, against the token-serial kernel: per-head relative error in the 2-norm.  A row read or
+    written 2^32 bytes off is another token's, an error of the order of 1; the output's fp16
+    operands leave 4.6e-4 and 6.0e-4 in the worst head, the state 7.6e-6 and 1.1e-5."""
+    import torch
+    if torch.cuda.mem_get_info()[1] < 160 << 30:
+        pytest.skip("needs 160 GB")
+    dt = torch.float16 if io == "f16" else torch.float32
+    g = torch.Generator(device=dev).manual_seed(hv)
+    rn = lambda *s: torch.randn(*s, device=dev, generator=g, dtype=dt)
+    q, k = (torch.nn.functional.normalize(rn(1, T, 1, D).float(), dim=-1).to(dt) for _ in range(2))
+    v = rn(1, T, hv, D)
+    gl = -torch.nn.functional.softplus(rn(1, T, hv).float())
+    beta = torch.sigmoid(rn(1, T, hv).float())
+    s = torch.zeros(1, hv, D, D, device=dev)
+    o = tsa.gdn_chunked_fwd(q, k, v, gl, beta, s)
+    s_ref = torch.zeros_like(s)
+    o_ref = tsa.gdn_recurrent_fwd(q, k, v, gl, beta, s_ref)
+    torch.cuda.synchronize()
+    worst_o = worst_s = 0.0
+    for h in range(0, hv, 8192):
+        a, b = o[0, :, h:h + 8192].float(), o_ref[0, :, h:h + 8192].float()
+        worst_o = max(worst_o, float(((a - b).norm(dim=(0, 2)) / b.norm(dim=(0, 2))).max()))
+        a, b = s[0, h:h + 8192], s_ref[0, h:h + 8192]
+        worst_s = max(worst_s, float(((a - b).norm(dim=(1, 2)) / b.norm(dim=(1, 2))).max()))
+    print(f"{io} Hv={hv} T={T}: worst head out rel {worst_o:.2e}  state rel {worst_s:.2e}")
+    assert worst_o < 2e-3 and worst_s < 1e-3
+
+
 @pytest.mark.parametrize("io", ["f16", "f32"])
 @pytest.mark.parametrize("T", [5, 6, 7, 8, 9, 15, 16, 17, 24, 33])
 def test_recurrent_token_blocks(dev, orc, T, io):

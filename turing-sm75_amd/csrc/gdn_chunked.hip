@@ -21,6 +21,7 @@
 //   (with W = T' diag(e^G) K and U = T' V formed by the prep it was 57 KiB each way: 372 MB per
 //   call at 32 heads, T = 4096, against 106 MB of inputs and outputs).
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
@@ -579,7 +580,9 @@ __device__ __forceinline__ void pin(float4_t& x) { asm volatile("" : "+v"(x)::"m
 // job: the whole sequence (kJobPlain), or the maps launch of the sequence split (segments of the
 // workgroup's unit, its start state and where its end state goes are derived below).
 // One workgroup per CU: two waves per SIMD, one of each role.
-template <typename TIO, int NC, bool kFlags>
+// kWide: V and the output are addressed in 64 bits a lane instead of by descriptors of a chunk's 64
+// rows, for rows of 2^31 / 64 bytes and more (65 536 heads in fp32, 131 072 in fp16).
+template <typename TIO, int NC, bool kFlags, bool kWide = false>
 __global__ void __launch_bounds__(kCarryThreads, 2)
 gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws, const unsigned* __restrict__ flags,
                 unsigned* __restrict__ aborts, int mode, unsigned wait_ticks, const float* state_in, float* state,
@@ -872,7 +875,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
     // last chunk), so rows past the end read as zero and their stores are dropped.  Per-lane
     // offsets are fixed.
     constexpr unsigned kE = sizeof(TIO);
-    const unsigned vrow = (unsigned)vs.t * kE;  // bytes between tokens of V
+    const unsigned vrow = (unsigned)vs.t * kE;  // bytes between tokens of V (not with kWide)
     const TIO* vh = v + b * vs.b + (long long)c0 * kC * vs.t + h * vs.h;
     const unsigned char* wsh = ws + ((size_t)bh * nch_all + c0) * ws_chunk<kF32>();
     const unsigned char* wsq = ws + (((size_t)b * Hv + hq) * nch_all + c0) * ws_chunk<kF32>();  // the QK head's rows
@@ -906,6 +909,16 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
             if (kF32) x.kl[kF32 ? j : 0] = bload4w<kFlags>(qr, kWsKlo + (unsigned)(4 * w + j) * 1024 + lane16);
         }
         x.gf = bload1w<kFlags>(rsrc_ws(wsh, ch), kWsG + 4 * (kC * w + lane));
+        if constexpr (kWide) {
+            const int t = ch * kC + 16 * w + (lane >> 2);
+            const uint4* p = reinterpret_cast<const uint4*>(vh + min(t, Tloc - 1) * vs.t + col0 + 4 * NC * (lane & 3));
+#pragma unroll
+            for (int i = 0; i < (int)(NC * kE) / 4; ++i) {
+                const uint4 y = p[i];
+                x.v[i] = ch < nch && t < Tloc ? y : make_uint4(0, 0, 0, 0);
+            }
+            return;
+        }
         const __amdgpu_buffer_rsrc_t vr = rsrc_of(vh + (long long)ch * kC * vs.t, span(ch, vrow, kD * kE));
         if constexpr (NC * kE == 2) {
             const u32x2_t y = __builtin_amdgcn_raw_buffer_load_b64(vr, voff, 0, 0);
@@ -979,11 +992,12 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
     };
 
     // Output rows: fp32 (fp32 I/O, or a map's rows in the workspace) or the caller's type.
-    const unsigned orow = obuf ? (unsigned)kD * 4 : (unsigned)Hv * kD * kE;
+    typedef typename std::conditional<kWide, size_t, unsigned>::type row_t;
+    const row_t orow = obuf ? (row_t)kD * 4 : (row_t)Hv * kD * kE;
     unsigned char* ob = obuf ? reinterpret_cast<unsigned char*>(obuf)
                              : reinterpret_cast<unsigned char*>(out + (((size_t)b * T + (size_t)c0 * kC) * Hv + h) * kD);
     const bool o32 = kF32 || obuf != nullptr;  // uniform
-    const unsigned ooff = (unsigned)(16 * w + c) * orow + (unsigned)(col0 + 4 * NC * g) * (o32 ? 4 : 2);
+    const unsigned ooff = (unsigned)(16 * w + c) * (unsigned)orow + (unsigned)(col0 + 4 * NC * g) * (o32 ? 4 : 2);
 
     // in: the next chunk's operands; o: this chunk's
     auto step = [&](In& in, Own& o, CarrySlot<TIO, NC>& cs, CarrySlot<TIO, NC>& nx, int ch) __attribute__((always_inline)) {
@@ -1033,8 +1047,27 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
             for (int r = 0; r < 4; ++r) ov[ct][r] = scale * fmaf(eq, qs[ct][r], av[r]);
             pin(ov[ct]);
         }
+        if constexpr (kWide) {
+            static_assert(NC == 2, "a lane's 8 columns are one or two 16-byte stores");
+            const int t = ch * kC + 16 * w + c;
+            if (ch < nch && t < Tloc) {
+                uint4* p = reinterpret_cast<uint4*>(ob + (size_t)t * orow + (size_t)(col0 + 4 * NC * g) * (o32 ? 4 : 2));
+                if (o32) {
+#pragma unroll
+                    for (int ct = 0; ct < NC; ++ct) p[ct] = __builtin_bit_cast(uint4, ov[ct]);
+                } else {
+                    half8_t oh;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) oh[e] = (half_t)ov[(e >> 2) & (NC - 1)][e & 3];
+                    *p = __builtin_bit_cast(uint4, oh);
+                }
+            }
+            load_a(o, ch + 2);
+            lds_barrier();
+            return;
+        }
         const __amdgpu_buffer_rsrc_t orr =
-            rsrc_of(ob + (size_t)ch * kC * orow, span(ch, orow, (unsigned)kD * (o32 ? 4 : 2)));
+            rsrc_of(ob + (size_t)ch * kC * orow, span(ch, (unsigned)orow, (unsigned)kD * (o32 ? 4 : 2)));
         if (o32) {
 #pragma unroll
             for (int ct = 0; ct < NC; ++ct)
@@ -1386,6 +1419,8 @@ hipError_t launch_chunked(const void* q, const void* k, const void* v, const flo
     unsigned* aborts = flags + (size_t)BHv * nch;
     const int nflags = BHv * nch + carry_wgs;
     const unsigned wait_ticks = carry_wait_ticks();
+    // a chunk's 64 rows of V or the output are out of a buffer descriptor's reach
+    const bool wide = std::max(st.v.t, (long long)Hv * kD) > INT_MAX / kC / (long long)sizeof(TIO);
     auto clear = [&]() {
         hipLaunchKernelGGL(gdn_flags_clear, dim3((nflags + 255) / 256), dim3(256), 0, stream, flags, nflags);
         return hipGetLastError();
@@ -1405,6 +1440,7 @@ hipError_t launch_chunked(const void* q, const void* k, const void* v, const flo
             return hipGetLastError();
         };
         if (mode != kCarryInOrder) return launch(gdn_chunk_carry<TIO, 2, true>, kAbortWgs);
+        if (wide) return launch(gdn_chunk_carry<TIO, 2, false, true>, kAbortWgs);
         // A workgroup takes a CU.  16 columns each while every workgroup then has a CU of its own,
         // else 32: a chunk step of 32 columns is ~1.25 steps of 16, and a second round costs a
         // whole one.  (us per carry, 16 / 32 columns: 32 heads, T = 4096 74 / 88; 48 heads, T = 1000
@@ -1453,7 +1489,7 @@ hipError_t launch_chunked(const void* q, const void* k, const void* v, const flo
     hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
     int dev = -1;
     SideStream* side = nullptr;
-    if (may_overlap && nch > 1 && overlap_requested() && hipStreamIsCapturing(stream, &cap) == hipSuccess &&
+    if (may_overlap && !wide && nch > 1 && overlap_requested() && hipStreamIsCapturing(stream, &cap) == hipSuccess &&
         cap == hipStreamCaptureStatusNone &&
         (stream ? hipStreamGetDevice(stream, &dev) == hipSuccess : hipGetDevice(&dev) == hipSuccess) &&
         dev >= 0 && dev < kMaxDevices) {
