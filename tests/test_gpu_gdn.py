@@ -465,6 +465,31 @@ def test_chunked_state_above_the_fp16_range(dev, orc, hv, T, nseg, io):
     assert es < TOL["chunked"][1] and eo < 1e-3
 
 
+@pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("hv,T", [(4, 1), (4, 64), (4, 200), (40, 200)])
+def test_chunked_residual_beyond_the_fp16_range(dev, orc, hv, T, io):
+    """V - e^G K S of up to ~2e5 beside a state and a Vnew that fit fp16 (small beta), in some rows
+    and columns of a chunk and not in others; all results finite and at the usual relative
+    errors (the state's largest entries are 6e4)."""
+    rng = np.random.default_rng(2300 + T + hv)
+    q, k, v, g, beta, st = _inputs(rng, 1, T, 2, hv)
+    st = np.clip(2.5e4 * rng.standard_normal(st.shape), -6e4, 6e4).astype(np.float32)
+    v = np.clip(2.5e4 * v.astype(np.float32), -6e4, 6e4).astype(np.float16)
+    beta = (0.002 + 0.008 * rng.random(beta.shape)).astype(np.float32)
+    g = (-0.002 * rng.random(g.shape)).astype(np.float32)
+    # the first token reads one column's state along its own direction: 64 < |S| / |S|_max < 128
+    st[0, 0, 7] = np.sign(k[0, 0, 0].astype(np.float32)) * 2.5e4
+    r0 = v[0, 0, 0].astype(np.float32) - np.exp(g[0, 0, 0]) * (st[0, 0] @ k[0, 0, 0].astype(np.float32))
+    assert np.abs(r0).max() > 1e5 and np.abs(r0).min() < 6e4
+    q, k, v = _as(io, q, k, v)
+    o, s = _gpu(dev, "chunked", q, k, v, g, beta, st)
+    o_ref, s_ref = orc.gdn_serial(q, k, v, g, beta, st)
+    assert np.isfinite(s).all() and np.isfinite(o).all()
+    es, eo = _rel(s, s_ref), _rel(o, o_ref)
+    print(f"{io} Hv={hv} T={T}: state rel {es:.2e}  out rel {eo:.2e}")
+    assert es < TOL["chunked"][1] and eo < 1e-3
+
+
 @pytest.mark.parametrize("io,hv,T", [("f16", 266400, 70), ("f32", 133200, 64)])
 def test_chunked_rows_past_32_bit_offsets(dev, io, hv, T):
     """Heads whose 63 token rows of V and the output lie more than 2^32 bytes apart, two chunks and

@@ -537,6 +537,11 @@ struct CarryLds {
     CarrySlot<TIO, NC> c[2];
     uint4 S[kF32 ? 2 : 1][NC][4][64];   // state operand, k-step, lane (fp32 I/O: hi, lo)
     uint4 R[2][NC][2][64];              // R hi, lo
+    uint4 Rb[2][NC][2][64];             // 2^-16 R hi, lo where |R| > kMaxHalf (written only then)
+    union {
+        unsigned char big[4];           // per chain wave: its rows of Rb hold this chunk's values
+        unsigned bigs;
+    };
     uint4 V[3][NC][2][64];              // Vnew e^{G_63 - G} hi, lo; Vnew
     int err[4];                         // per helper wave: a ready wait timed out
 };
@@ -569,6 +574,10 @@ __device__ __forceinline__ void split4(const float4_t& x, uint2& hi, uint2& lo) 
     hi = __builtin_bit_cast(uint2, h);
     lo = __builtin_bit_cast(uint2, l);
 }
+
+// R = V - e^G K S may lie beyond the fp16 range where Vnew = T' R does not (beta, a factor of T', is
+// small).  Such entries go to T' as 2^-16 R in a pair of their own, and 0 in R's place.
+constexpr float kMaxHalf = 65504.f;
 
 // Keeps the loads after it behind the products that make x.  Every reload must stay behind the
 // last use of what it replaces: with a use left below it the compiler takes other registers for
@@ -683,6 +692,26 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
                     if (kF32) put(sm.S[kF32 ? 1 : 0][ct][w], m, lo);
                 }
         };
+        auto put_r = [&](uint4 (&R)[2][NC][2][64], int ct, const float4_t& x) {
+            uint2 hi, lo;
+            split4(x, hi, lo);
+            put(R[0][ct][w >> 1], w & 1, hi);
+            put(R[1][ct][w >> 1], w & 1, lo);
+        };
+        auto put_v = [&](int ct, const float4_t& x, const float (&dg)[4]) {
+            float4_t vs;
+            half4_t vh;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                vs[r] = x[r] * dg[r];
+                vh[r] = (half_t)x[r];
+            }
+            uint2 hi, lo;
+            split4(vs, hi, lo);
+            put(sm.V[0][ct][w >> 1], w & 1, hi);
+            put(sm.V[1][ct][w >> 1], w & 1, lo);
+            put(sm.V[2][ct][w >> 1], w & 1, __builtin_bit_cast(uint2, vh));
+        };
         // step 1's operands that do not depend on the state, read ahead of the barrier before it
         half8_t kA[4], kAl[4];
         float v[NC][4], ek[4];
@@ -706,6 +735,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
             const float4 e = *reinterpret_cast<const float4*>(cs.G + kC + 16 * w + 4 * g);
             ek[0] = e.x; ek[1] = e.y; ek[2] = e.z; ek[3] = e.w;
         };
+        if (lane == 0) sm.big[w] = 0;
         auto step = [&](const CarrySlot<TIO, NC>& cs, const CarrySlot<TIO, NC>& nx) __attribute__((always_inline)) {
             // ---- 1. X = K S; R = V - e^G X ----
             half8_t Sh[NC][4], Sl[NC][4];
@@ -724,6 +754,8 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
                 tl[ks] = __builtin_bit_cast(half8_t, cs.T[(kTSlots + ts + min(ks, nks - 1)) * 64 + lane]);
             }
             __builtin_amdgcn_sched_barrier(0);
+            float4_t R[NC];
+            float m = 0.f;
 #pragma unroll
             for (int ct = 0; ct < NC; ++ct) {
                 float4_t x[2] = {};
@@ -735,13 +767,28 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
                         x[kk & 1] = mfma16(kAl[kk], Sh[ct][kk], x[kk & 1]);
                     }
                 }
-                float4_t r4;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) r4[r] = fmaf(-ek[r], x[0][r] + x[1][r], us * (kF32 ? v[ct][r] : (float)v4[ct][r]));
-                uint2 hi, lo;
-                split4(r4, hi, lo);
-                put(sm.R[0][ct][w >> 1], w & 1, hi);
-                put(sm.R[1][ct][w >> 1], w & 1, lo);
+                for (int r = 0; r < 4; ++r) R[ct][r] = fmaf(-ek[r], x[0][r] + x[1][r], us * (kF32 ? v[ct][r] : (float)v4[ct][r]));
+                put_r(sm.R, ct, R[ct]);
+                m = fmaxf(m, fmaxf(fmaxf(fabsf(R[ct][0]), fabsf(R[ct][1])), fmaxf(fabsf(R[ct][2]), fabsf(R[ct][3]))));
+            }
+            // Behind the whole step and out of line: a branch between the tiles cost 4 % of a call of
+            // 48 heads, T = 4096, this form 1.5 % (113.5 -> 115.0 us; 32 heads 89.9 -> 88.2).
+            const bool big = __builtin_amdgcn_ballot_w64(m > kMaxHalf) != 0;
+            if (__builtin_expect(big, 0)) {
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct) {
+                    float4_t y;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const bool out = fabsf(R[ct][r]) > kMaxHalf;
+                        y[r] = out ? R[ct][r] * 0x1p-16f : 0.f;
+                        if (out) R[ct][r] = 0.f;
+                    }
+                    put_r(sm.R, ct, R[ct]);
+                    put_r(sm.Rb, ct, y);
+                }
+                if (lane == 0) sm.big[w] = 1;
             }
             lds_barrier();
             // ---- 2. Vnew = T' R ----
@@ -753,6 +800,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
                     Rh[ct][ks] = __builtin_bit_cast(half8_t, sm.R[0][ct][ks][lane]);
                     Rl[ct][ks] = __builtin_bit_cast(half8_t, sm.R[1][ct][ks][lane]);
                 }
+            const unsigned bigs = sm.bigs;
             // K^T operands and factors of step 3 (and e^{G_63 - G}): under step 2
             half8_t aK[2][2], aKl[2][2];
             const float4 d4 = *reinterpret_cast<const float4*>(cs.G + 2 * kC + 16 * w + 4 * g);
@@ -769,6 +817,7 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
                 }
             __builtin_amdgcn_sched_barrier(0);
             const float dg[4] = {d4.x, d4.y, d4.z, d4.w};
+            float4_t V[NC];
 #pragma unroll
             for (int ct = 0; ct < NC; ++ct) {
                 float4_t vn[3] = {};
@@ -779,22 +828,33 @@ gdn_chunk_carry(const TIO* __restrict__ v, const unsigned char* __restrict__ ws,
                     vn[1] = mfma16(tl[ks], Rh[ct][ks], vn[1]);
                     vn[2] = mfma16(th[ks], Rl[ct][ks], vn[2]);
                 }
-                float4_t vs;
-                half4_t vh;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float x = vn[0][r] + (vn[1][r] + vn[2][r]);
-                    vs[r] = x * dg[r];
-                    vh[r] = (half_t)x;
+                for (int r = 0; r < 4; ++r) V[ct][r] = vn[0][r] + (vn[1][r] + vn[2][r]);
+                put_v(ct, V[ct], dg);
+            }
+            if (__builtin_expect(__builtin_amdgcn_readfirstlane(bigs) != 0, 0)) {
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct) {
+                    float4_t y = {};
+#pragma unroll
+                    for (int ks = 0; ks < 2; ++ks) {
+                        if (ks >= nks) break;
+                        // this lane's 8 rows of the k-step are those of wave 2 ks + g / 2
+                        const bool in = (bigs >> (8 * (2 * ks + (g >> 1)))) & 1;
+                        const half8_t h = in ? __builtin_bit_cast(half8_t, sm.Rb[0][ct][ks][lane]) : half8_t{};
+                        const half8_t l = in ? __builtin_bit_cast(half8_t, sm.Rb[1][ct][ks][lane]) : half8_t{};
+                        y = mfma16(th[ks], h, y);
+                        y = mfma16(tl[ks], h, y);
+                        y = mfma16(th[ks], l, y);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) V[ct][r] = fmaf(0x1p16f, y[r], V[ct][r]);
+                    put_v(ct, V[ct], dg);
                 }
-                uint2 hi, lo;
-                split4(vs, hi, lo);
-                put(sm.V[0][ct][w >> 1], w & 1, hi);
-                put(sm.V[1][ct][w >> 1], w & 1, lo);
-                put(sm.V[2][ct][w >> 1], w & 1, __builtin_bit_cast(uint2, vh));
             }
             lds_barrier();
             // ---- 3. S = e^{G_63} S + K^T Vs ----
+            if (__builtin_expect(big, 0) && lane == 0) sm.big[w] = 0;
             half8_t Vh[NC][2], Vl[NC][2];
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
