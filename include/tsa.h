@@ -96,7 +96,9 @@ int tsa_attn_gqa_naive(const void* q, const void* k, const void* v, const void* 
  * reference driver owns the two-pass scratch (src/gdn_sm75.cu:1341-1346); its contents on
  * entry do not matter (in order the two kernels use no ready flags; a call whose two kernels
  * run side by side, TSA_GDN_OVERLAP=1, clears them first), and calls that share one
- * ws must be ordered on one stream.  With few heads and many chunks (B*Hv <= 21, at least 16
+ * ws must be ordered on one stream.  out may be v itself; otherwise neither out nor state may
+ * lie on v, whose rows are read while others' outputs are written (this holds for every GDN
+ * entry point; the ggml adapter copies such a v first).  With few heads and many chunks (B*Hv <= 21, at least 16
  * chunks) the call splits the sequence into segments (segment state maps with their outputs
  * side by side, a combine, a parallel output fix-up) and the workspace grows by 192 KiB per
  * head and segment and 1 KiB per head and token after the first segment.  The plan, and so

@@ -607,6 +607,26 @@ def test_chunked_overlap_opt_in(dev, monkeypatch):
     assert np.array_equal(o1, o0) and np.array_equal(s1, s0)
 
 
+@pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("T,hq,hv", [(1024, 16, 32), (1500, 2, 4), (200, 8, 40)])
+@pytest.mark.parametrize("mode", ["in_order", "overlap", "overlap_wait0"])
+def test_chunked_output_over_v(dev, monkeypatch, mode, T, hq, hv, io):
+    """out = v itself: the same results bit for bit as with an output of its own, in order, with the
+    sequence split, and with the overlap asked for (a workgroup that gave up has written output
+    rows and reads V again, so such a call runs in order)."""
+    rng = np.random.default_rng(417)
+    q, k, v, g, beta, st = _inputs(rng, 1, T, hq, hv, sstd=0.02)
+    q, k, v = _as(io, q, k, v)
+    o0, s0 = _gpu(dev, "chunked", q, k, v, g, beta, st)
+    if mode != "in_order":
+        monkeypatch.setenv("TSA_GDN_OVERLAP", "1")
+    if mode == "overlap_wait0":
+        monkeypatch.setenv("TSA_GDN_CARRY_WAIT_US", "0")
+    tq, tk, tv, tg, tb, ts = _dev(dev, q, k, v, g, beta, st)
+    tsa.gdn_chunked_fwd(tq, tk, tv, tg, tb, ts, out=tv)
+    assert np.array_equal(tv.float().cpu().numpy(), o0) and np.array_equal(ts.cpu().numpy(), s0)
+
+
 def test_wrong_out_shape_raises_before_launch(dev):
     import torch
     rng = np.random.default_rng(408)

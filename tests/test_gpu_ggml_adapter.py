@@ -178,3 +178,23 @@ def test_rows_read_where_they_lie(dev, form, io, T):
     torch.cuda.synchronize()
     assert torch.equal(out.cpu(), o_ref) and torch.equal(ts_out.cpu(), s_ref)
     assert torch.equal(ts_in.cpu(), torch.from_numpy(st))
+
+
+@pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("shift", [0, 1, 40])
+@pytest.mark.parametrize("T", [1, 20, 96, 1100])
+def test_dense_output_over_v(dev, T, shift, io):
+    """A dense output on a dense v's memory, at the same place or some rows further on (every other
+    row's V is then written while it is still to be read): bit for bit the separate output."""
+    import torch
+    B, Hk, Hv = 1, 2, 4
+    q, k, v, g, beta, st = _data(np.random.default_rng(T + shift), B, T, Hk, Hv)
+    o_ref, s_ref = _direct(dev, q, k, v, g, beta, st, f32=io == "f32")
+    dt = torch.float32 if io == "f32" else torch.float16
+    buf = torch.zeros((T + shift) * Hv * D, device=dev, dtype=dt)
+    tv, out = (buf[i:i + T * Hv * D].view(B, T, Hv, D) for i in (0, shift * Hv * D))
+    tv.copy_(_t(dev, v))
+    ts = _t(dev, st)
+    tsa.ggml_gated_delta_net(_t(dev, q).to(dt), _t(dev, k).to(dt), tv, _t(dev, g), _t(dev, beta), ts, out)
+    torch.cuda.synchronize()
+    assert torch.equal(out.cpu(), o_ref) and torch.equal(ts.cpu(), s_ref)

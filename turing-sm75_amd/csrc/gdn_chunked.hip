@@ -1544,12 +1544,16 @@ hipError_t launch_chunked(const void* q, const void* k, const void* v, const flo
     // other runtime call.  The overlap (TSA_GDN_OVERLAP=1) is taken only when it cannot stall:
     // the carry's workgroups (one per CU) must leave at least half the CUs to the prep, and a
     // stream being captured into a graph runs the two kernels in order (a graph does not promise
-    // to run sibling nodes concurrently).  The side stream belongs to the device of the caller's
+    // to run sibling nodes concurrently), and so does an output that lies on v: a workgroup that
+    // gives up beside the prep has written output rows, and the second launch reads V again.  The side stream belongs to the device of the caller's
     // stream (the null stream: the current device), which need not be the current device.
     hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
     int dev = -1;
     SideStream* side = nullptr;
-    if (may_overlap && !wide && nch > 1 && overlap_requested() && hipStreamIsCapturing(stream, &cap) == hipSuccess &&
+    auto v_end = V + (B - 1) * st.v.b + (T - 1) * st.v.t + (Hv - 1) * st.v.h + kD;
+    auto O = static_cast<const TIO*>(out);
+    const bool on_v = O < v_end && V < O + (size_t)B * T * Hv * kD;
+    if (may_overlap && !wide && !on_v && nch > 1 && overlap_requested() && hipStreamIsCapturing(stream, &cap) == hipSuccess &&
         cap == hipStreamCaptureStatusNone &&
         (stream ? hipStreamGetDevice(stream, &dev) == hipSuccess : hipGetDevice(&dev) == hipSuccess) &&
         dev >= 0 && dev < kMaxDevices) {

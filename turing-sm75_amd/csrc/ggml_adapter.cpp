@@ -176,9 +176,10 @@ extern "C" int tsa_ggml_gated_delta_net(const tsa_tensor* q, const tsa_tensor* k
     // kernel's own time at a few sequences (8 sequences, 48 heads, one token: 3 x 2.4-2.8 us beside
     // its 8.2).
     // Not where the result would be written over them.
+    auto written = [&](const tsa_tensor& t) { return overlap(t, *out) || overlap(t, *state_out); };
     auto in_place = [&](const tsa_tensor& t) {
         const size_t es = f32 ? 4 : 2;
-        if (!dense(t) && (overlap(t, *out) || overlap(t, *state_out))) return false;
+        if (!dense(t) && written(t)) return false;
         if ((t.type == TSA_TYPE_F32) != f32 || t.nb[0] != es || ((uintptr_t)t.data & 15)) return false;
         for (int i = 1; i < 4; ++i)
             if (t.nb[i] % 16 || t.nb[i] > (size_t)INT64_MAX) return false;
@@ -194,16 +195,23 @@ extern "C" int tsa_ggml_gated_delta_net(const tsa_tensor* q, const tsa_tensor* k
     const tsa::GdnStrides rows{strides(*q), strides(*k), strides(*v)};
 
     // operands in the kernels' layout: used in place when already dense, else gathered
-    auto operand = [&](const tsa_tensor& t, size_t off, bool f16) -> void* {
-        if (dense(t) && (t.type == TSA_TYPE_F16) == f16) return t.data;
+    auto gather = [&](const tsa_tensor& t, size_t off, bool f16) -> void* {
         void* dst = w + off;
         if (ok()) e = tsa::copy4d(t.data, t.type == TSA_TYPE_F16, view_of(t), dst, f16 ? 1 : 0,
                                   dense_view(t.ne, f16 ? 2 : 4), st);
         return dst;
     };
+    auto operand = [&](const tsa_tensor& t, size_t off, bool f16) -> void* {
+        return dense(t) && (t.type == TSA_TYPE_F16) == f16 ? t.data : gather(t, off, f16);
+    };
     const void* qd = in_place(*q) ? q->data : operand(*q, p.q, !f32);
     const void* kd = in_place(*k) ? k->data : operand(*k, p.k, !f32);
-    const void* vd = in_place(*v) ? v->data : operand(*v, p.v, !f32);
+    // (a dense v under the result too: its rows are read beside the writing of others', which is safe
+    // only where the output is v itself)
+    const bool v_itself = dense(*out) && v->data == out->data && !overlap(*v, *state_out);
+    const void* vd = dense(*v) && written(*v) && !v_itself ? gather(*v, p.v, !f32)
+                     : in_place(*v)                        ? v->data
+                                                           : operand(*v, p.v, !f32);
     const float* gd = static_cast<const float*>(operand(*g, p.g, false));
     const float* bd = static_cast<const float*>(operand(*beta, p.beta, false));
     // the state the kernels write: state_out itself when it is dense, else scratch; they read
