@@ -272,3 +272,24 @@ def test_split_keys_dispatch(dev, B, Hq, Hkv, S, D, causal):
     err = float((o - ref).abs().max())
     print(f"B={B} {Hq}/{Hkv} S={S} D={D} causal={causal}: max-abs {err:.2e}")
     assert torch.isfinite(o).all() and err < 2e-3 * max(1.0, float(ref.abs().max()))
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [
+    # D <= 128: lengths at one key tile and around the lengths where the forms change, tiles on
+    # both sides of their rounds with and without a mask
+    (1, 6, 2, 64, 64), (1, 6, 2, 65, 64), (1, 40, 8, 191, 64), (1, 40, 8, 192, 64), (1, 64, 8, 511, 64), (1, 64, 8, 512, 64),
+    (2, 8, 8, 512, 64), (1, 66, 6, 1024, 64), (1, 3, 1, 64, 128), (1, 3, 1, 65, 128), (1, 16, 4, 511, 128), (1, 16, 4, 512, 128),
+    (1, 25, 5, 767, 128), (1, 25, 5, 768, 128), (1, 49, 7, 1000, 128),
+    # D = 256: short queries over one round of half tiles, ragged and even last tiles
+    (1, 96, 16, 300, 256), (1, 80, 8, 448, 256), (1, 80, 8, 449, 256), (1, 64, 8, 768, 256), (1, 64, 8, 769, 256),
+    (1, 104, 8, 512, 256), (1, 48, 4, 1100, 256), (1, 70, 7, 700, 256)])
+def test_split_keys_lines(dev, B, Hq, Hkv, S, D, causal):
+    """Sizes on both sides of the lines by length and mask, checked as test_split_keys_dispatch
+    checks its own; a call repeated gives the same values bit for bit."""
+    import torch
+    test_split_keys_dispatch(dev, B, Hq, Hkv, S, D, causal)
+    g = torch.Generator(device=dev).manual_seed(S + D)
+    q, k, v = (torch.randn(B, h, S, D, device=dev, generator=g).half() for h in (Hq, Hkv, Hkv))
+    o = tsa.attn_gqa_fwd(q, k, v, causal=causal)
+    assert all(torch.equal(tsa.attn_gqa_fwd(q, k, v, causal=causal), o) for _ in range(4))

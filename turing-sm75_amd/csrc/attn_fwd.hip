@@ -727,32 +727,59 @@ hipError_t launch(const half_t* q, const half_t* k, const half_t* v, const half_
                   int B, int Hq, int Hkv, int S, float scale, hipStream_t stream) {
     constexpr int kW = D == 256 ? 8 : 4;
     const int BH = B * Hq;
-    // The split-key form where whole query tiles leave the device idle, by the number of 32-row query
-    // tiles (D <= 128) or of 256-row ones (D = 256).  us per call, whole tiles / split, causal unless
-    // noted: D = 64 128 tiles 17.5 / 9.3, 512 18.5 / 10.8, 1024 18.5 / 13.9, 2000 63.8 / 53.6, 4000
-    // 91.9 / 95.4; D = 128 32 tiles 9.9 / 7.6, 252 39.9 / 26.1, 512 23.7 / 18.1, 1024 24.0 / 21.5, 1504
-    // 36.8 / 33.5, 2016 51.0 / 52.8, 4000 142 / 167; D = 256 12 tiles 58.6 / 42.6, 72 45.0 / 36.8, 144 86.6 / 64.8, 288 161 /
-    // 173.  At D = 256 a split tile moves its K and V for half the queries (10 TB/s from L2 at
-    // that rate), so without a mask's uneven tiles it pays only while its workgroups fit the CUs.
+    // The split-key forms where whole query tiles leave the device idle or end in a long tail.  The
+    // lines are by tiles (query tiles of all heads) and length, since each form's workgroups fill the
+    // device in rounds (two workgroups a CU at D <= 128, one at D = 256) and a split workgroup has the
+    // merge and a second tile's copy to pay back.  us per call, whole tiles / form:
     auto split = [&](auto kernel, int rows, int waves) {
         const int n = (S + rows - 1) / rows;
         hipLaunchKernelGGL(kernel, dim3(BH * n), dim3(64 * waves), 0, stream, q, k, v, gate, o, S, BH, n, Hq,
                            Hq / Hkv, scale * kLog2e);
         return hipGetLastError();
     };
+    auto tiles = [&](int rows) { return (long long)BH * ((S + rows - 1) / rows); };
     if constexpr (D == 256) {
-        const long long tiles = (long long)BH * ((S + 255) / 256), half = (long long)BH * ((S + 127) / 128);
-        if (S > 128 && (kCausal ? tiles <= 192 : half <= 256))
+        // 128 rows by two key groups.  Without a mask while its workgroups fit the CUs (96 tiles of
+        // S = 2048 100 / 68, 144 of S = 1500 81 / 107): it moves K and V for half the queries, 10 TB/s from
+        // L2 at that rate.
+        // With one, up to 192 whole tiles (72 tiles 45.0 / 36.8, 192 104.8 / 83.9; 216 118 / 121), where
+        // more than one round of it needs queries long enough for the mask's tail to weigh: 192 tiles
+        // of S = 300 24.9 / 31.1, 512 36.0 / 38.6, 1000 55.5 / 49.3; 160 tiles of S = 400 29.2 / 33.3, 500 34.9
+        // / 35.2, 640 36.5 / 34.0; 144 of S = 500 34.8 / 32.2.
+        const long long whole = tiles(256), half = tiles(128);
+        const bool fits = half <= 256 || (kCausal && whole <= (S > 768 ? 192 : S > 448 ? 160 : 0));
+        if (S > 128 && whole <= 192 && fits)
             return split(attn_ksplit_kernel<D, kCausal, 4, 2, 32>, 128, 8);
         // Somewhat more tiles than CUs leave a second round nearly empty: half tiles, two workgroups
         // per CU, 32-key steps and no split there (the same keys in the same order, so the same
-        // values; us, whole / half tiles, causal 216 tiles 119 / 106, 256 194 / 182, 264 137 / 126, 288
-        // 157.4 / 159.2; no mask 264 289 / 180, 288 337 / 319; from 384 on within 4 % either way).
-        if (tiles > 192 && tiles <= (kCausal ? 272 : 320)) return split(attn_ksplit_kernel<D, kCausal, 4, 1, 32>, 128, 4);
-    } else {
-        const long long tiles = (long long)BH * ((S + 31) / 32);
-        if (tiles <= (D == 64 ? 512 : 256)) return split(attn_ksplit_kernel<D, kCausal, 1, 4, 32>, 32, 4);
-        if (tiles <= (D == 64 ? 2048 : 1792)) return split(attn_ksplit_kernel<D, kCausal, 2, 2, D == 64 ? 64 : 32>, 64, 4);
+        // values).  Causal 216 tiles 119 / 106, 264 137 / 126, 288 157.4 / 159.2; no mask 264 289 / 180,
+        // 288 337 / 319; from 384 on within 4 % either way.  Without a mask 193 to 256 whole tiles are one
+        // even round, and half tiles gain what they leave out of a ragged last one (S = 1100, 240
+        // tiles 75.6 / 71.7; 300 30.6 / 26.3) or at short lengths (512 43.2 / 41.9), and else lose (S = 700,
+        // 255 tiles 59.3 / 65.8; 2048, 256 133.6 / 135.6; 2300, 216 142 / 146).
+        const bool ragged = half < 2 * whole && S <= 2048;
+        if (whole > 192 && whole <= (kCausal ? 272 : 320) && (kCausal || whole > 256 || S <= 512 || ragged))
+            return split(attn_ksplit_kernel<D, kCausal, 4, 1, 32>, 128, 4);
+    } else if (S > 64) {  // (one key tile has nothing to split: 128 heads of S = 64 4.2 / 5.2, D = 128 5.4 / 8.2)
+        // 32 rows by four key groups in its first round (D = 128: first workgroup per CU) at lengths
+        // that pay the merge: D = 64, causal, 512 tiles of S = 256 7.9 / 6.6 against 6.2 of the next
+        // form, 384 9.4 / 7.0 against 7.3, 1024 17.6 / 10.7; D = 128 256 tiles of S = 256 10.3 / 9.5
+        // against 8.6, 512 14.6 / 11.8, 1024 23.0 / 16.9.
+        const long long t32 = tiles(32), t64 = tiles(64);
+        if (D == 64 ? S >= 192 && t32 <= (S >= 384 ? 512 : 256) : S >= 512 && t32 <= 256)
+            return split(attn_ksplit_kernel<D, kCausal, 1, 4, 32>, 32, 4);
+        // 64 rows by two key groups.  Under a mask its first round of 512, and past it the more the
+        // longer the tail of whole tiles is: D = 64 512 tiles of S = 256 8.1 / 7.2, 640 8.7 / 10.6, 768 of
+        // S = 512 12.1 / 13.7, of S = 1024 18.6 / 17.8, 1024 of S = 1024 20.1 / 20.8, of S = 2048 33.8 / 32.2,
+        // 1280 39.5 / 42.6; D = 128 640 of S = 256 13.1 / 15.2, 768 of S = 1024 27.9 / 27.1, 896 of S = 2048
+        // 49.8 / 47.5, 1024 49.6 / 50.6.  Without one the tiles are even and the split's only gain is
+        // the idle half of the device: D = 64 512 tiles of S = 512 10.2 / 8.4, 1024 17.6 / 15.7, but 384 of
+        // S = 128 5.5 / 6.0, and past 512 640 of S = 1024 20.8 / 26.2; D = 128 384 tiles of S = 2048 41.8 /
+        // 38.9, but 512 of S = 512 16.1 / 17.3 and 384 of S = 256 10.2 / 11.0.
+        const int lim = kCausal   ? min(D == 64 ? 1024 : 896, 512 + max(0, S - 512) / 2)
+                        : D == 64 ? (S >= 512 ? 512 : 256)
+                                  : (S >= 768 ? 384 : 256);
+        if (t64 <= lim) return split(attn_ksplit_kernel<D, kCausal, 2, 2, D == 64 ? 64 : 32>, 64, 4);
     }
     const int n_qt = (S + 32 * kW - 1) / (32 * kW);
     hipLaunchKernelGGL((attn_fwd_kernel<D, kCausal, kW>), dim3(BH * n_qt), dim3(64 * kW), 0,
