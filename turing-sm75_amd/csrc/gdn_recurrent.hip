@@ -57,12 +57,49 @@ __device__ __forceinline__ void load_row16(const TIO* __restrict__ p, int j, flo
     }
 }
 
-template <typename TIO>
+// Where the rows of q, k and v and the entering state lie: in the dense layouts with the state in
+// place, or anywhere.  Types of their own, since a kernel's start waits for its arguments: with the
+// strides passed and multiplied in dense calls too, those of a few tokens took 0.2 to 0.5 us more
+// (fp16, T = 8, one head 4.8 -> 5.2 us, 48 heads 5.4 -> 5.7).
+struct Dense {
+    template <typename T>
+    __device__ __forceinline__ const T* q(const T* x, int, size_t bt, int, int hq, int Hq) const {
+        return x + (bt * Hq + hq) * kD;
+    }
+    template <typename T>
+    __device__ __forceinline__ const T* k(const T* x, int, size_t bt, int, int hq, int Hq) const {
+        return x + (bt * Hq + hq) * kD;
+    }
+    template <typename T>
+    __device__ __forceinline__ const T* v(const T* x, int, size_t bt, int, int h, int Hv) const {
+        return x + (bt * Hv + h) * kD;
+    }
+    __device__ __forceinline__ const float* state(const float* s) const { return s; }
+};
+struct Anywhere {
+    GdnStrides st;
+    const float* state_in;
+    template <typename T>
+    __device__ __forceinline__ const T* q(const T* x, int b, size_t, int t, int hq, int) const {
+        return x + b * st.q.b + t * st.q.t + hq * st.q.h;
+    }
+    template <typename T>
+    __device__ __forceinline__ const T* k(const T* x, int b, size_t, int t, int hq, int) const {
+        return x + b * st.k.b + t * st.k.t + hq * st.k.h;
+    }
+    template <typename T>
+    __device__ __forceinline__ const T* v(const T* x, int b, size_t, int t, int h, int) const {
+        return x + b * st.v.b + t * st.v.t + h * st.v.h;
+    }
+    __device__ __forceinline__ const float* state(const float*) const { return state_in; }
+};
+
+template <typename TIO, typename At>
 __global__ void __launch_bounds__(kThreads)
 gdn_recurrent_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
                      const TIO* __restrict__ v, const float* __restrict__ g_log,
-                     const float* __restrict__ beta, const float* state_in, float* state,
-                     TIO* __restrict__ out, int T, int Hq, int Hv, float scale, GdnStrides st) {
+                     const float* __restrict__ beta, float* state,
+                     TIO* __restrict__ out, int T, int Hq, int Hv, float scale, At at) {
     const int bh = blockIdx.x / kBlocksPerHead;
     const int cb = blockIdx.x % kBlocksPerHead;
     const int b = bh / Hv, h = bh % Hv, hq = h % Hq;
@@ -70,7 +107,7 @@ gdn_recurrent_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     const int col = cb * kColsPerBlock + (tid >> 3);
     const int j = tid & 7;
 
-    const float4_t* Si = reinterpret_cast<const float4_t*>(state_in + ((size_t)bh * kD + col) * kD);
+    const float4_t* Si = reinterpret_cast<const float4_t*>(at.state(state) + ((size_t)bh * kD + col) * kD);
     float4_t* Sc = reinterpret_cast<float4_t*>(state + ((size_t)bh * kD + col) * kD);
     float4_t s[4];
 #pragma unroll
@@ -79,11 +116,11 @@ gdn_recurrent_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     for (int t = 0; t < T; ++t) {
         const size_t bt = (size_t)b * T + t;
         float kr[16], qr[16];
-        load_row16(k + b * st.k.b + t * st.k.t + hq * st.k.h, j, kr);
-        load_row16(q + b * st.q.b + t * st.q.t + hq * st.q.h, j, qr);
+        load_row16(at.k(k, b, bt, t, hq, Hq), j, kr);
+        load_row16(at.q(q, b, bt, t, hq, Hq), j, qr);
         const float gl = g_log[bt * Hv + h];
         const float be = beta[bt * Hv + h];
-        const float vc = (float)v[b * st.v.b + t * st.v.t + h * st.v.h + col];
+        const float vc = (float)at.v(v, b, bt, t, h, Hv)[col];
         float kv = 0.f, sq = 0.f, kq = 0.f;
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
@@ -127,12 +164,12 @@ gdn_recurrent_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
 // at 256 heads.
 constexpr int kStagedMinT = 6;
 constexpr int kTB = 8;  // tokens per block: 32 threads of 4 elements load one token's row
-template <typename TIO>
+template <typename TIO, typename At>
 __global__ void __launch_bounds__(kThreads)
 gdn_serial_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
                   const TIO* __restrict__ v, const float* __restrict__ g_log,
-                  const float* __restrict__ beta, const float* state_in, float* state,
-                  TIO* __restrict__ out, int T, int Hq, int Hv, float scale, GdnStrides st) {
+                  const float* __restrict__ beta, float* state,
+                  TIO* __restrict__ out, int T, int Hq, int Hv, float scale, At at) {
     struct Block {
         float4_t k[kTB][kD / 4], q[kTB][kD / 4];
         float v[kTB][kColsPerBlock], g[kTB], be[kTB];
@@ -145,7 +182,7 @@ gdn_serial_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     const int cl = tid >> 3, col = cb * kColsPerBlock + cl;
     const int j = tid & 7;
 
-    const float4_t* Si = reinterpret_cast<const float4_t*>(state_in + ((size_t)bh * kD + col) * kD);
+    const float4_t* Si = reinterpret_cast<const float4_t*>(at.state(state) + ((size_t)bh * kD + col) * kD);
     float4_t* Sc = reinterpret_cast<float4_t*>(state + ((size_t)bh * kD + col) * kD);
     float4_t s[4];
 #pragma unroll
@@ -161,9 +198,9 @@ gdn_serial_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     auto load = [&](Share& x, int t0) {
         const int t = min(t0 + lt, T - 1);
         const size_t bt = (size_t)b * T + t;
-        x.k = load4(k + b * st.k.b + t * st.k.t + hq * st.k.h + 4 * le);
-        x.q = load4(q + b * st.q.b + t * st.q.t + hq * st.q.h + 4 * le);
-        x.v = (float)v[b * st.v.b + t * st.v.t + h * st.v.h + cb * kColsPerBlock + le];
+        x.k = load4(at.k(k, b, bt, t, hq, Hq) + 4 * le);
+        x.q = load4(at.q(q, b, bt, t, hq, Hq) + 4 * le);
+        x.v = (float)at.v(v, b, bt, t, h, Hv)[cb * kColsPerBlock + le];
         x.g = g_log[bt * Hv + h];
         x.be = beta[bt * Hv + h];
     };
@@ -255,12 +292,12 @@ __device__ __forceinline__ float sum_lanes(float x) {
 // nothing.  kFused: q / k are raw rows, normalised here (their norms come from the same
 // lane-group sums as the dot products), and g_log / beta come from the raw projections
 // a / b (gate arguments).
-template <int kCols, int kLpc, bool kFused, typename TIO>
+template <int kCols, int kLpc, bool kFused, typename TIO, typename At>
 __global__ void __launch_bounds__(kLpc * kCols)
 gdn_decode_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
                   const TIO* __restrict__ v, const float* __restrict__ g_log,
-                  const float* __restrict__ beta, GdnRawGates gates, const float* state_in, float* state,
-                  TIO* __restrict__ out, int Hq, int Hv, float scale, GdnStrides st) {
+                  const float* __restrict__ beta, GdnRawGates gates, float* state,
+                  TIO* __restrict__ out, int Hq, int Hv, float scale, At at) {
     static_assert(kLpc * kCols >= 64, "wave 0 loads the q / k rows");
     constexpr int kWgPerHead = kD / kCols;
     constexpr int kR = 32 / kLpc;  // float4 chunks of the column per lane
@@ -273,7 +310,7 @@ gdn_decode_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
 
     typedef typename std::conditional<std::is_same<TIO, float>::value, float4_t, half4_t>::type row4_t;
     __shared__ row4_t kq_rows[2][kD / 4];
-    const float4_t* Si = reinterpret_cast<const float4_t*>(state_in + ((size_t)bh * kD + col) * kD);
+    const float4_t* Si = reinterpret_cast<const float4_t*>(at.state(state) + ((size_t)bh * kD + col) * kD);
     float4_t* Sc = reinterpret_cast<float4_t*>(state + ((size_t)bh * kD + col) * kD);
     float4_t s[kR];
 #pragma unroll
@@ -286,10 +323,10 @@ gdn_decode_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0); expcnt, lgkmcnt left at their maxima
     __builtin_amdgcn_sched_barrier(0);
     if (tid < 64) {  // wave 0 -- lanes 0-31: k row, 32-63: q row, 4 elements each
-        const TIO* row = tid < 32 ? k + b * st.k.b + hq * st.k.h : q + b * st.q.b + hq * st.q.h;
+        const TIO* row = tid < 32 ? at.k(k, b, bt, 0, hq, Hq) : at.q(q, b, bt, 0, hq, Hq);
         kq_rows[tid >> 5][tid & 31] = *reinterpret_cast<const row4_t*>(row + 4 * (tid & 31));
     }
-    const float vc = (float)v[b * st.v.b + h * st.v.h + col];
+    const float vc = (float)at.v(v, b, bt, 0, h, Hv)[col];
     float g, be;
     if (kFused) {
         g = __expf(gdn_softplus(gates.a[bt * Hv + h] + gates.dt_bias[h]) * gates.A[h]);
@@ -381,9 +418,9 @@ gdn_naive_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
     }
 }
 
-template <typename TIO>
-hipError_t launch_recurrent(const void* q, const void* k, const void* v, const GdnStrides& st,
-                            const float* g_log, const float* beta, const float* state_in, float* state,
+template <typename TIO, typename At>
+hipError_t launch_recurrent(const void* q, const void* k, const void* v, const At& at,
+                            const float* g_log, const float* beta, float* state,
                             void* out, int B, int T, int Hq, int Hv, float scale, hipStream_t stream) {
     auto Q = static_cast<const TIO*>(q);
     auto K = static_cast<const TIO*>(k);
@@ -391,9 +428,9 @@ hipError_t launch_recurrent(const void* q, const void* k, const void* v, const G
     auto O = static_cast<TIO*>(out);
     if (T == 1) {
         const unsigned blocks = (unsigned)(B * Hv * (kD / kDecodeCols));
-        hipLaunchKernelGGL((gdn_decode_kernel<kDecodeCols, kDecodeLpc, false, TIO>), dim3(blocks),
+        hipLaunchKernelGGL((gdn_decode_kernel<kDecodeCols, kDecodeLpc, false, TIO, At>), dim3(blocks),
                            dim3(kDecodeLpc * kDecodeCols), 0, stream, Q, K, V, g_log, beta,
-                           GdnRawGates{}, state_in, state, O, Hq, Hv, scale, st);
+                           GdnRawGates{}, state, O, Hq, Hv, scale, at);
         return hipGetLastError();
     }
     const unsigned blocks = (unsigned)(B * Hv * kBlocksPerHead);
@@ -401,12 +438,12 @@ hipError_t launch_recurrent(const void* q, const void* k, const void* v, const G
     // heads, fp32 I/O, T = 2 3.3 / 4.3, 4 4.3 / 4.7, 6 5.5 / 5.3, 8 6.6 / 5.7, 31 20.0 / 11.8; four
     // sequences, fp16, T = 4 7.6 / 8.1, 6 9.3 / 8.9, 8 11.1 / 9.9, 31 33.3 / 21.8).
     if (T >= kStagedMinT) {
-        hipLaunchKernelGGL(gdn_serial_kernel<TIO>, dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
-                           g_log, beta, state_in, state, O, T, Hq, Hv, scale, st);
+        hipLaunchKernelGGL((gdn_serial_kernel<TIO, At>), dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
+                           g_log, beta, state, O, T, Hq, Hv, scale, at);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(gdn_recurrent_kernel<TIO>, dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
-                       g_log, beta, state_in, state, O, T, Hq, Hv, scale, st);
+    hipLaunchKernelGGL((gdn_recurrent_kernel<TIO, At>), dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
+                       g_log, beta, state, O, T, Hq, Hv, scale, at);
     return hipGetLastError();
 }
 
@@ -428,26 +465,33 @@ hipError_t launch_naive(const void* q, const void* k, const void* v, const float
 hipError_t gdn_recurrent(const void* q, const void* k, const void* v, const float* g_log,
                          const float* beta, float* state, void* out, int B, int T, int Hq,
                          int Hv, float scale, bool f32, hipStream_t stream) {
-    return gdn_recurrent_strided(q, k, v, gdn_dense(T, Hq, Hv), g_log, beta, state, state, out, B, T, Hq, Hv, scale,
-                                 f32, stream);
+    return f32 ? launch_recurrent<float>(q, k, v, Dense{}, g_log, beta, state, out, B, T, Hq, Hv, scale, stream)
+               : launch_recurrent<half_t>(q, k, v, Dense{}, g_log, beta, state, out, B, T, Hq, Hv, scale, stream);
 }
 
 hipError_t gdn_recurrent_strided(const void* q, const void* k, const void* v, const GdnStrides& st,
                                  const float* g_log, const float* beta, const float* state_in, float* state,
                                  void* out, int B, int T, int Hq, int Hv, float scale, bool f32,
                                  hipStream_t stream) {
-    return f32 ? launch_recurrent<float>(q, k, v, st, g_log, beta, state_in, state, out, B, T, Hq, Hv, scale, stream)
-               : launch_recurrent<half_t>(q, k, v, st, g_log, beta, state_in, state, out, B, T, Hq, Hv, scale, stream);
+    const GdnStrides d = gdn_dense(T, Hq, Hv);
+    auto same = [&](const RowStride& a, const RowStride& b, int H) {  // in the dimensions there are
+        return (a.b == b.b || B == 1) && (a.t == b.t || T == 1) && (a.h == b.h || H == 1);
+    };
+    if (state_in == state && same(st.q, d.q, Hq) && same(st.k, d.k, Hq) && same(st.v, d.v, Hv))
+        return gdn_recurrent(q, k, v, g_log, beta, state, out, B, T, Hq, Hv, scale, f32, stream);
+    const Anywhere at{st, state_in};
+    return f32 ? launch_recurrent<float>(q, k, v, at, g_log, beta, state, out, B, T, Hq, Hv, scale, stream)
+               : launch_recurrent<half_t>(q, k, v, at, g_log, beta, state, out, B, T, Hq, Hv, scale, stream);
 }
 
 hipError_t gdn_decode_fused(const void* q, const void* k, const void* v, const GdnRawGates& gates,
                             float* state, void* out, int B, int Hq, int Hv, float scale,
                             hipStream_t stream) {
     const unsigned blocks = (unsigned)(B * Hv * (kD / kDecodeCols));
-    hipLaunchKernelGGL((gdn_decode_kernel<kDecodeCols, kDecodeLpc, true, half_t>), dim3(blocks),
+    hipLaunchKernelGGL((gdn_decode_kernel<kDecodeCols, kDecodeLpc, true, half_t, Dense>), dim3(blocks),
                        dim3(kDecodeLpc * kDecodeCols), 0, stream, static_cast<const half_t*>(q),
                        static_cast<const half_t*>(k), static_cast<const half_t*>(v), nullptr, nullptr,
-                       gates, state, state, static_cast<half_t*>(out), Hq, Hv, scale, gdn_dense(1, Hq, Hv));
+                       gates, state, static_cast<half_t*>(out), Hq, Hv, scale, Dense{});
     return hipGetLastError();
 }
 
