@@ -524,7 +524,7 @@ def test_chunked_rows_past_32_bit_offsets(dev, io, hv, T):
 @pytest.mark.parametrize("io", ["f16", "f32"])
 @pytest.mark.parametrize("T", [5, 6, 7, 8, 9, 15, 16, 17, 24, 33])
 def test_recurrent_token_blocks(dev, orc, T, io):
-    """The token-serial kernel's two forms around their line (6 tokens) and at the remainders of
+    """The token-serial kernel's two forms around their lines and at the remainders of
     the staged form's blocks of 8: bit for bit T decode steps, whose lanes and sums both share."""
     import torch
     rng = np.random.default_rng(700 + T)
@@ -536,6 +536,21 @@ def test_recurrent_token_blocks(dev, orc, T, io):
     steps = [tsa.gdn_decode_step(*(x[:, t].contiguous() for x in (tq, tk, tv, tg, tb)), ts) for t in range(T)]
     assert np.array_equal(torch.stack(steps, 1).float().cpu().numpy(), o) and np.array_equal(ts.cpu().numpy(), s)
     _check(o, s, *orc.gdn_serial(q, k, v, g, beta, st), *TOL["recurrent"], label=f"recurrent {io} T={T}")
+
+
+@pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("hv,T", [(2, 8), (2, 9), (2, 10), (9, 6), (64, 9), (64, 10), (65, 6), (65, 7), (65, 16)])
+def test_recurrent_forms_by_heads(dev, hv, T, io):
+    """The lines between the token-serial kernel's two forms by type and heads: bit for bit T decode
+    steps on either side."""
+    import torch
+    rng = np.random.default_rng(900 + T + hv)
+    arrays = _inputs(rng, 1, T, 2, hv, sstd=0.02)
+    q, k, v = _as(io, *arrays[:3])
+    o, s = _gpu(dev, "recurrent", q, k, v, *arrays[3:])
+    tq, tk, tv, tg, tb, ts = _dev(dev, q, k, v, *arrays[3:])
+    steps = [tsa.gdn_decode_step(*(x[:, t].contiguous() for x in (tq, tk, tv, tg, tb)), ts) for t in range(T)]
+    assert np.array_equal(torch.stack(steps, 1).float().cpu().numpy(), o) and np.array_equal(ts.cpu().numpy(), s)
 
 
 def _ws_fill(ws, kind):

@@ -14,8 +14,8 @@
 //   * the state is read and written with nontemporal loads/stores: it is touched once
 //     per launch, and keeping it out of the caches measured 4.6 -> 5.6 TB/s for the
 //     in-place read-modify-write stream of a 16 x 32 head decode step;
-//   * T > 1: a 256-thread workgroup owns 32 columns of one (b, h) for all T tokens (from 6 tokens
-//     on with the tokens staged through LDS, gdn_serial_kernel);
+//   * T > 1: a 256-thread workgroup owns 32 columns of one (b, h) for all T tokens (from 6
+//     to 10 tokens on with the tokens staged through LDS, gdn_serial_kernel);
 //     decode (T = 1): a one-wave workgroup owns 8 columns, so a decode step of 16 x 32
 //     heads is 8192 independent workgroups.
 // The reference's token-serial family (serial/smem/occ/occ2/occ4/occ4p/occ8,
@@ -162,7 +162,6 @@ gdn_recurrent_kernel(const TIO* __restrict__ q, const TIO* __restrict__ k,
 // fp32 I/O (T = 512: 299 -> 139 us).  Unrolled without the end-of-sequence test per token (LDS
 // reads of the next token ahead, 130 registers) it measured 136 us there and 339 instead of 314
 // at 256 heads.
-constexpr int kStagedMinT = 6;
 constexpr int kTB = 8;  // tokens per block: 32 threads of 4 elements load one token's row
 template <typename TIO, typename At>
 __global__ void __launch_bounds__(kThreads)
@@ -434,10 +433,15 @@ hipError_t launch_recurrent(const void* q, const void* k, const void* v, const A
         return hipGetLastError();
     }
     const unsigned blocks = (unsigned)(B * Hv * kBlocksPerHead);
-    // From 6 tokens on the staged form, below it the direct one (us per call, direct / staged: 48
-    // heads, fp32 I/O, T = 2 3.3 / 4.3, 4 4.3 / 4.7, 6 5.5 / 5.3, 8 6.6 / 5.7, 31 20.0 / 11.8; four
-    // sequences, fp16, T = 4 7.6 / 8.1, 6 9.3 / 8.9, 8 11.1 / 9.9, 31 33.3 / 21.8).
-    if (T >= kStagedMinT) {
+    // The staged form from the number of tokens on that pays its first block: fewer with fp32 rows
+    // (the direct form's loads are twice as wide) and with more than a workgroup per CU, more with a
+    // few heads, whose rows stay in one XCD's L2.  us per call, direct / staged: fp16, 1 head T = 9 5.2 /
+    // 5.2, 10 5.6 / 5.5; 48 heads 6 4.7 / 5.3, 8 5.5 / 5.7, 10 6.2 / 6.2, 12 6.9 / 6.5; 96 heads 6 6.3 / 6.4, 7 6.9 /
+    // 6.7; 384 heads 6 14.0 / 12.3.  fp32, 4 heads 6 4.5 / 4.8, 8 5.1 / 5.2, 9 5.5 / 5.4; 16 heads 5 4.6 / 4.7, 6
+    // 5.2 / 4.9; 48 heads 6 5.4 / 5.2, 8 6.5 / 5.7, 31 20.0 / 11.8; 192 heads 5 7.5 / 7.6, 6 8.3 / 8.0.
+    constexpr bool kF32 = std::is_same<TIO, float>::value;
+    const int staged_min_t = kF32 ? (blocks <= 32 ? 9 : 6) : (blocks <= 256 ? 10 : 7);
+    if (T >= staged_min_t) {
         hipLaunchKernelGGL((gdn_serial_kernel<TIO, At>), dim3(blocks), dim3(kThreads), 0, stream, Q, K, V,
                            g_log, beta, state, O, T, Hq, Hv, scale, at);
         return hipGetLastError();
