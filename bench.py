@@ -90,9 +90,9 @@ def attn_flops(B, H, S, D, causal, **_):
 
 def prefill_flops(B, T, Hq, Hv, d, chunk, **_):
     # per (head, chunk), full (not triangle-halved) products:
-    # K K^T, Q K^T, Tm K, Tm V, (M.QK^T) Vnew, W S, Q S, K^T Vnew
+    # K K^T, Q K^T, T' (V - e^G K S), (M.QK^T) Vnew, K S, Q S, K^T Vnew
     nch = math.ceil(T / chunk)
-    per = 2 * chunk * (chunk * (3 * d + 2 * d) + 3 * d * d)
+    per = 2 * chunk * (chunk * 4 * d + 3 * d * d)
     return float(B * Hv * nch * per)
 
 
