@@ -98,7 +98,10 @@ int tsa_attn_gqa_naive(const void* q, const void* k, const void* v, const void* 
  * run side by side, TSA_GDN_OVERLAP=1, clears them first), and calls that share one
  * ws must be ordered on one stream.  out may be v itself; otherwise neither out nor state may
  * lie on v, whose rows are read while others' outputs are written (this holds for every GDN
- * entry point; the ggml adapter copies such a v first).  With few heads and many chunks (B*Hv <= 21, at least 16
+ * entry point; the ggml adapter copies such a v first).  q, k, v, the state entering a chunk and
+ * Vnew = (I + A)^-1 diag(beta) (V - e^G K S) are fp16 MFMA operands (single or hi + lo): beyond
+ * 65504 they are infinite there, as outputs of fp16 I/O are; V - e^G K S and the final state may
+ * be larger.  With few heads and many chunks (B*Hv <= 21, at least 16
  * chunks) the call splits the sequence into segments (segment state maps with their outputs
  * side by side, a combine, a parallel output fix-up) and the workspace grows by 192 KiB per
  * head and segment and 1 KiB per head and token after the first segment.  The plan, and so
@@ -114,8 +117,8 @@ int tsa_gdn_chunked_fwd(const void* q, const void* k, const void* v, const float
 /* The same prefill with fp32 q, k, v, out (the reference's GDN kernels and gdn_cpu take fp32,
  * src/gdn_sm75.cu:57-64,1078-1106): the inputs are converted to the fp16 MFMA operands in
  * registers, never narrowed in memory, and the output is stored in fp32.  Its workspace is
- * larger (the prep leaves fp16 copies of each chunk's K and Q rows there for the state
- * carry): tsa_gdn_chunked_workspace_bytes_f32(...). */
+ * larger (the prep leaves K's low halves there beside the fp16 copies of each chunk's K and Q
+ * rows that it leaves in either form): tsa_gdn_chunked_workspace_bytes_f32(...). */
 size_t tsa_gdn_chunked_workspace_bytes_f32(int B, int T, int Hq, int Hv, int dk, int dv,
                                            int chunk);
 int tsa_gdn_chunked_fwd_f32(const float* q, const float* k, const float* v, const float* g_log,

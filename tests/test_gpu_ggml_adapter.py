@@ -95,8 +95,8 @@ def test_fp32_views_of_a_fused_projection(dev, T):
     assert torch.equal(ts_out.cpu(), s_ref)
     # on fp16-exact inputs the decode and token-serial fp32 paths (T < 32) carry the fp16 path's
     # state bit for bit (their outputs may differ in the last rounding, tests/test_gpu_gdn.py
-    # covers that); the chunked fp32 path takes its W S state operand and W's A operand as
-    # fp16 hi + lo pairs, so its state agrees with the fp16 path's to the latter's rounding
+    # covers that); the chunked fp32 path takes the state operand of K S as an fp16
+    # hi + lo pair, so its state agrees with the fp16 path's to the latter's rounding
     if T < 32:
         assert torch.equal(s_ref, s16)
     else:

@@ -9,8 +9,14 @@ Budgets (per kernel: registers = VGPRs + AGPRs of one wave; waves per SIMD; LDS 
   attn_fwd_kernel<128>          2 waves / SIMD,  64 KiB LDS
   attn_fwd_kernel<256>          2 waves / SIMD, 128 KiB LDS (8-wave workgroups, one per CU)
   gdn_chunk_prep (fp16 I/O)     4 workgroups / CU: 128 registers, 40 KiB LDS
-  gdn_chunk_prep (fp32 I/O)     3 workgroups / CU (the V_lo tile: 53.25 KiB of LDS)
+  attn_ksplit_kernel<64>        two 4-wave workgroups / CU: 2 waves / SIMD, 80 KiB LDS
+  attn_ksplit_kernel<128, 2, 2> two 4-wave workgroups / CU: 2 waves / SIMD, 80 KiB LDS
+  attn_ksplit_kernel<128, 1, 4> one 4-wave workgroup / CU (128-key tiles, 128 KiB of K and V)
+  attn_ksplit_kernel<256, 4, 2> one 8-wave workgroup / CU: 2 waves / SIMD
+  attn_ksplit_kernel<256, 4, 1> two 4-wave workgroups / CU: 2 waves / SIMD, 80 KiB LDS
+  gdn_chunk_prep (fp32 I/O)     3 workgroups / CU (K's low halves: 49 KiB of LDS)
   gdn_chunk_carry               one 8-wave workgroup per CU: 2 waves / SIMD, up to 160 KiB LDS
+  gdn_serial_kernel             4 waves / SIMD, 20 KiB LDS (8 workgroups / CU)
   gdn_decode_kernel, gdn_recurrent_kernel, the pre/post-op passes: 8 waves / SIMD
   and no kernel on the product path spills (scratch 0).  The naive check kernels are exempt
   from the spill rule: they are the drivers' correctness references, not hot paths.
@@ -33,11 +39,17 @@ BUDGETS = [
     (r"attn_fwd_kernelILi64E", 4, 128, 32 << 10),
     (r"attn_fwd_kernelILi128E", 2, 256, 64 << 10),
     (r"attn_fwd_kernelILi256E", 2, 256, 128 << 10),
+    (r"attn_ksplit_kernelILi64E", 2, 256, 80 << 10),
+    (r"attn_ksplit_kernelILi128ELb[01]ELi2ELi2E", 2, 256, 80 << 10),
+    (r"attn_ksplit_kernelILi128ELb[01]ELi1ELi4E", 1, 256, 160 << 10),
+    (r"attn_ksplit_kernelILi256ELb[01]ELi4ELi2E", 2, 256, 160 << 10),
+    (r"attn_ksplit_kernelILi256ELb[01]ELi4ELi1E", 2, 256, 80 << 10),
     (r"gdn_chunk_prepILb[01]EDF16_E", 4, 128, 40 << 10),
     (r"gdn_chunk_prepILb0EfE", 3, 168, (160 << 10) // 3),
     (r"gdn_chunk_carry", 2, 256, 160 << 10),
     (r"gdn_decode_kernel", 8, 64, 4 << 10),
     (r"gdn_recurrent_kernel", 8, 64, 4 << 10),
+    (r"gdn_serial_kernel", 4, 128, 20 << 10),
     (r"gated_rmsnorm_kernel", 8, 64, 0),
     (r"l2norm_rows_kernel", 8, 64, 0),
     (r"gdn_gates_kernel", 8, 64, 0),

@@ -100,11 +100,11 @@ constexpr int kCarryBeside = 1;   // beside the prep: a timed-out workgroup abor
 constexpr int kCarryRetry = 2;    // after the prep: only the first launch's aborted workgroups run
 
 // Sequence split (few heads, many chunks): T is cut into nseg segments of seg_len chunks (the
-// last takes the rest).  The state update is linear in the state and in U, so the state
+// last takes the rest).  The state update is linear in the state and in V, so the state
 // after a segment is an affine map of the state E entering it, S_out = Phi E + Z, where Z is
-// the segment's chain run from S = 0 and Phi its chain run from S = I with U = 0; and a
+// the segment's chain run from S = 0 and Phi its chain run from S = I with V = 0; and a
 // chunk's output, O = A S + B, is then O = O_Z + M E, where O_Z is the output of the Z chain
-// and M = A Phi_<c the output of the Phi chain (U = 0 makes B vanish).  Three launches after
+// and M = A Phi_<c the output of the Phi chain (V = 0 makes B vanish).  Three launches after
 // the prep:
 //   maps    -- segment 0's chain from the caller's state (its outputs, and its end state as
 //              segment 1's entry), and, side by side, the Z and Phi chains of segments
@@ -1382,6 +1382,12 @@ long env_long(const char* name, long def, long hi) {
 // long: a function of the shapes only, so a workspace sized once serves every call of a shape.
 // An explicit request (tsa_gdn_chunked_plan_fwd) replaces it: req = 1 never splits, req >= 2
 // asks for req segments (fewer if the sequence has fewer chunks: no segment is empty).
+// us per call, fp16, no split / this plan / the best of 1 to 8 segments: T = 4096 1 head 63.4 / 35.8 / 35.8,
+// 4 heads 63.6 / 44.3 / 40.9 (4 segments), 8 67.1 / 55.4 / 54.8, 16 70.2 / 78.0 / 70.2; T = 2048 1 head 38.0 /
+// 30.9, 4 37.8 / 34.5, 8 38.3 / 40.6, 16 39.9 / 49.1; T = 1536 4 31.1 / 32.2; T = 1024 1 24.9 / 28.1, 4 24.6 / 29.5, 16
+// 25.5 / 39.7; T = 16384 4 229 / 97.  The plan was set for carry steps of 32 columns alone; an unsplit
+// carry of few heads now takes 16, so up to 16 chunks, and from 8 to 16 heads on, the plan is
+// the slower one (with the carry it was set for, T = 1024, 4 heads took 52 unsplit and 35.6 split).
 constexpr int kSplitCUs = 256;
 constexpr int kMinSegChunks = 8;
 struct SegPlan {
