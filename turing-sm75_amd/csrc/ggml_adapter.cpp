@@ -32,9 +32,9 @@ namespace {
 constexpr int64_t kS = 128;
 // Token count from which the chunked prefill is used.  Measured on MI355X at the target
 // model's 16 QK / 48 V heads, fp16 (token-serial vs chunked, us per call): one sequence T=24
-// 10.3 vs 14.1, T=32 12.1 vs 14.5, T=40 14.8 vs 14.7, T=48 16.6 vs 14.8; four sequences T=24
-// 17.2 vs 24.6, T=32 20.0 vs 23.9, T=40 24.0 vs 23.6, T=48 26.9 vs 24.2.  The kernels cross at
-// 40, so 32 costs up to 2.4 us (one sequence) and 3.9 us (four) from T = 32 to 39.
+// 10.4 vs 14.1, T=32 12.1 vs 14.5-15.4, T=40 14.8 vs 14.8, T=48 16.6 vs 14.6; four sequences
+// T=24 17.2 vs 24.0, T=32 20.0 vs 24.1, T=40 24.1 vs 23.8, T=48 27.1 vs 24.3.  The kernels cross
+// at 40, so 32 costs up to 3.3 us (one sequence) and 4.1 us (four) from T = 32 to 39.
 constexpr int64_t kChunkedMinT = 32;
 
 size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
