@@ -8,7 +8,7 @@
  * one synchronous call).  Every kernel runs on the caller's stream, in order, as the
  * reference's launches run on one stream with caller-owned scratch (src/gdn_sm75.cu:1341-1346).
  * Opt-in only: with the environment variable TSA_GDN_OVERLAP=1 the chunked prefill (not under
- * graph capture) runs its two kernels side by side on the caller's stream and on a second
+ * graph capture, nor with an output that lies on v) runs its two kernels side by side on the caller's stream and on a second
  * stream of the same device, which it creates with two events on the first such call on that
  * device (under a mutex) and keeps until the process ends.  Errors come back as TSA_* codes,
  * never as exit() or exceptions (the reference's CUDA_CHECK exits, src/attn_sm75.cu:40-48).
