@@ -641,6 +641,19 @@ def test_chunked_output_over_v(dev, monkeypatch, mode, T, hq, hv, io):
     assert np.array_equal(tv.float().cpu().numpy(), o0) and np.array_equal(ts.cpu().numpy(), s0)
 
 
+@pytest.mark.parametrize("io", ["f16", "f32"])
+@pytest.mark.parametrize("T", [1, 4, 33])
+def test_recurrent_output_over_v(dev, T, io):
+    """The decode step and both token-serial forms with out = v itself: bit for bit as without."""
+    rng = np.random.default_rng(418)
+    q, k, v, g, beta, st = _inputs(rng, 2, T, 2, 6, sstd=0.02)
+    q, k, v = _as(io, q, k, v)
+    o0, s0 = _gpu(dev, "recurrent", q, k, v, g, beta, st)
+    tq, tk, tv, tg, tb, ts = _dev(dev, q, k, v, g, beta, st)
+    tsa.gdn_recurrent_fwd(tq, tk, tv, tg, tb, ts, out=tv)
+    assert np.array_equal(tv.float().cpu().numpy(), o0) and np.array_equal(ts.cpu().numpy(), s0)
+
+
 def test_wrong_out_shape_raises_before_launch(dev):
     import torch
     rng = np.random.default_rng(408)
